@@ -6,11 +6,15 @@
 #include <cstdio>
 #include <cmath>
 #include <cstring>
+#include <future>
+#include <new>
 #include <string>
+#include <system_error>
 #include <thread>
 
 #include "host_query.h"
 #include "render_host.h"
+#include "wide_build.h"
 
 namespace ptx {
 
@@ -31,8 +35,8 @@ double now_s() {
 
 namespace {
 
-template <class T>
-int upload(ptx_scene *s, const std::vector<T> &v, const T **dst) {
+template <class T, class A>
+int upload(ptx_scene *s, const std::vector<T, A> &v, const T **dst) {
    *dst = nullptr;
    if (v.empty()) return PTX_OK;
    void *p = nullptr;
@@ -137,11 +141,50 @@ const Node64 *scene_windows(ptx_scene *s, const ptx_tuning &t) {
    return s->windows;
 }
 
+namespace {
+
+// Queries for hits or frames take the four-wide form; the counters count
+// binary boxes, and ray_windows = ON asks for the window records.
+bool wide_query(const ptx_scene *s, const ptx_tuning &t, const ptx_ray_counters *counters) {
+   return s->w.faces && !counters && t.ray_windows != PTX_WINDOWS_ON;
+}
+
+uint32_t wide_query_grid(const ptx_device *dev, const ptx_tuning &t, uint32_t lds, bool frames) {
+   int per_cu = closest_hit_wide_blocks_per_cu(lds, frames);
+   if (t.blocks_per_cu) per_cu = std::min<int>(per_cu, (int)t.blocks_per_cu);
+   return (uint32_t)(dev->num_cus * per_cu);
+}
+
+size_t wide_spill_bytes(const ptx_scene *s, uint32_t grid, uint32_t lds) {
+   return s->w.stack > lds ? size_t(s->w.stack - lds) * grid * 256 * 8 : 0;
+}
+
+uint32_t wide_refill_lanes_of(const ptx_tuning &t) {
+   return t.refill_lanes ? std::min(64u, t.refill_lanes) : kDefaultWideRefillLanes;
+}
+uint32_t wide_leaf_lanes_of(const ptx_tuning &t) {
+   return t.leaf_lanes ? std::min(64u, t.leaf_lanes) : kDefaultWideLeafLanes;
+}
+
+}  // namespace
+
 // Closest-hit launch with stack-spill scratch taken from the stream-ordered allocator.
 int run_closest_hit(ptx_scene *s, const float *d_rays, uint32_t n, ptx_hit *d_hits, ptx_ray_counters *d_counters,
                     ptx_hit_frame *d_frames, hipStream_t stream, const ptx_tuning &t) {
    ptx_device *dev = s->dev;
    const uint32_t lds = lds_depth_of(t);
+   if (wide_query(s, t, d_counters)) {
+      const uint32_t grid = std::max(1u, std::min(wide_query_grid(dev, t, lds, d_frames != nullptr), (n + 255) / 256));
+      void *scratch = nullptr;
+      PTX_HIP_TRY(pool_malloc(dev, &scratch, 256 + wide_spill_bytes(s, grid, lds), stream));
+      const int rc = launch_closest_hit_wide(s->d, s->w, d_rays, n, d_hits, d_frames, static_cast<uint32_t *>(scratch),
+                                             static_cast<char *>(scratch) + 256, grid, lds, wide_refill_lanes_of(t),
+                                             wide_leaf_lanes_of(t), stream);
+      const hipError_t fe = hipFreeAsync(scratch, stream);
+      if (rc != 0) return set_error(PTX_ERR_HIP, "closest-hit launch failed");
+      if (fe != hipSuccess) return set_error(PTX_ERR_HIP, std::string("hipFreeAsync: ") + hipGetErrorString(fe));
+      return PTX_OK;
+   }
    const Node64 *win = n ? scene_windows(s, t) : nullptr;
    uint32_t grid = closest_hit_grid(dev, t, lds, d_counters != nullptr || d_frames != nullptr, win != nullptr);
    const uint32_t needed_blocks = (n + 255) / 256;
@@ -318,14 +361,47 @@ int ptx_scene_create(ptx_device *dev, const ptx_scene_desc *desc, ptx_scene **ou
       build_s = now_s() - t0;
    }
    HostImage img;
-   const int lrc = layout_scene(meshes, s->bvh, img);
+   const int lrc = layout_scene(meshes, s->bvh, img, desc->build_threads);
    if (lrc != PTX_OK) return lrc;
    const double t1 = now_s();
    int rc;
+   // the four-wide form is built while the arrays it does not need go up; the
+   // thread is joined on every way out (~std::future)
+   WideImage wide;
+   auto make_wide = [&] {
+      try {
+         return build_wide(s->bvh, img, desc->build_threads, wide);
+      } catch (const std::bad_alloc &) {         // no memory for it: the scene does without
+         return false;
+      }
+   };
+   std::future<bool> wide_built;
+   try {
+      wide_built = std::async(std::launch::async, make_wide);
+   } catch (const std::system_error &) {         // no thread to be had: built below by this one
+   }
    if ((rc = upload(s.get(), img.nodes, &s->d.nodes)) != PTX_OK) return rc;
    if ((rc = upload(s.get(), img.tris, &s->d.tris)) != PTX_OK) return rc;
    if ((rc = upload(s.get(), s->bvh.pairs, &s->d.pairs)) != PTX_OK) return rc;
    if ((rc = upload(s.get(), img.meshes, &s->d.meshes)) != PTX_OK) return rc;
+   if (wide_built.valid() ? wide_built.get() : make_wide()) {
+      if ((rc = upload(s.get(), wide.nodes, &s->w.nodes)) != PTX_OK) return rc;
+      if ((rc = upload(s.get(), wide.leaves, &s->w.leaves)) != PTX_OK) return rc;
+      // the faces from the triangles and ids just uploaded
+      const size_t bytes = size_t(img.num_tris) * sizeof(WideFace);
+      void *faces = nullptr;
+      PTX_HIP_TRY(hipMalloc(&faces, bytes));
+      s->allocations.push_back(faces);
+      s->info.device_bytes += bytes;
+      if (launch_build_wide_faces(s->d.tris, s->d.pairs, img.num_tris, static_cast<WideFace *>(faces), nullptr) != 0) {
+         (void)hipGetLastError();
+         return set_error(PTX_ERR_HIP, "four-wide face records");
+      }
+      PTX_HIP_TRY(hipStreamSynchronize(nullptr));
+      s->w.faces = static_cast<const WideFace *>(faces);
+      s->w.root = wide.root;
+      s->w.stack = wide.stack;
+   }
    if (s->has_texture) {
       // one texture record per leaf-ordered triangle, then the texel pool (each
       // texture that a mesh uses, once), in one allocation
@@ -466,6 +542,22 @@ int ptx_intersect_closest_device_noalloc(ptx_scene *scene, const float *d_rays, 
    PTX_HIP_TRY(hipSetDevice(dev->ordinal));
    uint32_t *work = static_cast<uint32_t *>(dev->noalloc_scratch);
    uint4 *spill = reinterpret_cast<uint4 *>(static_cast<char *>(dev->noalloc_scratch) + 256);
+   // the four-wide form wherever its spill takes no fewer blocks
+   if (wide_query(scene, t, d_counters)) {
+      uint32_t wgrid = wide_query_grid(dev, t, lds, d_frames != nullptr);
+      const size_t block = wide_spill_bytes(scene, 1, lds);
+      if (block) wgrid = (uint32_t)std::min<size_t>(wgrid, (kNoAllocScratchBytes - 256) / block);
+      wgrid = std::min(wgrid, std::max(1u, (n + 255) / 256));
+      if (wgrid >= std::min(grid, (uint32_t)dev->num_cus)) {
+         if (launch_closest_hit_wide(scene->d, scene->w, d_rays, n, d_hits, d_frames, work, spill, wgrid, lds,
+                                     wide_refill_lanes_of(t), wide_leaf_lanes_of(t),
+                                     static_cast<hipStream_t>(stream)) != 0) {
+            (void)hipGetLastError();
+            return set_error(PTX_ERR_HIP, "closest-hit launch failed");
+         }
+         return PTX_OK;
+      }
+   }
    const uint32_t refill = refill_lanes_of(t);
    // the work counters are cleared by a kernel at the head of the launch (no memset)
    if (launch_closest_hit(scene->d, d_rays, n, d_hits, d_counters, d_frames, work, spill, grid, lds, refill,

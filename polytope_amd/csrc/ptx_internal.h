@@ -37,6 +37,40 @@ static_assert(sizeof(Node64) == 64, "Node64 is 64 bytes");
 
 constexpr uint32_t kLeafBit = 0x80000000u;
 
+// Four-wide form of the tree (wide.h): up to four descendants of a binary
+// node, their boxes in steps of 2^exponent from the node's low corner, rounded
+// outwards.  planes: low and high x, low and high y, low and high z, child k in
+// byte k.  later[q], q = octant of the rays whose z direction is not negative
+// (bit a set: direction a negative): bits 4 k .. 4 k + 3 = the children visited
+// after child k; the octant with every sign flipped visits in reverse.  Only
+// the children in `used` (bit k) are there: an empty one (low 255, high 0) may
+// pass a test and has no place in the order.
+struct alignas(64) WideNode {
+   float org[3];
+   int8_t exponent[3];       // x, y, z
+   uint8_t used;
+   uint8_t planes[6][4];
+   uint32_t ref[4];
+   uint16_t later[4];
+};
+static_assert(sizeof(WideNode) == 64, "WideNode is 64 bytes");
+
+// A face as the four-wide traversal reads it, at its leaf-ordered index.
+struct alignas(16) WideFace {
+   float v[9];               // world v0, v1, v2
+   uint32_t mesh, face;      // the reference's ids
+   uint32_t pad;
+};
+static_assert(sizeof(WideFace) == 48, "WideFace layout");
+
+// A leaf of more than two faces, or whose box is not its corners': leaf 0 of a
+// scene is the empty one.
+struct alignas(16) WideLeaf {
+   float box[6];
+   uint32_t first, count;
+};
+static_assert(sizeof(WideLeaf) == 32, "WideLeaf layout");
+
 // Per-mesh shading record (9 words, read as one block by the shading step).
 // Glossy meshes that are not lights keep the lobe's constant reflectance in
 // refl and its roughness in emission[0].  A textured Lambert mesh
@@ -84,6 +118,15 @@ struct DevScene {
    const TexTri *tex_tris;   // texture records per leaf-ordered triangle, then the texel pool; or null
 };
 static_assert(sizeof(DevScene) == 112, "DevScene layout");
+
+// Device view of a scene's four-wide form.
+struct WideScene {
+   const WideNode *nodes;
+   const WideFace *faces;    // null: the scene has no such form
+   const WideLeaf *leaves;
+   uint32_t root;            // a node's index or a leaf reference
+   uint32_t stack;           // 8-byte stack entries a lane needs, the sentinel and exact_trace's words among them
+};
 
 // Per-job constants of a render, device-resident in the job table.
 struct JobDev {

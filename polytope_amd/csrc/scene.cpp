@@ -101,11 +101,11 @@ void world_vertices(const ptx_mesh_desc &m, WorldMesh &out, bool shading) {
    }
 }
 
-int layout_scene(const std::vector<WorldMesh> &meshes, const HostBvh &bvh, HostImage &img) {
+int layout_scene(const std::vector<WorldMesh> &meshes, const HostBvh &bvh, HostImage &img, unsigned threads) {
    const size_t nn = bvh.nodes.size();
    const size_t np = bvh.pairs.size() / 2;
    if (nn == 0) return set_error(PTX_ERR_INVALID, "scene has no faces");
-   std::vector<uint32_t> ref(nn);
+   UnsetVector<uint32_t> ref(nn);
    uint32_t n_int = 0, n_leaf = 0;
    for (size_t i = 0; i < nn; i++) {
       const ptx_bvh_node &b = bvh.nodes[i];
@@ -115,43 +115,45 @@ int layout_scene(const std::vector<WorldMesh> &meshes, const HostBvh &bvh, HostI
          ref[i] = kLeafBit | b.offset;
          n_leaf++;
       } else {
+         if (i + 1 >= nn || i + b.offset >= nn || b.offset < 2 || b.flags > 2)
+            return set_error(PTX_ERR_INVALID, "BVH interior node has an out-of-range child");
          ref[i] = n_int++;
       }
    }
-   img.nodes.assign(n_int, Node64{});
-   for (size_t i = 0; i < nn; i++) {
-      const ptx_bvh_node &b = bvh.nodes[i];
-      if (b.num_faces > 0) continue;
-      const size_t lo = i + 1, hi = i + b.offset;
-      if (lo >= nn || hi >= nn || b.offset < 2 || b.flags > 2)
-         return set_error(PTX_ERR_INVALID, "BVH interior node has an out-of-range child");
-      Node64 &r = img.nodes[ref[i]];
-      const ptx_bvh_node &c0 = bvh.nodes[lo], &c1 = bvh.nodes[hi];
-      for (int k = 0; k < 3; k++) {
-         r.box[k] = c0.p0[k]; r.box[3 + k] = c0.p1[k];
-         r.box[6 + k] = c1.p0[k]; r.box[9 + k] = c1.p1[k];
-      }
-      r.ref[0] = ref[lo];
-      r.ref[1] = ref[hi];
-      // a leaf child's slot holds its face count, an interior child's its split
-      // axis (which the closest-hit kernel's window records are selected by)
-      const uint32_t k0 = c0.num_faces ? (uint32_t)c0.num_faces : (uint32_t)c0.flags;
-      const uint32_t k1 = c1.num_faces ? (uint32_t)c1.num_faces : (uint32_t)c1.flags;
-      r.counts = k0 | (k1 << 16);
-      r.axis = b.flags;
-   }
-   // deepest chain of interior nodes bounds the deferred stack
-   {
-      std::vector<std::pair<uint32_t, uint32_t>> st = {{0u, 0u}};
-      uint32_t depth = 0;
-      while (!st.empty()) {
-         const auto [i, d] = st.back();
-         st.pop_back();
+   img.nodes.resize(n_int);
+   host_ranges(nn, threads, 65536, [&](size_t first, size_t last) {
+      for (size_t i = first; i < last; i++) {
          const ptx_bvh_node &b = bvh.nodes[i];
          if (b.num_faces > 0) continue;
-         depth = std::max(depth, d + 1);
-         st.push_back({i + 1, d + 1});
-         st.push_back({i + b.offset, d + 1});
+         const size_t lo = i + 1, hi = i + b.offset;
+         Node64 &r = img.nodes[ref[i]];
+         const ptx_bvh_node &c0 = bvh.nodes[lo], &c1 = bvh.nodes[hi];
+         for (int k = 0; k < 3; k++) {
+            r.box[k] = c0.p0[k]; r.box[3 + k] = c0.p1[k];
+            r.box[6 + k] = c1.p0[k]; r.box[9 + k] = c1.p1[k];
+         }
+         r.ref[0] = ref[lo];
+         r.ref[1] = ref[hi];
+         // a leaf child's slot holds its face count, an interior child's its split
+         // axis (which the closest-hit kernel's window records are selected by)
+         const uint32_t k0 = c0.num_faces ? (uint32_t)c0.num_faces : (uint32_t)c0.flags;
+         const uint32_t k1 = c1.num_faces ? (uint32_t)c1.num_faces : (uint32_t)c1.flags;
+         r.counts = k0 | (k1 << 16);
+         r.axis = b.flags;
+      }
+   });
+   // deepest chain of interior nodes bounds the deferred stack; children
+   // follow their parents
+   {
+      std::vector<uint32_t> level(nn, 0);
+      uint32_t depth = 0;
+      for (size_t i = 0; i < nn; i++) {
+         const ptx_bvh_node &b = bvh.nodes[i];
+         if (b.num_faces > 0) continue;
+         const uint32_t d = level[i] + 1;
+         depth = std::max(depth, d);
+         level[i + 1] = std::max(level[i + 1], d);
+         level[i + b.offset] = std::max(level[i + b.offset], d);
       }
       img.max_stack = depth + 1;
    }
@@ -161,21 +163,25 @@ int layout_scene(const std::vector<WorldMesh> &meshes, const HostBvh &bvh, HostI
       img.root_box[k] = bvh.nodes[0].p0[k];
       img.root_box[3 + k] = bvh.nodes[0].p1[k];
    }
+   for (size_t p = 0; p < np; p++)
+      if (bvh.pairs[2 * p] >= meshes.size() || bvh.pairs[2 * p + 1] >= meshes[bvh.pairs[2 * p]].nf)
+         return set_error(PTX_ERR_INVALID, "leaf pair names a face that does not exist");
    // 32 floats of padding: a traversal step loads 72 bytes (Node64 form) or 128
    // bytes (window form) from a leaf's first face
-   img.tris.assign(9 * np + 32, 0.f);
+   img.tris.resize(9 * np + 32);
+   std::fill(img.tris.end() - 32, img.tris.end(), 0.f);
    img.num_tris = (uint32_t)np;
    bool any_normals = false;
    for (const auto &m : meshes) any_normals |= m.has_normals;
-   if (any_normals) img.normals.assign(9 * np, 0.f);
-   for (size_t p = 0; p < np; p++) {
-      const uint32_t mi = bvh.pairs[2 * p], f = bvh.pairs[2 * p + 1];
-      if (mi >= meshes.size() || f >= meshes[mi].nf)
-         return set_error(PTX_ERR_INVALID, "leaf pair names a face that does not exist");
-      std::copy(&meshes[mi].wv[9 * size_t(f)], &meshes[mi].wv[9 * size_t(f)] + 9, &img.tris[9 * p]);
-      if (any_normals && meshes[mi].has_normals)
-         std::copy(&meshes[mi].wn[9 * size_t(f)], &meshes[mi].wn[9 * size_t(f)] + 9, &img.normals[9 * p]);
-   }
+   if (any_normals) img.normals.resize(9 * np);
+   host_ranges(np, threads, 65536, [&](size_t first, size_t last) {
+      for (size_t p = first; p < last; p++) {
+         const uint32_t mi = bvh.pairs[2 * p], f = bvh.pairs[2 * p + 1];
+         std::copy(&meshes[mi].wv[9 * size_t(f)], &meshes[mi].wv[9 * size_t(f)] + 9, &img.tris[9 * p]);
+         if (any_normals && meshes[mi].has_normals)
+            std::copy(&meshes[mi].wn[9 * size_t(f)], &meshes[mi].wn[9 * size_t(f)] + 9, &img.normals[9 * p]);
+      }
+   });
    img.meshes.resize(meshes.size());
    for (size_t i = 0; i < meshes.size(); i++) img.meshes[i] = meshes[i].rec;
    img.num_interior = n_int;

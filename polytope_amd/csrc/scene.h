@@ -1,9 +1,12 @@
 // Host-side scene image and the device scene object behind ptx_scene.
 #pragma once
 
+#include <algorithm>
 #include <atomic>
 #include <memory>
 #include <mutex>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "launch.h"
@@ -29,9 +32,26 @@ struct HostQueryStaging;
 
 namespace ptx {
 
+// A vector whose resize leaves new elements unset: large arrays that several
+// threads fill are then first touched by those threads.
+template <class T>
+struct UnsetAlloc : std::allocator<T> {
+   template <class U>
+   struct rebind {
+      using other = UnsetAlloc<U>;
+   };
+   template <class U, class... A>
+   void construct(U *p, A &&...a) {
+      if constexpr (sizeof...(A) == 0) ::new (static_cast<void *>(p)) U;
+      else ::new (static_cast<void *>(p)) U(std::forward<A>(a)...);
+   }
+};
+template <class T>
+using UnsetVector = std::vector<T, UnsetAlloc<T>>;
+
 struct HostImage {
-   std::vector<Node64> nodes;
-   std::vector<float> tris;
+   UnsetVector<Node64> nodes;
+   UnsetVector<float> tris;
    std::vector<float> normals;
    std::vector<MeshRec> meshes;
    float root_box[6] = {0, 0, 0, 0, 0, 0};
@@ -41,7 +61,27 @@ struct HostImage {
    uint32_t num_tris = 0;
 };
 
-int layout_scene(const std::vector<WorldMesh> &meshes, const HostBvh &bvh, HostImage &img);
+// threads 0 = all host cores.
+int layout_scene(const std::vector<WorldMesh> &meshes, const HostBvh &bvh, HostImage &img, unsigned threads = 0);
+
+// f(lo, hi) over [0, n) on up to `threads` host threads (0 = all cores, at most
+// 16), none with fewer than `least` items; the calling thread takes a share.
+template <class F>
+void host_ranges(size_t n, unsigned threads, size_t least, F f) {
+   if (threads == 0) threads = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
+   const size_t parts = std::max<size_t>(1, std::min<size_t>(threads, n / std::max<size_t>(1, least)));
+   std::vector<std::thread> ts;
+   ts.reserve(parts - 1);
+   for (size_t t = 1; t < parts; t++) {
+      try {
+         ts.emplace_back(f, n * t / parts, n * (t + 1) / parts);
+      } catch (const std::system_error &) {      // no thread to be had
+         f(n * t / parts, n * (t + 1) / parts);
+      }
+   }
+   f(size_t(0), n / parts);
+   for (std::thread &t : ts) t.join();
+}
 
 double now_s();
 const char *last_error_cstr();
@@ -55,6 +95,12 @@ uint32_t lds_depth_of(const ptx_tuning &t);
 // 16 for the render kernels (whose leaf and shading steps share the wave).
 constexpr uint32_t kDefaultLeafLanes = 1;
 constexpr uint32_t kDefaultRenderLeafLanes = 16;
+// Four-wide ray queries: a leaf step runs for the whole wave beside one in nine
+// node steps, so it waits for 24 lanes (8, 16, 24 and 32 lanes: 1,434, 1,371,
+// 1,348 and 1,344 us on a 4K frame's primary rays, 760, 718, 717 and 720 on
+// 2^21 incoherent ones, 1.3 M faces); new rays for 8 idle lanes (1 %).
+constexpr uint32_t kDefaultWideLeafLanes = 24;
+constexpr uint32_t kDefaultWideRefillLanes = 8;
 // Idle lanes a ray-query wave waits for before it takes new rays: 2, 4 and 8
 // measured 2,377-2,383 Mrays/s against 2,342 for 1 and 2,349 for 16 (2^21
 // incoherent rays on 1.3 M faces).
@@ -121,6 +167,7 @@ struct ptx_scene {
    ptx_device *dev = nullptr;
    ptx::HostBvh bvh;                 // reference-layout BVH (kept for ptx_scene_copy_bvh)
    ptx::DevScene d{};                // device pointers + root
+   ptx::WideScene w{};               // four-wide form, if the scene has one
    std::vector<void *> allocations;
    ptx_scene_info info{};
    uint32_t num_meshes = 0;

@@ -7,6 +7,7 @@
 
 #include "launch.h"
 #include "traverse.h"
+#include "wide.h"
 
 #pragma clang fp contract(off)
 
@@ -99,6 +100,59 @@ k_closest_hit(DevScene sc, const float *__restrict__ rays, uint32_t n, ptx_hit *
    persistent_trace<kLds>(q, n, work, spill, refill_min, leaf_min, sc.max_stack);
 }
 
+// The four-wide form (hits, and frames when asked for): the reference's
+// counters count binary boxes, so queries that want them step over the binary
+// records above.
+template <bool kFrames>
+struct WideQuery {
+   struct Words {};
+   DevScene sc;
+   WideScene wide;
+   const float *rays;
+   ptx_hit *hits;
+   ptx_hit_frame *frames;
+   __device__ __forceinline__ void prepare(uint32_t id, Trav &s, Words &) const {
+      const float *rp = rays + 6 * (size_t)id;
+      make_ray(s.r, rp[0], rp[1], rp[2], rp[3], rp[4], rp[5]);
+      wide_ray(s.r);
+      wide_begin(s, sc.root_box, wide.root);
+   }
+   __device__ __forceinline__ Words lane_words(uint32_t, const Words &w) const { return w; }
+   __device__ __forceinline__ const WideNode *nodes(const Words &) const { return wide.nodes; }
+   __device__ __forceinline__ const WideFace *faces(const Words &) const { return wide.faces; }
+   __device__ __forceinline__ const WideLeaf *leaves(const Words &) const { return wide.leaves; }
+   __device__ __forceinline__ BinaryScene binary(const Words &) const {
+      return BinaryScene{sc.nodes, sc.tris, sc.root_box, sc.root_ref, sc.root_count};
+   }
+   __device__ __forceinline__ bool debug_pixel(uint32_t, const Words &) const { return false; }
+   __device__ __forceinline__ void finish(uint32_t id, const Words &, const Trav &s) const {
+      ptx_hit h;
+      h.mesh = s.mesh; h.face = s.face;
+      h.t = s.min_t; h.u = s.hu; h.v = s.hv; h.w = s.hw;      // a miss holds +inf and zeros
+      hits[id] = h;
+      if (kFrames) {
+         ptx_hit_frame fr = {};
+         if (s.hit != 0xFFFFFFFFu) {
+            Frame f;
+            const float *cn = sc.normals ? sc.normals + 9 * (size_t)s.hit : nullptr;
+            if (cn && !(sc.meshes[s.mesh].flags & kRecNormals)) cn = nullptr;
+            hit_frame(sc.tris + 9 * (size_t)s.hit, cn, s.r, s.hu, s.hv, s.hw, s.after, f);
+            fr = ptx_hit_frame{{f.lx, f.ly, f.lz}, {f.nx, f.ny, f.nz}, {f.t1x, f.t1y, f.t1z},
+                               {f.t2x, f.t2y, f.t2z}, {f.ex, f.ey, f.ez}};
+         }
+         frames[id] = fr;
+      }
+   }
+};
+
+template <int kLds, bool kFrames>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
+k_closest_hit_wide(DevScene sc, WideScene w, const float *__restrict__ rays, uint32_t n, ptx_hit *__restrict__ hits,
+                   ptx_hit_frame *frames, uint32_t *work, uint2 *spill, uint32_t refill_min, uint32_t leaf_min) {
+   const WideQuery<kFrames> q{sc, w, rays, hits, frames};
+   wide_trace<kLds>(q, n, work, spill, refill_min, leaf_min, w.stack);
+}
+
 // One thread per window: window w of interior node i is win[4 i + 2 w] (the
 // node's record) and win[4 i + 2 w + 1] (the record of the child visited first
 // for direction sign w on the node's axis: child 1 when w = 1, child 0 when
@@ -113,6 +167,19 @@ __global__ void k_build_windows(const Node64 *__restrict__ nodes, uint32_t n_int
    if (!(child & kLeafBit)) b = nodes[child];
    win[2 * t] = a;
    win[2 * t + 1] = b;
+}
+
+__global__ void k_build_wide_faces(const float *__restrict__ tris, const uint32_t *__restrict__ pairs, uint32_t np,
+                                   WideFace *__restrict__ out) {
+   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+   if (p >= np) return;
+   WideFace f;
+#pragma unroll
+   for (int k = 0; k < 9; k++) f.v[k] = tris[9 * (size_t)p + k];
+   f.mesh = pairs[2 * (size_t)p];
+   f.face = pairs[2 * (size_t)p + 1];
+   f.pad = 0;
+   out[p] = f;
 }
 
 __global__ void k_zero_u32(uint32_t *p, uint32_t n) {
@@ -199,6 +266,55 @@ int blocks_lds(bool extra, bool windows) {
 
 }  // namespace
 
+namespace {
+
+template <int kLds>
+void launch_wide(const DevScene &sc, const WideScene &w, const float *d_rays, uint32_t n, ptx_hit *d_hits, ptx_hit_frame *d_frames,
+                 uint32_t *d_work, uint2 *d_spill, uint32_t grid, uint32_t refill_min, uint32_t leaf_min,
+                 hipStream_t stream) {
+   if (d_frames)
+      hipLaunchKernelGGL((dev::k_closest_hit_wide<kLds, true>), dim3(grid), dim3(256), 0, stream, sc, w, d_rays, n, d_hits,
+                         d_frames, d_work, d_spill, refill_min, leaf_min);
+   else
+      hipLaunchKernelGGL((dev::k_closest_hit_wide<kLds, false>), dim3(grid), dim3(256), 0, stream, sc, w, d_rays, n,
+                         d_hits, d_frames, d_work, d_spill, refill_min, leaf_min);
+}
+
+template <int kLds>
+int blocks_wide(bool frames) {
+   int b = 0;
+   const hipError_t e =
+         frames ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, dev::k_closest_hit_wide<kLds, true>, 256, 0)
+                : hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, dev::k_closest_hit_wide<kLds, false>, 256, 0);
+   return e == hipSuccess && b > 0 ? b : 1;
+}
+
+}  // namespace
+
+int launch_closest_hit_wide(const DevScene &sc, const WideScene &w, const float *d_rays, uint32_t n, ptx_hit *d_hits,
+                            ptx_hit_frame *d_frames, uint32_t *d_work, void *d_spill, uint32_t grid,
+                            uint32_t lds_depth, uint32_t refill_min, uint32_t leaf_min, hipStream_t stream) {
+   hipLaunchKernelGGL(dev::k_zero_u32, dim3(1), dim3(64), 0, stream, d_work, (uint32_t)dev::kWorkWords);
+   if (n == 0) return 0;
+   uint2 *spill = static_cast<uint2 *>(d_spill);
+   switch (lds_depth) {
+      case 8: launch_wide<8>(sc, w, d_rays, n, d_hits, d_frames, d_work, spill, grid, refill_min, leaf_min, stream); break;
+      case 16: launch_wide<16>(sc, w, d_rays, n, d_hits, d_frames, d_work, spill, grid, refill_min, leaf_min, stream); break;
+      case 24: launch_wide<24>(sc, w, d_rays, n, d_hits, d_frames, d_work, spill, grid, refill_min, leaf_min, stream); break;
+      default: launch_wide<12>(sc, w, d_rays, n, d_hits, d_frames, d_work, spill, grid, refill_min, leaf_min, stream); break;
+   }
+   return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+int closest_hit_wide_blocks_per_cu(uint32_t lds_depth, bool frames) {
+   switch (lds_depth) {
+      case 8: return blocks_wide<8>(frames);
+      case 16: return blocks_wide<16>(frames);
+      case 24: return blocks_wide<24>(frames);
+      default: return blocks_wide<12>(frames);
+   }
+}
+
 int launch_closest_hit(const DevScene &sc, const float *d_rays, uint32_t n, ptx_hit *d_hits,
                        ptx_ray_counters *d_counters, ptx_hit_frame *d_frames, uint32_t *d_work, uint4 *d_spill,
                        uint32_t grid, uint32_t lds_depth, uint32_t refill_min, uint32_t leaf_min,
@@ -233,6 +349,12 @@ int closest_hit_blocks_per_cu(uint32_t lds_depth, bool extra, bool windows) {
       case 24: return blocks_lds<24>(extra, windows);
       default: return blocks_lds<12>(extra, windows);
    }
+}
+
+int launch_build_wide_faces(const float *tris, const uint32_t *pairs, uint32_t np, WideFace *out, hipStream_t stream) {
+   if (np == 0) return 0;
+   hipLaunchKernelGGL(dev::k_build_wide_faces, dim3((np + 255) / 256), dim3(256), 0, stream, tris, pairs, np, out);
+   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int launch_build_windows(const Node64 *nodes, uint32_t n_int, Node64 *win, hipStream_t stream) {

@@ -13,6 +13,9 @@
 
 #pragma clang fp contract(off)
 
+// Arithmetic that a host check compiles too.
+#define PTX_HD __host__ __device__ __forceinline__
+
 namespace ptx {
 namespace dev {
 
@@ -26,16 +29,16 @@ constexpr float kGamma5 = (5 * kMachineEpsilon) / (1 - 5 * kMachineEpsilon);
 constexpr float kGamma7 = (7 * kMachineEpsilon) / (1 - 7 * kMachineEpsilon);
 constexpr float kSlabScale = 1 + 2 * gamma_n(3);              // BoundingBox.cpp:27
 
-__device__ __forceinline__ float fmaf_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+PTX_HD float fmaf_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
 // src/cpu/constants.h:121-133
-__device__ __forceinline__ float diff_of_products(float a, float b, float c, float d) {
+PTX_HD float diff_of_products(float a, float b, float c, float d) {
    const float cd = c * d;
    const float dop = fmaf_(a, b, -cd);
    const float err = fmaf_(-c, d, cd);
    return dop + err;
 }
-__device__ __forceinline__ float sum_of_products(float a, float b, float c, float d) {
+PTX_HD float sum_of_products(float a, float b, float c, float d) {
    const float cd = c * d;
    const float sop = fmaf_(a, b, cd);
    const float err = fmaf_(c, d, -cd);
@@ -63,15 +66,16 @@ struct Ray {
    float ox, oy, oz, dx, dy, dz;
    float ix, iy, iz;          // 1 / d  (bvh.cpp:477-481)
    uint32_t nk;               // bit a (0-2): inverse_direction[a] < 0 (bvh.cpp:483); bits 3-4: the
-                              // Wald dominant axis kz, with kx = kz+1, ky = kz+2 (mod 3)
+                              // Wald dominant axis kz, with kx = kz+1, ky = kz+2 (mod 3); bits 5-7:
+                              // the four-wide traversal's classes of rays (wide.h)
    float Sx, Sy, Sz;
 };
 
-__device__ __forceinline__ float pick3(uint32_t k, float a, float b, float c) {
+PTX_HD float pick3(uint32_t k, float a, float b, float c) {
    return k == 0 ? a : (k == 1 ? b : c);
 }
 
-__device__ __forceinline__ void make_ray(Ray &r, float ox, float oy, float oz, float dx, float dy, float dz) {
+PTX_HD void make_ray(Ray &r, float ox, float oy, float oz, float dx, float dy, float dz) {
    r.ox = ox; r.oy = oy; r.oz = oz; r.dx = dx; r.dy = dy; r.dz = dz;
    r.ix = 1.f / dx; r.iy = 1.f / dy; r.iz = 1.f / dz;
    const uint32_t neg = (r.ix < 0 ? 1u : 0u) | (r.iy < 0 ? 2u : 0u) | (r.iz < 0 ? 4u : 0u);
@@ -108,7 +112,7 @@ __device__ __forceinline__ void make_ray(Ray &r, float ox, float oy, float oz, f
 // because near starts at 0 and is never NaN (likewise far from +inf).  The
 // two can differ only in the sign of a zero result, and near and far are only
 // ever compared, where -0 == +0.
-__device__ __forceinline__ void slab(float b0, float b1, float b2, float b3, float b4, float b5,
+PTX_HD void slab(float b0, float b1, float b2, float b3, float b4, float b5,
                                      const Ray &r, float &near, float &far) {
    near = 0.f;
    far = kInf;
@@ -129,13 +133,13 @@ __device__ __forceinline__ void slab(float b0, float b1, float b2, float b3, flo
 // input is NaN.  Its results feed only deltaT, which matters only through
 // `t <= deltaT`, and a NaN input (a NaN coordinate, U, V or W) makes det or T,
 // and so t, NaN: the comparison is then false whatever deltaT is.
-__device__ __forceinline__ float max_component(float x, float y, float z) {
+PTX_HD float max_component(float x, float y, float z) {
    return fmaxf(fmaxf(x, y), z);
 }
 
 // Mesh::intersect test part for one face (mesh.cpp:196-340).  On acceptance
 // updates min_t and the hit's (u, v, w) and returns true.
-__device__ __forceinline__ bool test_triangle(const float *v, const Ray &r, float &min_t,
+PTX_HD bool test_triangle(const float *v, const Ray &r, float &min_t,
                                               float &hu, float &hv, float &hw, bool debug_pixel) {
    if (debug_pixel && r.dx != r.dx) return false;              // mesh.cpp:192-194
    const float v0x = v[0], v0y = v[1], v0z = v[2];
@@ -145,7 +149,7 @@ __device__ __forceinline__ bool test_triangle(const float *v, const Ray &r, floa
    const float a0 = v0x - r.ox, a1 = v0y - r.oy, a2 = v0z - r.oz;
    const float b0 = v1x - r.ox, b1 = v1y - r.oy, b2 = v1z - r.oz;
    const float c0 = v2x - r.ox, c1 = v2y - r.oy, c2 = v2z - r.oz;
-   const uint32_t kz = r.nk >> 3;
+   const uint32_t kz = (r.nk >> 3) & 3u;
    // kz = 0 -> (y, z, x); kz = 1 -> (z, x, y); kz = 2 -> (x, y, z)
    float p0x = pick3(kz, a1, a2, a0), p0y = pick3(kz, a2, a0, a1), p0z = pick3(kz, a0, a1, a2);
    float p1x = pick3(kz, b1, b2, b0), p1y = pick3(kz, b2, b0, b1), p1z = pick3(kz, b0, b1, b2);
@@ -298,6 +302,7 @@ struct Trav {
    Ray r;
    float min_t, hu, hv, hw;
    uint32_t hit;          // leaf-ordered triangle index, 0xFFFFFFFF = none
+   uint32_t mesh, face;   // the hit's ids (four-wide traversal, whose face records carry them)
    uint32_t after;        // face tests since (and including) the accepting one
    uint32_t cur;          // node to process next: kLeafBit | first triangle, or interior index
    uint32_t cnt;          // faces left in the leaf `cur` (0 for an interior node)

@@ -1,0 +1,106 @@
+"""The four-wide traversal (polytope_amd/csrc/wide.h) against the binary one.
+
+CPU: the headers' tests and the host builder, compiled for the host, visit the
+leaves of the reference's traversal in its order (tests/wide_check.cpp).  GPU:
+queries for hits and frames take the four-wide form and queries for counters
+the binary one, so both answers for the same rays must be equal bit for bit:
+scenes of one face, of leaves past two faces and of none that a small LDS stack
+holds, sizes around a wave and a block, and rays with zero, negative-zero,
+tiny, infinite and NaN components and origins on the vertices' planes."""
+from __future__ import annotations
+
+import shutil
+import subprocess
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+from polytope_amd import scenes as S
+
+ROOT = Path(__file__).resolve().parents[1]
+
+
+def test_wide_traversal_visits_the_reference_leaves(tmp_path):
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not Path(hipcc).exists():
+        pytest.skip("hipcc not found")
+    exe = tmp_path / "wide_check"
+    csrc = ROOT / "polytope_amd" / "csrc"
+    subprocess.run([hipcc, "-O2", "-std=c++17", "-ffp-contract=off", "-x", "hip", "--offload-arch=gfx950",
+                    "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                    f"-I{csrc}", f"-I{ROOT / 'include'}", str(ROOT / "tests" / "wide_check.cpp"),
+                    *(str(csrc / f) for f in ("wide_build.cpp", "bvh_build.cpp", "scene.cpp")), "-lpthread",
+                    "-o", str(exe)], check=True, capture_output=True, timeout=300)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stdout
+    assert " 0 mismatches" in out.stdout
+
+
+def _edge_rays(rays: np.ndarray, verts: np.ndarray) -> np.ndarray:
+    """Every second ray of ``rays`` with components that make slab values infinite or NaN."""
+    r = rays.copy()
+    rng = np.random.default_rng(3)
+    n = len(r)
+    for a in range(3):
+        k = rng.integers(0, 24, n)
+        for i, x in enumerate((0.0, -0.0, 1e-39, -1e-30, 1e25)):
+            r[(k == i) & (np.arange(n) % 2 == 1), 3 + a] = x
+        on = (k > 18) & (np.arange(n) % 2 == 1)
+        r[on, a] = verts[rng.integers(0, len(verts), on.sum()), a]
+    k = np.arange(n) % 301
+    for i, (j, x) in enumerate(((3, np.nan), (4, np.inf), (0, np.nan), (1, -np.inf), (2, 1e25))):
+        r[k == i, j] = x
+    r[k == 7, 3:] = 0.0
+    return r
+
+
+def _scene(name: str):
+    if name == "face":
+        v = np.array([[0, 0, 0], [1, 0, 0], [0, 1, 0.5]], np.float32)
+        return v, np.array([[0, 1, 2]], np.uint32)
+    if name == "duplicates":                     # leaves of many faces: the same three triangles 20 times
+        v, f = S.icosphere(0, noise=0.0, seed=1)
+        return v, np.concatenate([f[:3]] * 20)
+    if name == "slivers":
+        return S.sliver_grid(48, 2.0)
+    return S.icosphere(6, noise=0.05, seed=2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["face", "duplicates", "slivers", "sphere"])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 60_001])
+def test_wide_and_binary_queries_agree(name, n):
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from polytope_amd import Device, Scene
+    verts, faces = _scene(name)
+    meshes = [S.MeshData(verts, faces)]
+    lo, hi = S.scene_bounds(meshes)
+    rays = _edge_rays(S.rays_incoherent(np.asarray(lo) - 0.2, np.asarray(hi) + 0.2, n, 9), verts)
+    dev = Device(0)
+    scene = Scene(dev, meshes)
+    r = torch.from_numpy(rays).cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def query(counters: bool, frames: bool):
+        h = torch.full((n, 6), -7, dtype=torch.int32, device="cuda")
+        c = torch.zeros((n, 3), dtype=torch.int32, device="cuda")
+        f = torch.full((n, 15), -7.0, dtype=torch.float32, device="cuda")
+        scene.intersect_device(r.data_ptr(), n, h.data_ptr(), c.data_ptr() if counters else 0,
+                               f.data_ptr() if frames else 0, stream)
+        torch.cuda.synchronize()
+        return h.cpu().numpy(), f.cpu().numpy().view(np.uint32)
+
+    try:
+        hits, frames = query(True, True)
+        for lds, leaf in ((0, 0), (8, 1), (24, 64)):
+            dev.set_tuning(lds_stack=lds, leaf_lanes=leaf)
+            assert np.array_equal(query(False, False)[0], hits)
+            wide = query(False, True)
+            assert np.array_equal(wide[0], hits)
+            assert np.array_equal(wide[1], frames)
+    finally:
+        scene.close()
+        dev.close()
