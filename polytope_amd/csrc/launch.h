@@ -43,15 +43,19 @@ int noalloc_scratch_address(int ordinal, void **ptr);
 namespace ptx {
 
 uint32_t render_lds_depth();
-// 0 extend, 1 primary, 2 plain megakernel, 3 plain with next-event estimation, 4 shadow connection
+// 0 extend, 1 primary, 2 plain megakernel, 3 plain with next-event estimation, 4 shadow connection;
+// over the four-wide form 5 primary, 6 plain, 7 plain with next-event estimation
 int render_blocks_per_cu(int which);
-void launch_primary(const DevScene &S, const JobDev &J, uint32_t *work, uint4 *spill, uint32_t leaf_min, uint32_t grid,
-                    hipStream_t st);
+// W / wides: the scenes' four-wide forms, which the kernel then steps over
+// (every scene of the launch has one whose stack fits the spill); null = the
+// binary records.
+void launch_primary(const DevScene &S, const WideScene *W, const JobDev &J, uint32_t *work, uint4 *spill,
+                    uint32_t leaf_min, uint32_t grid, hipStream_t st);
 // Primary records of every job of a batch in one launch: jobs / scenes are the
 // device tables, offsets (njobs + 1 entries, device) the first pixel id of
 // each job and the total; max_stack bounds every scene's deferred stack.
-void launch_primaries(const JobDev *jobs, const DevScene *scenes, const uint32_t *offsets, uint32_t njobs,
-                      uint32_t *work, uint4 *spill, uint32_t leaf_min, uint32_t max_stack, uint32_t grid,
+void launch_primaries(const JobDev *jobs, const DevScene *scenes, const WideScene *wides, const uint32_t *offsets,
+                      uint32_t njobs, uint32_t *work, uint4 *spill, uint32_t leaf_min, uint32_t max_stack, uint32_t grid,
                       hipStream_t st);
 // Shadow connection of the wavefront form (rounds with next-event jobs):
 // the vertex queue (48 B per entry, one entry per path slot at most), its
@@ -84,11 +88,12 @@ int paths_blocks_per_cu();
 uint32_t paths_max_chunks();
 uint32_t paths_max_scenes();
 void launch_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jobs, const DevScene *scenes,
-                  uint32_t nscenes, float *res, uint32_t *work, uint4 *spill, uint32_t max_stack, uint32_t shade_min,
-                  uint32_t leaf_min, float4 *nee_scratch, bool glossy, bool textured, uint32_t grid, hipStream_t st);
+                  const WideScene *wides, uint32_t nscenes, float *res, uint32_t *work, uint4 *spill,
+                  uint32_t max_stack, uint32_t shade_min, uint32_t leaf_min, float4 *nee_scratch, bool glossy,
+                  bool textured, uint32_t grid, hipStream_t st);
 // textured: the scene has textured meshes; cached: start every path from the
 // pixel's primary record in J.primary (written by launch_primary).
-void launch_mega(const DevScene &S, const JobDev &J, uint32_t sample, uint4 *spill, bool textured, bool cached,
-                 uint32_t grid, hipStream_t st);
+void launch_mega(const DevScene &S, const WideScene *W, const JobDev &J, uint32_t sample, uint4 *spill, bool textured,
+                 bool cached, uint32_t grid, hipStream_t st);
 
 }  // namespace ptx

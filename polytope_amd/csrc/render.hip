@@ -27,6 +27,7 @@
 #include "launch.h"
 #include "divmagic.h"
 #include "traverse.h"
+#include "wide.h"
 
 #pragma clang fp contract(off)
 
@@ -289,6 +290,26 @@ __device__ __forceinline__ bool occluded(const DevScene &S, const Stack<kLds> &s
    return false;
 }
 
+__device__ __forceinline__ BinaryScene binary_of(const DevScene &S) {
+   return BinaryScene{S.nodes, S.tris, S.root_box, S.root_ref, S.root_count};
+}
+
+// Lanes of a wave that gather at leaves in the inline traversals of k_mega, and
+// idle lanes for which a primary-ray wave takes new pixels.
+constexpr uint32_t kMegaLeafLanes = 24, kWideRefill = 8;
+
+// The same over the four-wide form.
+template <int kLds>
+__device__ __forceinline__ bool occluded(const DevScene &S, const WideScene &W, const WideStack<kLds> &st, float ox,
+                                         float oy, float oz, const float l[3], float tmax) {
+   Trav s;
+   make_ray(s.r, ox, oy, oz, l[0], l[1], l[2]);
+   wide_ray(s.r);
+   wide_begin(s, S.root_box, W.root, tmax);
+   wide_run(s, W, binary_of(S), st, kMegaLeafLanes, false, true);
+   return s.hit != kNone;
+}
+
 __device__ __forceinline__ Frame frame_of(const DevScene &S, uint32_t tri, const float d[3], float u, float v,
                                           float w, uint32_t after, uint32_t mesh) {
    Ray r;
@@ -467,6 +488,96 @@ struct PrimariesPolicy {
       write_primary_record(scenes[J.scene], J, id - offsets[ctx.job], s);
    }
 };
+
+// The same two over the four-wide form: staged policies (wide_trace).
+struct WidePrimary {
+   struct Words {};
+   DevScene S;
+   WideScene W;
+   JobDev J;
+   __device__ __forceinline__ void prepare(uint32_t id, Trav &s, Words &) const {
+      float o[3], d[3];
+      camera_ray(J, id % J.width, id / J.width, o, d);
+      make_ray(s.r, o[0], o[1], o[2], d[0], d[1], d[2]);
+      wide_ray(s.r);
+      wide_begin(s, S.root_box, W.root);
+   }
+   __device__ __forceinline__ Words lane_words(uint32_t, const Words &w) const { return w; }
+   __device__ __forceinline__ const WideNode *nodes(const Words &) const { return W.nodes; }
+   __device__ __forceinline__ const WideFace *faces(const Words &) const { return W.faces; }
+   __device__ __forceinline__ const WideLeaf *leaves(const Words &) const { return W.leaves; }
+   __device__ __forceinline__ BinaryScene binary(const Words &) const { return binary_of(S); }
+   __device__ __forceinline__ bool debug_pixel(uint32_t id, const Words &) const {
+      return J.width > 128u && id == 128u * J.width + 128u;
+   }
+   __device__ __forceinline__ void finish(uint32_t id, const Words &, const Trav &s) const {
+      write_primary_record(S, J, id, s);
+   }
+};
+
+struct WidePrimaries {
+   // job and the job's scene; the arrays a step reads, kept per lane
+   struct Words {
+      uint32_t job, nodes_lo, nodes_hi, faces_lo, faces_hi;
+   };
+   const JobDev *jobs;
+   const DevScene *scenes;
+   const WideScene *wides;
+   const uint32_t *offsets;
+   uint32_t njobs;
+   __device__ __forceinline__ void prepare(uint32_t id, Trav &s, Words &w) const {
+      uint32_t lo = 0, hi = njobs;
+      while (hi - lo > 1) {
+         const uint32_t mid = (lo + hi) / 2;
+         if (offsets[mid] <= id) lo = mid; else hi = mid;
+      }
+      const JobDev &J = jobs[lo];
+      const uint32_t p = id - offsets[lo];
+      float o[3], d[3];
+      camera_ray(J, p % J.width, p / J.width, o, d);
+      make_ray(s.r, o[0], o[1], o[2], d[0], d[1], d[2]);
+      wide_ray(s.r);
+      const WideScene &W = wides[J.scene];
+      wide_begin(s, scenes[J.scene].root_box, W.root);
+      const uint64_t n = reinterpret_cast<uint64_t>(W.nodes), f = reinterpret_cast<uint64_t>(W.faces);
+      w = Words{lo, (uint32_t)n, (uint32_t)(n >> 32), (uint32_t)f, (uint32_t)(f >> 32)};
+   }
+   __device__ __forceinline__ Words lane_words(uint32_t from, const Words &w) const {
+      return Words{lane_read(from, w.job), lane_read(from, w.nodes_lo), lane_read(from, w.nodes_hi),
+                   lane_read(from, w.faces_lo), lane_read(from, w.faces_hi)};
+   }
+   __device__ __forceinline__ const WideNode *nodes(const Words &w) const {
+      return reinterpret_cast<const WideNode *>((uint64_t)w.nodes_lo | (uint64_t)w.nodes_hi << 32);
+   }
+   __device__ __forceinline__ const WideFace *faces(const Words &w) const {
+      return reinterpret_cast<const WideFace *>((uint64_t)w.faces_lo | (uint64_t)w.faces_hi << 32);
+   }
+   __device__ __forceinline__ const WideLeaf *leaves(const Words &w) const { return wides[jobs[w.job].scene].leaves; }
+   __device__ __forceinline__ BinaryScene binary(const Words &w) const { return binary_of(scenes[jobs[w.job].scene]); }
+   __device__ __forceinline__ bool debug_pixel(uint32_t id, const Words &w) const {
+      const uint32_t width = jobs[w.job].width;
+      return width > 128u && id - offsets[w.job] == 128u * width + 128u;
+   }
+   __device__ __forceinline__ void finish(uint32_t id, const Words &w, const Trav &s) const {
+      const JobDev &J = jobs[w.job];
+      write_primary_record(scenes[J.scene], J, id - offsets[w.job], s);
+   }
+};
+
+template <int kLds>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
+k_primary_wide(DevScene S, WideScene W, JobDev J, uint32_t *work, uint2 *spill, uint32_t leaf_min) {
+   const WidePrimary P{S, W, J};
+   wide_trace<kLds>(P, J.width * J.height, work, spill, kWideRefill, leaf_min, W.stack);
+}
+
+template <int kLds>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
+k_primaries_wide(const JobDev *jobs, const DevScene *scenes, const WideScene *wides, const uint32_t *offsets,
+                 uint32_t njobs, uint32_t *work, uint2 *spill, uint32_t leaf_min, uint32_t max_stack) {
+   const WidePrimaries P{jobs, scenes, wides, offsets, njobs};
+   wide_trace<kLds>(P, offsets[njobs], work, spill, kWideRefill, leaf_min, max_stack);
+}
 
 template <int kLds>
 __global__ void __launch_bounds__(256) k_primary(DevScene S, JobDev J, uint32_t *work, uint4 *spill, uint32_t leaf_min) {
@@ -842,6 +953,26 @@ __global__ void k_zero_floats(float *a, size_t n) {
       a[i] = 0.f;
 }
 
+// The deferred stack of a traversal over the binary or the four-wide form, in
+// one block of LDS words.
+template <int kLds, bool kWide>
+struct TraceStack {
+   static constexpr uint32_t kWords = kLds * 256 * 5 / 2;
+   static __device__ __forceinline__ Stack<kLds> make(uint32_t *lds, uint4 *spill, uint32_t max_stack) {
+      return Stack<kLds>{lds, reinterpret_cast<float *>(lds + kLds * 256),
+                         reinterpret_cast<uint16_t *>(lds + 2 * kLds * 256), reinterpret_cast<u32x4 *>(spill),
+                         threadIdx.x, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, max_stack};
+   }
+};
+template <int kLds>
+struct TraceStack<kLds, true> {
+   static constexpr uint32_t kWords = kLds * 256 * 2;
+   static __device__ __forceinline__ WideStack<kLds> make(uint32_t *lds, uint4 *spill, uint32_t max_stack) {
+      return WideStack<kLds>{lds, reinterpret_cast<u32x2 *>(spill), threadIdx.x,
+                             blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, max_stack};
+   }
+};
+
 // ---------------------------------------------------------------- plain path
 
 // One sample of every pixel: one thread per pixel path, all bounces inline.
@@ -849,13 +980,15 @@ __global__ void k_zero_floats(float *a, size_t n) {
 // pixel's primary record (k_primary: CenterSampler gives every sample of a
 // pixel the same primary ray) and traces from bounce 1; otherwise it traces
 // its primary ray itself, as the reference's CUDA path does for every sample.
-template <int kLds, bool kNee, bool kTex, bool kCached>
-__global__ void __launch_bounds__(256) k_mega(DevScene S, JobDev J, uint32_t sample, uint4 *spill) {
-   __shared__ uint32_t lds_ref[kLds * 256];
-   __shared__ float lds_near[kLds * 256];
-   __shared__ uint16_t lds_cnt[kLds * 256];
-   const Stack<kLds> st{lds_ref, lds_near, lds_cnt, reinterpret_cast<u32x4 *>(spill), threadIdx.x,
-                        blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, S.max_stack};
+template <int kLds, bool kNee, bool kTex, bool kCached, bool kWide>
+__global__ void __launch_bounds__(256) k_mega(DevScene S, WideScene W, JobDev J, uint32_t sample, uint4 *spill) {
+   __shared__ uint32_t lds[TraceStack<kLds, kWide>::kWords];
+   const auto st = TraceStack<kLds, kWide>::make(lds, spill, kWide ? W.stack : S.max_stack);
+   if constexpr (kWide) st.sentinel();
+   auto shadowed = [&](float ox, float oy, float oz, const float l[3], float tmax) {
+      if constexpr (kWide) return occluded<kLds>(S, W, st, ox, oy, oz, l, tmax);
+      else return occluded<kLds>(S, st, ox, oy, oz, l, tmax);
+   };
    const uint32_t npix = J.width * J.height;
    for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < npix; p += gridDim.x * blockDim.x) {
       const uint32_t x = p % J.width, y = p / J.width;
@@ -893,7 +1026,7 @@ __global__ void __launch_bounds__(256) k_mega(DevScene S, JobDev J, uint32_t sam
                   const float *light = S.lights + 6 * (size_t)j;
                   float l[3], dist, g;
                   if (!light_setup(light, fr.lx, fr.ly, fr.lz, fr.nx, fr.ny, fr.nz, l, dist, g)) continue;
-                  if (occluded<kLds>(S, st, fr.lx, fr.ly, fr.lz, l, dist)) continue;
+                  if (shadowed(fr.lx, fr.ly, fr.lz, l, dist)) continue;
                   direct[0] = direct[0] + (src[0] * M.refl[0]) * (light[3] * g);
                   direct[1] = direct[1] + (src[1] * M.refl[1]) * (light[4] * g);
                   direct[2] = direct[2] + (src[2] * M.refl[2]) * (light[5] * g);
@@ -912,11 +1045,17 @@ __global__ void __launch_bounds__(256) k_mega(DevScene S, JobDev J, uint32_t sam
          if (src_is_zero(src)) break;
          Trav s;
          make_ray(s.r, o[0], o[1], o[2], d[0], d[1], d[2]);
-         begin(s, S.root_box, S.root_ref, S.root_count);
-         while (s.cur != kNone) {
-            Fetched f;
-            fetch(s, S.nodes, S.tris, f);
-            if (!advance<kLds>(s, f, st, dbg)) break;
+         if constexpr (kWide) {
+            wide_ray(s.r);
+            wide_begin(s, S.root_box, W.root);
+            wide_run(s, W, binary_of(S), st, kMegaLeafLanes, dbg, false);
+         } else {
+            begin(s, S.root_box, S.root_ref, S.root_count);
+            while (s.cur != kNone) {
+               Fetched f;
+               fetch(s, S.nodes, S.tris, f);
+               if (!advance<kLds>(s, f, st, dbg)) break;
+            }
          }
          if (s.hit == kNone) {
             L = miss_radiance(S, src);
@@ -938,7 +1077,7 @@ __global__ void __launch_bounds__(256) k_mega(DevScene S, JobDev J, uint32_t sam
                const float *light = S.lights + 6 * (size_t)j;
                float l[3], dist, g;
                if (!light_setup(light, fr.lx, fr.ly, fr.lz, fr.nx, fr.ny, fr.nz, l, dist, g)) continue;
-               if (occluded<kLds>(S, st, fr.lx, fr.ly, fr.lz, l, dist)) continue;
+               if (shadowed(fr.lx, fr.ly, fr.lz, l, dist)) continue;
                direct[0] = direct[0] + (src[0] * M.refl[0]) * (light[3] * g);
                direct[1] = direct[1] + (src[1] * M.refl[1]) * (light[4] * g);
                direct[2] = direct[2] + (src[2] * M.refl[2]) * (light[5] * g);
@@ -1020,6 +1159,17 @@ __device__ __forceinline__ uint32_t lds_find_chunk(const LdsChunk *c, uint32_t n
    return lo;
 }
 
+// The start of a traversal of s.r (set up by make_ray), bounded by tmax.
+template <bool kWide>
+__device__ __forceinline__ void p_begin(const DevScene &S, uint32_t wroot, Trav &s, float tmax = kInf) {
+   if constexpr (kWide) {
+      wide_ray(s.r);
+      wide_begin(s, S.root_box, wroot, tmax);
+   } else {
+      begin(s, S.root_box, S.root_ref, S.root_count, tmax);
+   }
+}
+
 // Terminal radiance of a path plus its next-event sum (paths of next-event jobs).
 template <bool kNee>
 __device__ __forceinline__ Radiance fin(Radiance R, const float direct[3], uint32_t lane_word) {
@@ -1033,10 +1183,10 @@ __device__ __forceinline__ Radiance fin(Radiance R, const float direct[3], uint3
 
 // Starts the traversal of ray s.r in scene S; returns the next state, or kPIdle
 // after writing the miss result when the root box is missed.
-template <bool kNee>
-__device__ __forceinline__ uint32_t p_root(const DevScene &S, Trav &s, float *res, uint32_t slot,
+template <bool kNee, bool kWide>
+__device__ __forceinline__ uint32_t p_root(const DevScene &S, uint32_t wroot, Trav &s, float *res, uint32_t slot,
                                            const float src[3], const float direct[3], uint32_t lane_word) {
-   begin(s, S.root_box, S.root_ref, S.root_count);
+   p_begin<kWide>(S, wroot, s);
    if (s.cur != kNone) return kPTrace;
    write_res(res, slot, fin<kNee>(miss_radiance(S, src), direct, lane_word));
    return kPIdle;
@@ -1049,16 +1199,17 @@ struct NeeRecord {
 };
 
 // kGlossy: some scene of the round has glossy meshes; kTex: some has textured ones.
-template <int kLds, bool kNee, bool kGlossy, bool kTex>
+// kWide: every scene of the round has a four-wide form, which the traversals
+// step over.
+template <int kLds, bool kNee, bool kGlossy, bool kTex, bool kWide>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
 k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jobs, const DevScene *scenes,
-        uint32_t nscenes, float *res, uint32_t *work, uint4 *spill, uint32_t max_stack, uint32_t shade_min,
-        uint32_t leaf_min, float4 *nee_scratch) {
-   __shared__ uint32_t lds_ref[kLds * 256];
-   __shared__ float lds_near[kLds * 256];
-   __shared__ uint16_t lds_cnt[kLds * 256];
+        const WideScene *wides, uint32_t nscenes, float *res, uint32_t *work, uint4 *spill, uint32_t max_stack,
+        uint32_t shade_min, uint32_t leaf_min, float4 *nee_scratch) {
+   __shared__ uint32_t lds[TraceStack<kLds, kWide>::kWords];
    __shared__ LdsChunk sch[kMaxRoundChunks];
    __shared__ DevScene ssc[kMaxRoundScenes];
+   __shared__ WideScene swd[kWide ? kMaxRoundScenes : 1];
    for (uint32_t i = threadIdx.x; i < nchunks; i += blockDim.x) {
       const Chunk c = chunks[i];
       const JobDev &J = jobs[c.job];
@@ -1068,12 +1219,15 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
       l.primary = J.primary; l.by_npix = div_u32_setup(c.npix);
       sch[i] = l;
    }
-   for (uint32_t i = threadIdx.x; i < nscenes; i += blockDim.x) ssc[i] = scenes[i];
+   for (uint32_t i = threadIdx.x; i < nscenes; i += blockDim.x) {
+      ssc[i] = scenes[i];
+      if constexpr (kWide) swd[i] = wides[i];
+   }
    __syncthreads();
    const uint32_t lane = __lane_id();
    const uint32_t gtid = blockIdx.x * blockDim.x + threadIdx.x;
-   const Stack<kLds> st{lds_ref, lds_near, lds_cnt, reinterpret_cast<u32x4 *>(spill), threadIdx.x,
-                        gtid, gridDim.x * blockDim.x, max_stack};
+   const auto st = TraceStack<kLds, kWide>::make(lds, spill, max_stack);
+   if constexpr (kWide) st.sentinel();
    RaySource srcq;
    srcq.init(nslots, work, lane);
    Trav s;
@@ -1091,8 +1245,24 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
    float src[3] = {1.f, 1.f, 1.f};
    float direct[3] = {0.f, 0.f, 0.f};    // next-event sum of the path (kNee)
    float pend[3] = {0.f, 0.f, 0.f};      // the light term a running shadow ray decides (kNee)
-   const Node64 *nodes = nullptr;
-   const float *tris = nullptr;
+   // the lane's scene arrays: the records its traversal steps over and its faces
+   const std::conditional_t<kWide, WideNode, Node64> *nodes = nullptr;
+   const std::conditional_t<kWide, WideFace, float> *tris = nullptr;
+   auto scene_of = [&](uint32_t lane_word) { return sch[lw_chunk(lane_word)].scene; };
+   // the 9 corner coordinates of the hit's face
+   auto hit_corners = [&](float *v) {
+      if constexpr (kWide) {
+         const PTX_GLOBAL f32x4u *p = as_global(reinterpret_cast<const f32x4u *>(tris + s.hit));
+         const f32x4u a = p[0], b = p[1];
+         v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+         v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+         v[8] = as_global(reinterpret_cast<const float *>(tris + s.hit))[8];
+      } else {
+         const PTX_GLOBAL float *p = as_global(tris + 9 * (size_t)s.hit);
+#pragma unroll
+         for (int j = 0; j < 9; j++) v[j] = p[j];
+      }
+   };
    // At a Lambert vertex of a next-event job: keep the vertex in this lane's
    // record and go through the lights before tracing the bounce ray.
    auto nee_vertex = [&](const Frame &fr, const float refl[3], const float wout[3], uint32_t next_mode) {
@@ -1126,23 +1296,66 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
             srcq.pool_left -= take;
          }
       }
-      const uint32_t m0 = mode & kPModeMask;
+      uint32_t m0 = mode & kPModeMask;
       if (!__any(m0 != kPIdle)) break;
+      uint32_t shade_now = shade_min;
+      if constexpr (kWide) {
+         // node steps until leaf_min lanes are at leaves, or shade_min have ended
+         // or wait for something else; then a leaf step
+         const bool tr = m0 == kPTrace || m0 == kPShadow;
+         const uint32_t waiting =
+               (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(!tr && (m0 != kPIdle || !srcq.done)));
+         const uint32_t busy = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(m0 != kPIdle));
+         const uint32_t leaf_now = wide_gather(leaf_min, busy);
+         shade_now = wide_gather(shade_min, busy);
+         const bool shadow = kNee && m0 == kPShadow;
+         while (true) {
+            const bool node = tr && (int)s.cur >= 0;
+            if (!__builtin_amdgcn_ballot_w64(node)) break;
+            if (node) wide_node_step(s, nodes, st);
+            const uint32_t held = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(tr && (int)s.cur < 0 && s.cur != kNone));
+            const uint32_t ended = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(tr && s.cur == kNone));
+            if (held >= leaf_now || waiting + ended >= shade_now) break;
+         }
+         const bool leaf = tr && (int)s.cur < 0 && s.cur != kNone;
+         if ((uint32_t)__popcll(__builtin_amdgcn_ballot_w64(leaf)) >= leaf_now ||
+             !__builtin_amdgcn_ballot_w64(tr && (int)s.cur >= 0)) {
+            if (leaf) {
+               const uint32_t sc = scene_of(mode);
+               wide_leaf_or_exact(s, tris, swd[sc].leaves, binary_of(ssc[sc]), st, !shadow && (mode & kPDbg) != 0,
+                                  shadow);
+               if (shadow && s.hit != kNone) s.cur = kNone;      // occluded
+            }
+         }
+         if (tr && s.cur == kNone) {
+            if (shadow) {
+               t1 = s.hit == kNone ? 1.f : 0.f;
+               mode = lw_with_state(mode, kPLight);
+            } else if (s.hit == kNone) {
+               write_res(res, slot, fin<kNee>(miss_radiance(ssc[scene_of(mode)], src), direct, mode));
+               mode = kPIdle;
+            } else {
+               t0 = s.mesh;
+               mode = lw_with_state(mode, kTex ? kPShade1 : kPShade2);
+            }
+            m0 = mode & kPModeMask;
+         }
+      }
       const bool heavy = m0 == kPPrim || m0 == kPShade2 || m0 == kPShade3;
       const bool tracing = m0 == kPTrace || m0 == kPShadow;
       // single-load steps that never wait for the wave
       const bool light_step = m0 == kPShade1 || m0 == kPLight;
-      const bool run_heavy = (uint32_t)__popcll(__ballot(heavy)) >= shade_min || !__any(tracing || light_step);
+      const bool run_heavy = (uint32_t)__popcll(__ballot(heavy)) >= shade_now || !__any(tracing || light_step);
       // leaf steps gather the same way; lanes at interior nodes, in Shade1 or in
       // Light always step, so some lane progresses whenever any lane holds
       const bool at_leaf = tracing && (s.cur & kLeafBit) != 0;
       const bool run_leaf = (uint32_t)__popcll(__ballot(at_leaf)) >= leaf_min ||
                             !__any((tracing && !at_leaf) || light_step);
-      const uint32_t m = (heavy && !run_heavy) || (at_leaf && !run_leaf) ? kPHold : m0;
+      const uint32_t m = (heavy && !run_heavy) || (kWide ? tracing : at_leaf && !run_leaf) ? kPHold : m0;
       // ------------------------------------------------------------ fetch
       Fetched f;
-      if (m == kPTrace || m == kPShadow) {
-         fetch(s, nodes, tris, f);
+      if (!kWide && (m == kPTrace || m == kPShadow)) {
+         if constexpr (!kWide) fetch(s, nodes, tris, f);
       } else if (m == kPPrim) {
          const uint32_t cf = lds_find_chunk(sch, nchunks, slot);
          mode = kPPrim | (cf << kPChunkShift);
@@ -1157,7 +1370,7 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
          f.q[12] = q3.x; f.q[13] = q3.y; f.q[14] = q3.z; f.q[15] = q3.w;
       } else if (m == kPShade1) {
          const DevScene &S = ssc[sch[lw_chunk(mode)].scene];
-         f.q[0] = __uint_as_float(as_global(S.pairs)[2 * (size_t)s.hit]);
+         if (!kWide) f.q[0] = __uint_as_float(as_global(S.pairs)[2 * (size_t)s.hit]);
          if (kTex) {                                // the triangle's texture record (flags 0 without one)
             f.q[7] = 0.f;
             if (S.tex_tris) {
@@ -1177,14 +1390,12 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
 #pragma unroll
             for (int k = 0; k < 9; k++) f.q[k] = __uint_as_float(mr[k]);
          }
-         const PTX_GLOBAL float *v = as_global(tris + 9 * (size_t)s.hit);
-#pragma unroll
-         for (int k = 0; k < 9; k++) f.q[9 + k] = v[k];
+         hit_corners(&f.q[9]);
       } else if (m == kPShade3) {
-         const PTX_GLOBAL float *v = as_global(tris + 9 * (size_t)s.hit);
+         hit_corners(&f.q[0]);
          const PTX_GLOBAL float *nrm = as_global(ssc[sch[lw_chunk(mode)].scene].normals + 9 * (size_t)s.hit);
 #pragma unroll
-         for (int k = 0; k < 9; k++) { f.q[k] = v[k]; f.q[9 + k] = nrm[k]; }
+         for (int k = 0; k < 9; k++) f.q[9 + k] = nrm[k];
       } else if (kNee && m == kPLight) {
          const PTX_GLOBAL f32x4u *rec = as_global(reinterpret_cast<const f32x4u *>(nee_scratch + 3 * (size_t)gtid));
          const f32x4u a = rec[0], b = rec[1], c = rec[2];
@@ -1201,8 +1412,10 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
          }
       }
       // ------------------------------------------------------------ compute
-      if (m == kPTrace) {
-         if (!advance<kLds>(s, f, st, (mode & kPDbg) != 0)) {
+      if (!kWide && m == kPTrace) {
+         bool more = false;
+         if constexpr (!kWide) more = advance<kLds>(s, f, st, (mode & kPDbg) != 0);
+         if (!more) {
             if (s.hit == kNone) {
                write_res(res, slot, fin<kNee>(miss_radiance(ssc[sch[lw_chunk(mode)].scene], src), direct, mode));
                mode = kPIdle;
@@ -1210,8 +1423,9 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
                mode = lw_with_state(mode, kPShade1);
             }
          }
-      } else if (kNee && m == kPShadow) {
-         const bool more = advance<kLds>(s, f, st, false);
+      } else if (!kWide && kNee && m == kPShadow) {
+         bool more = false;
+         if constexpr (!kWide) more = advance<kLds>(s, f, st, false);
          if (s.hit != kNone) {                    // occluded
             t1 = 0.f;
             mode = lw_with_state(mode, kPLight);
@@ -1236,7 +1450,7 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
                pend[1] = f.q[7] * (f.q[16] * g);
                pend[2] = f.q[8] * (f.q[17] * g);
                make_ray(s.r, f.q[0], f.q[1], f.q[2], l[0], l[1], l[2]);
-               begin(s, S.root_box, S.root_ref, S.root_count, dist);
+               p_begin<kWide>(S, kWide ? swd[scene_of(mode)].root : 0u, s, dist);
                if (s.cur == kNone) t1 = 1.f;       // root box missed: nothing in the way
                else mode = lw_with_state(mode, kPShadow);
             }
@@ -1245,7 +1459,8 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
             mode = kPIdle;
          } else {                                 // trace the bounce ray
             make_ray(s.r, f.q[0], f.q[1], f.q[2], f.q[3], f.q[4], f.q[5]);
-            const uint32_t next = p_root<kNee>(S, s, res, slot, src, direct, mode);
+            const uint32_t next = p_root<kNee, kWide>(S, kWide ? swd[scene_of(mode)].root : 0u, s, res, slot, src,
+                                                      direct, mode);
             mode = next == kPIdle ? kPIdle : lw_with_state(mode, next);
          }
       } else {
@@ -1302,7 +1517,7 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
                shade = true;
             }
          } else if (m == kPShade1) {
-            t0 = __float_as_uint(f.q[0]);
+            if (!kWide) t0 = __float_as_uint(f.q[0]);
             if (kTex) {
                const uint32_t wh = __float_as_uint(f.q[7]);
                s.r.oy = f.q[7];                    // the texture record's flags
@@ -1401,8 +1616,13 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
             const float s_before[3] = {src[0], src[1], src[2]};
             float wout[3];
             bounce<kGlossy>(M, fr, lin, pixel, sample, b, seed, wout, src);
-            nodes = S.nodes;
-            tris = S.tris;
+            if constexpr (kWide) {
+               nodes = swd[scene].nodes;
+               tris = swd[scene].faces;
+            } else {
+               nodes = S.nodes;
+               tris = S.tris;
+            }
             if (nee) {
                const float keep[3] = {src[0], src[1], src[2]};
                src[0] = s_before[0]; src[1] = s_before[1]; src[2] = s_before[2];
@@ -1414,7 +1634,8 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
                mode = kPIdle;
             } else {
                make_ray(s.r, fr.lx, fr.ly, fr.lz, wout[0], wout[1], wout[2]);
-               const uint32_t next = p_root<kNee>(S, s, res, slot, src, direct, mode);
+               const uint32_t next =
+                     p_root<kNee, kWide>(S, kWide ? swd[scene].root : 0u, s, res, slot, src, direct, mode);
                mode = next == kPIdle ? kPIdle : nb | next;
             }
          }
@@ -1434,26 +1655,41 @@ uint32_t render_lds_depth() { return kRenderLds; }
 int render_blocks_per_cu(int which) {
    int b = 0;
    hipError_t e = hipSuccess;
-   if (which == 0) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, dev::k_extend<kRenderLds>, 256, 0);
-   else if (which == 1) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, dev::k_primary<kRenderLds>, 256, 0);
-   else if (which == 2) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, dev::k_mega<kRenderLds, false, false, false>, 256, 0);
-   else if (which == 3) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, dev::k_mega<kRenderLds, true, false, false>, 256, 0);
-   else e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, dev::k_connect<kRenderLds>, 256, 0);
+#define PTX_OCC(...) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, __VA_ARGS__, 256, 0)
+   switch (which) {
+      case 0: PTX_OCC(dev::k_extend<kRenderLds>); break;
+      case 1: PTX_OCC(dev::k_primary<kRenderLds>); break;
+      case 2: PTX_OCC((dev::k_mega<kRenderLds, false, false, false, false>)); break;
+      case 3: PTX_OCC((dev::k_mega<kRenderLds, true, false, false, false>)); break;
+      case 4: PTX_OCC(dev::k_connect<kRenderLds>); break;
+      case 5: PTX_OCC(dev::k_primaries_wide<kRenderLds>); break;
+      case 6: PTX_OCC((dev::k_mega<kRenderLds, false, false, true, true>)); break;
+      default: PTX_OCC((dev::k_mega<kRenderLds, true, false, true, true>)); break;
+   }
+#undef PTX_OCC
    return e == hipSuccess && b > 0 ? b : 1;
 }
 
-void launch_primary(const DevScene &S, const JobDev &J, uint32_t *work, uint4 *spill, uint32_t leaf_min, uint32_t grid,
-                    hipStream_t st) {
+void launch_primary(const DevScene &S, const WideScene *W, const JobDev &J, uint32_t *work, uint4 *spill,
+                    uint32_t leaf_min, uint32_t grid, hipStream_t st) {
    hipLaunchKernelGGL(dev::k_zero_words, dim3(1), dim3(64), 0, st, work, 8u, (uint32_t *)nullptr, 0u);
-   hipLaunchKernelGGL(dev::k_primary<kRenderLds>, dim3(grid), dim3(256), 0, st, S, J, work, spill, leaf_min);
+   if (W)
+      hipLaunchKernelGGL(dev::k_primary_wide<kRenderLds>, dim3(grid), dim3(256), 0, st, S, *W, J, work,
+                         reinterpret_cast<uint2 *>(spill), leaf_min);
+   else
+      hipLaunchKernelGGL(dev::k_primary<kRenderLds>, dim3(grid), dim3(256), 0, st, S, J, work, spill, leaf_min);
 }
 
-void launch_primaries(const JobDev *jobs, const DevScene *scenes, const uint32_t *offsets, uint32_t njobs,
-                      uint32_t *work, uint4 *spill, uint32_t leaf_min, uint32_t max_stack, uint32_t grid,
-                      hipStream_t st) {
+void launch_primaries(const JobDev *jobs, const DevScene *scenes, const WideScene *wides, const uint32_t *offsets,
+                      uint32_t njobs, uint32_t *work, uint4 *spill, uint32_t leaf_min, uint32_t max_stack,
+                      uint32_t grid, hipStream_t st) {
    hipLaunchKernelGGL(dev::k_zero_words, dim3(1), dim3(64), 0, st, work, 8u, (uint32_t *)nullptr, 0u);
-   hipLaunchKernelGGL(dev::k_primaries<kRenderLds>, dim3(grid), dim3(256), 0, st, jobs, scenes, offsets, njobs, work,
-                      spill, leaf_min, max_stack);
+   if (wides)
+      hipLaunchKernelGGL(dev::k_primaries_wide<kRenderLds>, dim3(grid), dim3(256), 0, st, jobs, scenes, wides, offsets,
+                         njobs, work, reinterpret_cast<uint2 *>(spill), leaf_min, max_stack);
+   else
+      hipLaunchKernelGGL(dev::k_primaries<kRenderLds>, dim3(grid), dim3(256), 0, st, jobs, scenes, offsets, njobs,
+                         work, spill, leaf_min, max_stack);
 }
 
 void launch_round_start(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jobs,
@@ -1500,39 +1736,41 @@ void launch_zero_floats(float *a, size_t n, hipStream_t st) {
 }
 
 int paths_blocks_per_cu() {
-   int b[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-   hipError_t e[8];
-#define PTX_PATHS_OCC(I, N, G, T) \
-   e[I] = hipOccupancyMaxActiveBlocksPerMultiprocessor(&b[I], dev::k_paths<kRenderLds, N, G, T>, 256, 0)
-   PTX_PATHS_OCC(0, false, false, false);
-   PTX_PATHS_OCC(1, true, false, false);
-   PTX_PATHS_OCC(2, false, true, false);
-   PTX_PATHS_OCC(3, true, true, false);
-   PTX_PATHS_OCC(4, false, false, true);
-   PTX_PATHS_OCC(5, true, false, true);
-   PTX_PATHS_OCC(6, false, true, true);
-   PTX_PATHS_OCC(7, true, true, true);
+   int least = 1 << 30;
+   bool ok = true;
+   auto occ = [&](auto *kernel) {
+      int b = 0;
+      ok = ok && hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, kernel, 256, 0) == hipSuccess;
+      least = std::min(least, b);
+   };
+#define PTX_PATHS_OCC(N, G, T)                     \
+   occ(dev::k_paths<kRenderLds, N, G, T, false>); \
+   occ(dev::k_paths<kRenderLds, N, G, T, true>)
+   PTX_PATHS_OCC(false, false, false);
+   PTX_PATHS_OCC(true, false, false);
+   PTX_PATHS_OCC(false, true, false);
+   PTX_PATHS_OCC(true, true, false);
+   PTX_PATHS_OCC(false, false, true);
+   PTX_PATHS_OCC(true, false, true);
+   PTX_PATHS_OCC(false, true, true);
+   PTX_PATHS_OCC(true, true, true);
 #undef PTX_PATHS_OCC
-   int m = b[0];
-   for (int i = 0; i < 8; i++) {
-      if (e[i] != hipSuccess) return 1;
-      m = std::min(m, b[i]);
-   }
-   return std::max(1, m);   // one grid and one scratch area serve every variant
+   return ok ? std::max(1, least) : 1;   // one grid and one scratch area serve every variant
 }
 
 uint32_t paths_max_chunks() { return kMaxRoundChunks; }
 uint32_t paths_max_scenes() { return dev::kMaxRoundScenes; }
 
-void launch_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jobs, const DevScene *scenes,
-                  uint32_t nscenes, float *res, uint32_t *work, uint4 *spill, uint32_t max_stack, uint32_t shade_min,
-                  uint32_t leaf_min, float4 *nee_scratch, bool glossy, bool textured, uint32_t grid, hipStream_t st) {
-   hipLaunchKernelGGL(dev::k_zero_words, dim3(1), dim3(64), 0, st, work, 8u, (uint32_t *)nullptr, 0u);
-#define PTX_LAUNCH_PATHS(N, G, T)                                                                                     \
-   hipLaunchKernelGGL((dev::k_paths<kRenderLds, N, G, T>), dim3(grid), dim3(256), 0, st, chunks, nchunks, nslots, jobs, \
-                      scenes, nscenes, res, work, spill, max_stack, shade_min, leaf_min, nee_scratch)
-   const int v = (nee_scratch ? 1 : 0) | (glossy ? 2 : 0) | (textured ? 4 : 0);
-   switch (v) {
+namespace {
+template <bool W>
+void launch_paths_t(int variant, const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jobs,
+                    const DevScene *scenes, const WideScene *wides, uint32_t nscenes, float *res, uint32_t *work,
+                    uint4 *spill, uint32_t max_stack, uint32_t shade_min, uint32_t leaf_min, float4 *nee_scratch,
+                    uint32_t grid, hipStream_t st) {
+#define PTX_LAUNCH_PATHS(N, G, T)                                                                                  \
+   hipLaunchKernelGGL((dev::k_paths<kRenderLds, N, G, T, W>), dim3(grid), dim3(256), 0, st, chunks, nchunks, nslots, \
+                      jobs, scenes, wides, nscenes, res, work, spill, max_stack, shade_min, leaf_min, nee_scratch)
+   switch (variant) {
       case 0: PTX_LAUNCH_PATHS(false, false, false); break;
       case 1: PTX_LAUNCH_PATHS(true, false, false); break;
       case 2: PTX_LAUNCH_PATHS(false, true, false); break;
@@ -1544,26 +1782,50 @@ void launch_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const 
    }
 #undef PTX_LAUNCH_PATHS
 }
+}  // namespace
+
+void launch_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jobs, const DevScene *scenes,
+                  const WideScene *wides, uint32_t nscenes, float *res, uint32_t *work, uint4 *spill,
+                  uint32_t max_stack, uint32_t shade_min, uint32_t leaf_min, float4 *nee_scratch, bool glossy,
+                  bool textured, uint32_t grid, hipStream_t st) {
+   hipLaunchKernelGGL(dev::k_zero_words, dim3(1), dim3(64), 0, st, work, 8u, (uint32_t *)nullptr, 0u);
+   const int v = (nee_scratch ? 1 : 0) | (glossy ? 2 : 0) | (textured ? 4 : 0);
+   if (wides)
+      launch_paths_t<true>(v, chunks, nchunks, nslots, jobs, scenes, wides, nscenes, res, work, spill, max_stack,
+                           shade_min, leaf_min, nee_scratch, grid, st);
+   else
+      launch_paths_t<false>(v, chunks, nchunks, nslots, jobs, scenes, wides, nscenes, res, work, spill, max_stack,
+                            shade_min, leaf_min, nee_scratch, grid, st);
+}
 
 namespace {
-template <bool T, bool C>
-void launch_mega_t(const DevScene &S, const JobDev &J, uint32_t sample, uint4 *spill, uint32_t grid, hipStream_t st) {
+template <bool T, bool C, bool W>
+void launch_mega_t(const DevScene &S, const WideScene &wide, const JobDev &J, uint32_t sample, uint4 *spill,
+                   uint32_t grid, hipStream_t st) {
    if (J.flags & PTX_JOB_NEE)
-      hipLaunchKernelGGL((dev::k_mega<kRenderLds, true, T, C>), dim3(grid), dim3(256), 0, st, S, J, sample, spill);
+      hipLaunchKernelGGL((dev::k_mega<kRenderLds, true, T, C, W>), dim3(grid), dim3(256), 0, st, S, wide, J, sample,
+                         spill);
    else
-      hipLaunchKernelGGL((dev::k_mega<kRenderLds, false, T, C>), dim3(grid), dim3(256), 0, st, S, J, sample, spill);
+      hipLaunchKernelGGL((dev::k_mega<kRenderLds, false, T, C, W>), dim3(grid), dim3(256), 0, st, S, wide, J, sample,
+                         spill);
+}
+template <bool W>
+void launch_mega_w(const DevScene &S, const WideScene &wide, const JobDev &J, uint32_t sample, uint4 *spill,
+                   bool textured, bool cached, uint32_t grid, hipStream_t st) {
+   if (cached) {
+      if (textured) launch_mega_t<true, true, W>(S, wide, J, sample, spill, grid, st);
+      else launch_mega_t<false, true, W>(S, wide, J, sample, spill, grid, st);
+   } else {
+      if (textured) launch_mega_t<true, false, W>(S, wide, J, sample, spill, grid, st);
+      else launch_mega_t<false, false, W>(S, wide, J, sample, spill, grid, st);
+   }
 }
 }  // namespace
 
-void launch_mega(const DevScene &S, const JobDev &J, uint32_t sample, uint4 *spill, bool textured, bool cached,
-                 uint32_t grid, hipStream_t st) {
-   if (cached) {
-      if (textured) launch_mega_t<true, true>(S, J, sample, spill, grid, st);
-      else launch_mega_t<false, true>(S, J, sample, spill, grid, st);
-   } else {
-      if (textured) launch_mega_t<true, false>(S, J, sample, spill, grid, st);
-      else launch_mega_t<false, false>(S, J, sample, spill, grid, st);
-   }
+void launch_mega(const DevScene &S, const WideScene *W, const JobDev &J, uint32_t sample, uint4 *spill, bool textured,
+                 bool cached, uint32_t grid, hipStream_t st) {
+   if (W) launch_mega_w<true>(S, *W, J, sample, spill, textured, cached, grid, st);
+   else launch_mega_w<false>(S, WideScene{}, J, sample, spill, textured, cached, grid, st);
 }
 
 }  // namespace ptx

@@ -148,7 +148,7 @@ void RenderEngine::release() {
    }
    dfree(qa); dfree(qb); dfree(hits); dfree(qs); dfree(direct); dfree(res); dfree(words); dfree(spill);
    dfree(nee_scratch);
-   dfree(d_jobs); dfree(d_offsets); dfree(d_scenes); dfree(d_chunks);
+   dfree(d_jobs); dfree(d_offsets); dfree(d_scenes); dfree(d_wides); dfree(d_chunks);
    cap = qcap = 0;
    jobs_cap = scenes_cap = chunks_cap = 0;
    spill_entries = 0;
@@ -165,7 +165,8 @@ bool RenderEngine::regen_round(uint32_t nchunks, uint32_t nscenes) const {
           nscenes <= paths_max_scenes();
 }
 
-int RenderEngine::ensure(uint32_t paths, uint32_t max_stack, uint32_t njobs, uint32_t nscenes, uint32_t nchunks) {
+int RenderEngine::ensure(uint32_t paths, uint32_t max_stack, uint32_t wide_stack, uint32_t njobs, uint32_t nscenes,
+                         uint32_t nchunks) {
    const uint32_t lds = render_lds_depth();
    if (!ext_grid) {
       ext_grid = (uint32_t)(dev->num_cus * render_blocks_per_cu(0));
@@ -174,9 +175,16 @@ int RenderEngine::ensure(uint32_t paths, uint32_t max_stack, uint32_t njobs, uin
       mega_nee_grid = (uint32_t)(dev->num_cus * render_blocks_per_cu(3));
       paths_grid = (uint32_t)(dev->num_cus * paths_blocks_per_cu());
       connect_grid = (uint32_t)(dev->num_cus * render_blocks_per_cu(4));
+      primary_wide_grid = (uint32_t)(dev->num_cus * render_blocks_per_cu(5));
+      mega_wide_grid = (uint32_t)(dev->num_cus * render_blocks_per_cu(6));
+      mega_wide_nee_grid = (uint32_t)(dev->num_cus * render_blocks_per_cu(7));
    }
-   const uint32_t stride_threads = std::max({ext_grid, mega_grid, mega_nee_grid, paths_grid, connect_grid}) * 256;
-   const size_t need_spill = max_stack > lds ? (size_t)(max_stack - lds) * stride_threads : 0;
+   const uint32_t stride_threads = std::max({ext_grid, mega_grid, mega_nee_grid, paths_grid, connect_grid,
+                                             primary_wide_grid, mega_wide_grid, mega_wide_nee_grid}) * 256;
+   // 16-byte entries of the binary stack, or 8-byte ones of the four-wide
+   const uint32_t levels = std::max(max_stack > lds ? max_stack - lds : 0u,
+                                    wide_stack > lds ? (wide_stack - lds + 1) / 2 : 0u);
+   const size_t need_spill = (size_t)levels * stride_threads;
    int rc;
    if (paths > cap) {
       dfree(res);
@@ -201,6 +209,7 @@ int RenderEngine::ensure(uint32_t paths, uint32_t max_stack, uint32_t njobs, uin
       stack_cap = max_stack;
       graphs_stale = true;
    }
+   wide_cap = lds + 2 * (uint32_t)(spill_entries / stride_threads);
    // a table's capacity is recorded only once its allocation succeeded
    if (njobs > jobs_cap) {
       dfree(d_jobs);
@@ -214,9 +223,11 @@ int RenderEngine::ensure(uint32_t paths, uint32_t max_stack, uint32_t njobs, uin
    }
    if (nscenes > scenes_cap) {
       dfree(d_scenes);
+      dfree(d_wides);
       scenes_cap = 0;
       const uint32_t want = std::max(nscenes, 16u);
       if ((rc = dalloc(this, &d_scenes, want))) return rc;
+      if ((rc = dalloc(this, &d_wides, want))) return rc;
       scenes_cap = want;
       graphs_stale = true;
    }
@@ -321,7 +332,13 @@ std::vector<std::vector<Chunk>> schedule_rounds(const std::vector<RenderJob> &jo
    return rounds;
 }
 
-int RenderEngine::start_job(JobDev &J, const DevScene &S, uint32_t npix, bool trace_primary) {
+void RenderEngine::trace_primary_of(const JobDev &J, const ptx_scene *scene, uint32_t npix) {
+   const bool wide = wide_scene(scene);
+   launch_primary(scene->d, wide ? &scene->w : nullptr, J, words + kWork, spill, leaf_lanes_of(tun, true),
+                  std::min<uint32_t>(wide ? primary_wide_grid : ext_grid, (npix + 255) / 256), stream);
+}
+
+int RenderEngine::start_job(JobDev &J, const ptx_scene *scene, uint32_t npix, bool trace_primary) {
    // stream-ordered: a job's buffers come and go between the rounds that use
    // them without waiting for the device
    J.film = nullptr;
@@ -334,14 +351,12 @@ int RenderEngine::start_job(JobDev &J, const DevScene &S, uint32_t npix, bool tr
       return set_error(PTX_ERR_OOM, std::string("job film and primary records: ") + hipGetErrorString(e));
    }
    launch_zero_floats(J.film, (size_t)npix * 3, stream);
-   if (trace_primary)
-      launch_primary(S, J, words + kWork, spill, leaf_lanes_of(tun, true),
-                     std::min<uint32_t>(ext_grid, (npix + 255) / 256), stream);
+   if (trace_primary) trace_primary_of(J, scene, npix);
    return PTX_OK;
 }
 
 int RenderEngine::round(const Chunk *d_round, const std::vector<Chunk> &r, uint32_t depth, uint32_t nscenes,
-                       bool nee, bool glossy, bool textured) {
+                       bool nee, bool glossy, bool textured, bool wide) {
    uint32_t nslots = 0;
    for (const Chunk &c : r) nslots = std::max(nslots, c.base + c.k * c.npix);
    if (nee && regen_round((uint32_t)r.size(), nscenes) && !nee_scratch) {
@@ -350,8 +365,8 @@ int RenderEngine::round(const Chunk *d_round, const std::vector<Chunk> &r, uint3
    }
    if (regen_round((uint32_t)r.size(), nscenes)) {
       const uint32_t shade_min = tun.shade_lanes ? tun.shade_lanes : kDefaultShadeLanes;
-      launch_paths(d_round, (uint32_t)r.size(), nslots, d_jobs, d_scenes, nscenes, res, words + kWork, spill, stack_cap,
-                   shade_min, leaf_lanes_of(tun, true), nee ? nee_scratch : nullptr, glossy, textured,
+      launch_paths(d_round, (uint32_t)r.size(), nslots, d_jobs, d_scenes, wide ? d_wides : nullptr, nscenes, res,
+                   words + kWork, spill, wide ? wide_cap : stack_cap, shade_min, leaf_lanes_of(tun, true), nee ? nee_scratch : nullptr, glossy, textured,
                    std::min<uint32_t>(paths_grid, (nslots + 255) / 256), stream);
       launch_accumulate(d_round, (uint32_t)r.size(), d_jobs, res, nullptr, shade_grid, stream);
       return PTX_OK;
@@ -398,9 +413,12 @@ uint32_t RenderEngine::capacity_for(uint64_t total_paths, uint32_t max_npix, boo
 int RenderEngine::run_batch(const std::vector<RenderJob> &jobs, const std::vector<const ptx_scene *> &scenes,
                             const std::vector<float *> &films_host) {
    const uint32_t nj = (uint32_t)jobs.size();
-   uint32_t max_stack = 1, max_npix = 1;
+   uint32_t max_stack = 1, wide_stack = 0, max_npix = 1;
    uint64_t total_paths = 0;
-   for (const auto *s : scenes) max_stack = std::max(max_stack, s->d.max_stack);
+   for (const auto *s : scenes) {
+      max_stack = std::max(max_stack, s->d.max_stack);
+      wide_stack = std::max(wide_stack, s->w.stack);
+   }
    for (const auto &j : jobs) {
       max_npix = std::max(max_npix, j.npix);
       total_paths += (uint64_t)j.npix * j.desc.spp;
@@ -410,7 +428,7 @@ int RenderEngine::run_batch(const std::vector<RenderJob> &jobs, const std::vecto
    const auto rounds = schedule_rounds(jobs, paths, regen ? paths_max_chunks() : 0xFFFFFFFFu);
    size_t nchunks = 0;
    for (const auto &r : rounds) nchunks += r.size();
-   int rc = ensure(paths, max_stack, nj, (uint32_t)scenes.size(), (uint32_t)nchunks);
+   int rc = ensure(paths, max_stack, wide_stack, nj, (uint32_t)scenes.size(), (uint32_t)nchunks);
    if (rc) return rc;
    hipStream_t st = stream;
    std::vector<JobDev> jd(nj);
@@ -418,7 +436,13 @@ int RenderEngine::run_batch(const std::vector<RenderJob> &jobs, const std::vecto
       for (auto &J : jd) free_job(J);
    };
    std::vector<DevScene> sd(scenes.size());
-   for (size_t i = 0; i < scenes.size(); i++) sd[i] = scenes[i]->d;
+   std::vector<WideScene> wd(scenes.size());
+   bool wide = true;
+   for (size_t i = 0; i < scenes.size(); i++) {
+      sd[i] = scenes[i]->d;
+      wd[i] = scenes[i]->w;
+      wide = wide && wide_scene(scenes[i]);
+   }
    // every job's primary rays in one launch once the tables are up (one
    // launch per job when the batch has more pixels than 32-bit ids cover)
    std::vector<uint32_t> offsets(nj + 1, 0);
@@ -431,7 +455,7 @@ int RenderEngine::run_batch(const std::vector<RenderJob> &jobs, const std::vecto
    offsets[nj] = (uint32_t)total_pixels;
    for (uint32_t j = 0; j < nj; j++) {
       jd[j] = job_dev(jobs[j].desc, jobs[j].scene_index);
-      if ((rc = start_job(jd[j], sd[jobs[j].scene_index], jobs[j].npix, !one_launch))) {
+      if ((rc = start_job(jd[j], scenes[jobs[j].scene_index], jobs[j].npix, !one_launch))) {
          (void)hipStreamSynchronize(st);
          cleanup();
          return rc;
@@ -445,6 +469,8 @@ int RenderEngine::run_batch(const std::vector<RenderJob> &jobs, const std::vecto
       hipError_t e = hipMemcpyAsync(d_jobs, jd.data(), nj * sizeof(JobDev), hipMemcpyHostToDevice, st);
       if (e == hipSuccess)
          e = hipMemcpyAsync(d_scenes, sd.data(), sd.size() * sizeof(DevScene), hipMemcpyHostToDevice, st);
+      if (e == hipSuccess && wide)
+         e = hipMemcpyAsync(d_wides, wd.data(), wd.size() * sizeof(WideScene), hipMemcpyHostToDevice, st);
       if (e == hipSuccess && !all.empty())
          e = hipMemcpyAsync(d_chunks, all.data(), all.size() * sizeof(Chunk), hipMemcpyHostToDevice, st);
       if (e == hipSuccess && one_launch)
@@ -457,8 +483,10 @@ int RenderEngine::run_batch(const std::vector<RenderJob> &jobs, const std::vecto
       }
    }
    if (one_launch)
-      launch_primaries(d_jobs, d_scenes, d_offsets, nj, words + kWork, spill, leaf_lanes_of(tun, true), max_stack,
-                       (uint32_t)std::min<uint64_t>(ext_grid, (total_pixels + 255) / 256), st);
+      launch_primaries(d_jobs, d_scenes, wide ? d_wides : nullptr, d_offsets, nj, words + kWork, spill,
+                       leaf_lanes_of(tun, true), wide ? wide_cap : max_stack,
+                       (uint32_t)std::min<uint64_t>(wide ? primary_wide_grid : ext_grid, (total_pixels + 255) / 256),
+                       st);
    size_t off = 0;
    for (const auto &r : rounds) {
       uint32_t depth = 0;
@@ -469,7 +497,7 @@ int RenderEngine::run_batch(const std::vector<RenderJob> &jobs, const std::vecto
          glossy |= scenes[jobs[c.job].scene_index]->has_glossy;
          textured |= scenes[jobs[c.job].scene_index]->has_texture;
       }
-      if ((rc = round(d_chunks + off, r, depth, (uint32_t)scenes.size(), nee, glossy, textured))) {
+      if ((rc = round(d_chunks + off, r, depth, (uint32_t)scenes.size(), nee, glossy, textured, wide))) {
          (void)hipStreamSynchronize(st);
          cleanup();
          return rc;
@@ -495,7 +523,7 @@ int RenderEngine::run_batch(const std::vector<RenderJob> &jobs, const std::vecto
 
 int RenderEngine::run_plain(const ptx_scene *scene, const ptx_job_desc &desc, float *film_host) {
    const uint32_t npix = desc.camera.width * desc.camera.height;
-   int rc = ensure(cap ? cap : 1u, scene->d.max_stack, 1, 1, 1);
+   int rc = ensure(cap ? cap : 1u, scene->d.max_stack, scene->w.stack, 1, 1, 1);
    if (rc) return rc;
    hipStream_t st = stream;
    // the default traces each pixel's primary ray once (every sample of a pixel
@@ -514,12 +542,12 @@ int RenderEngine::run_plain(const ptx_scene *scene, const ptx_job_desc &desc, fl
    J.film = film;
    J.primary = primary;
    launch_zero_floats(film, (size_t)npix * 3, st);
-   if (cached)
-      launch_primary(scene->d, J, words + kWork, spill, leaf_lanes_of(tun, true),
-                     std::min<uint32_t>(ext_grid, (npix + 255) / 256), st);
-   const uint32_t grid =
-         std::min<uint32_t>((desc.flags & PTX_JOB_NEE) ? mega_nee_grid : mega_grid, (npix + 255) / 256);
-   for (uint32_t s = 0; s < desc.spp; s++) launch_mega(scene->d, J, s, spill, scene->has_texture, cached, grid, st);
+   if (cached) trace_primary_of(J, scene, npix);
+   const bool wide = wide_scene(scene), nee = (desc.flags & PTX_JOB_NEE) != 0;
+   const uint32_t full = wide ? (nee ? mega_wide_nee_grid : mega_wide_grid) : (nee ? mega_nee_grid : mega_grid);
+   const uint32_t grid = std::min<uint32_t>(full, (npix + 255) / 256);
+   for (uint32_t s = 0; s < desc.spp; s++)
+      launch_mega(scene->d, wide ? &scene->w : nullptr, J, s, spill, scene->has_texture, cached, grid, st);
    launch_finalize(film, npix, desc.spp, st);
    rc = download_host(dev, st,
                       {Span{reinterpret_cast<char *>(film_host), reinterpret_cast<char *>(film),

@@ -47,15 +47,18 @@ struct RenderEngine {
    uint4 *spill = nullptr;
    float4 *nee_scratch = nullptr;           // per resident lane of the regeneration kernel, 48 bytes
    size_t spill_entries = 0;
-   uint32_t stack_cap = 0;
+   uint32_t stack_cap = 0;                  // binary stack levels the spill holds
+   uint32_t wide_cap = 0;                   // four-wide stack entries it holds
    JobDev *d_jobs = nullptr;
    uint32_t *d_offsets = nullptr;           // jobs_cap + 1 entries: first primary-ray id of each job
    uint32_t jobs_cap = 0;
    DevScene *d_scenes = nullptr;
+   WideScene *d_wides = nullptr;            // the scenes' four-wide forms, beside d_scenes
    uint32_t scenes_cap = 0;
    Chunk *d_chunks = nullptr;
    uint32_t chunks_cap = 0;
    uint32_t ext_grid = 0, shade_grid = 0, mega_grid = 0, mega_nee_grid = 0, paths_grid = 0, connect_grid = 0;
+   uint32_t primary_wide_grid = 0, mega_wide_grid = 0, mega_wide_nee_grid = 0;
    // Device buffers of finished jobs (films, primary records) kept for later
    // jobs on this engine's stream: freeing them costs about 0.2 ms of host
    // time each (7 ms per batch of the 16-job render workload).  At most
@@ -88,7 +91,13 @@ struct RenderEngine {
    // Whether a round of nchunks chunks over nscenes scenes runs as one
    // path-regeneration launch under the engine's tuning.
    bool regen_round(uint32_t nchunks, uint32_t nscenes) const;
-   int ensure(uint32_t paths, uint32_t max_stack, uint32_t njobs, uint32_t nscenes, uint32_t nchunks);
+   // wide_stack: stack entries of the call's four-wide forms (0 = none).
+   int ensure(uint32_t paths, uint32_t max_stack, uint32_t wide_stack, uint32_t njobs, uint32_t nscenes,
+              uint32_t nchunks);
+   // Whether a scene's traversals step over its four-wide form here: it has
+   // one, and its stack fits the spill.  (The wavefront kernels step over the binary
+   // records always.)
+   bool wide_scene(const ptx_scene *s) const { return s->w.faces && s->w.stack <= wide_cap; }
    // Wavefront queues and hit records for at least `need` slots, and the
    // per-bounce graphs.
    int ensure_queues(uint32_t need);
@@ -96,13 +105,16 @@ struct RenderEngine {
    // Allocates the job's film and primary records, zeroes the film and, with
    // trace_primary, traces the primary hits (a batch traces every job's in
    // one launch instead).  J.film / J.primary are set.
-   int start_job(JobDev &J, const DevScene &S, uint32_t npix, bool trace_primary = true);
+   int start_job(JobDev &J, const ptx_scene *scene, uint32_t npix, bool trace_primary = true);
+   // The job's primary records, traced on the engine's stream.
+   void trace_primary_of(const JobDev &J, const ptx_scene *scene, uint32_t npix);
    // One round over the chunks in d_round (a device copy of r); the job and
    // scene tables must hold the round's jobs, the scene table nscenes entries.
    // nee: some job of the round uses next-event estimation;
-   // glossy / textured: some scene of the round has glossy / textured meshes.
+   // glossy / textured: some scene of the round has glossy / textured meshes;
+   // wide: wide_scene() of every scene of the round.
    int round(const Chunk *d_round, const std::vector<Chunk> &r, uint32_t depth, uint32_t nscenes, bool nee,
-             bool glossy, bool textured);
+             bool glossy, bool textured, bool wide);
    // Queues the film's finalisation and, when film_host is not NULL (the
    // server's pinned films), its copy there.
    int finish_job(JobDev &J, uint32_t npix, uint32_t spp, float *film_host);

@@ -58,7 +58,8 @@ struct JobState {
    bool retired = false;         // left the server: no device work or memory of it remains
    hipEvent_t done_ev = nullptr;
    JobDev jd{};
-   DevScene sd{};                // staged copy for the device scene table
+   DevScene sd{};                // staged copies for the device scene tables
+   WideScene wd{};
    float *film = nullptr;        // pinned host copy of the film (from the server's pool)
    size_t film_bytes = 0;
 };
@@ -293,12 +294,15 @@ void ptx_server::loop() {
       // the rounds already enqueued, which never read these table entries)
       for (auto &j : admitted) {
          j->jd = job_dev(j->desc, j->scene_slot);
-         int rc = eng.start_job(j->jd, j->scene->d, j->npix);
+         int rc = eng.start_job(j->jd, j->scene, j->npix);
          if (rc == PTX_OK) {
             j->started = true;
             j->sd = j->scene->d;
+            j->wd = j->scene->w;
             if (hipMemcpyAsync(eng.d_scenes + j->scene_slot, &j->sd, sizeof(DevScene), hipMemcpyHostToDevice, stream) !=
                       hipSuccess ||
+                hipMemcpyAsync(eng.d_wides + j->scene_slot, &j->wd, sizeof(WideScene), hipMemcpyHostToDevice,
+                               stream) != hipSuccess ||
                 hipMemcpyAsync(eng.d_jobs + j->slot, &j->jd, sizeof(JobDev), hipMemcpyHostToDevice, stream) !=
                       hipSuccess) {
                (void)hipGetLastError();
@@ -329,7 +333,7 @@ void ptx_server::loop() {
          chunks.clear();
          uint64_t used = 0;
          uint32_t depth = 0;
-         bool nee = false, glossy = false, textured = false;
+         bool nee = false, glossy = false, textured = false, wide = true;
          const uint64_t share = paths / cand.size();
          for (auto &j : cand) {
             const uint32_t left = j->desc.spp - j->next_sample;
@@ -344,6 +348,7 @@ void ptx_server::loop() {
             nee |= (j->desc.flags & PTX_JOB_NEE) != 0;
             glossy |= j->scene->has_glossy;
             textured |= j->scene->has_texture;
+            wide = wide && eng.wide_scene(j->scene);
          }
          // the table this round fills was last read by a round that has completed
          std::copy(chunks.begin(), chunks.end(), chunk_host[table]);
@@ -354,7 +359,7 @@ void ptx_server::loop() {
             (void)hipGetLastError();
             r.rc = set_error(PTX_ERR_HIP, std::string("server: chunk table upload: ") + hipGetErrorString(e));
          } else {
-            r.rc = eng.round(d_table, chunks, depth, kMaxServerScenes, nee, glossy, textured);
+            r.rc = eng.round(d_table, chunks, depth, kMaxServerScenes, nee, glossy, textured, wide);
          }
          rounds++;
          r.ev = take_event();
@@ -456,7 +461,7 @@ int ptx_server_create(ptx_device *dev, const ptx_server_config *cfg, ptx_server 
                                   : (s->eng.tun.paths_per_wave ? s->eng.tun.paths_per_wave
                                      : queues ? RenderEngine::kDefaultPaths : regen_paths);
    // the path pool is sized for scenes up to 64 levels deep; deeper scenes grow the spill
-   int rc = s->eng.ensure(s->paths, 64, kMaxServerJobs, kMaxServerScenes, 4 * kMaxServerJobs);
+   int rc = s->eng.ensure(s->paths, 64, 0, kMaxServerJobs, kMaxServerScenes, 4 * kMaxServerJobs);
    if (rc == PTX_OK && queues) rc = s->eng.ensure_queues(s->paths);
    if (rc) {
       s->eng.release();

@@ -266,7 +266,7 @@ __device__ __forceinline__ bool advance(Trav &s, const Fetched &f, const Stack<k
    return interior_step(s, f.q, st) != kStepDone;
 }
 
-constexpr uint32_t kBatch = 64;        // ids handed to a wave at a time
+constexpr uint32_t kBatch = 64;        // ids handed to a wave at a time, at most
 constexpr uint32_t kWorkWords = 8;     // u32 words of work counters a launch clears
 
 // Per-wave source of work ids, in batches of 64 consecutive ids.  The first
