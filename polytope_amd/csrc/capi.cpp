@@ -174,10 +174,12 @@ int run_closest_hit(ptx_scene *s, const float *d_rays, uint32_t n, ptx_hit *d_hi
    ptx_device *dev = s->dev;
    const uint32_t lds = lds_depth_of(t);
    if (wide_query(s, t, d_counters)) {
-      const uint32_t grid = std::max(1u, std::min(wide_query_grid(dev, t, lds, d_frames != nullptr), (n + 255) / 256));
+      Deal deal;
+      const uint32_t grid =
+            deal_ids(wide_query_grid(dev, t, lds, d_frames != nullptr), (uint32_t)dev->num_cus, n, deal);
       void *scratch = nullptr;
       PTX_HIP_TRY(pool_malloc(dev, &scratch, 256 + wide_spill_bytes(s, grid, lds), stream));
-      const int rc = launch_closest_hit_wide(s->d, s->w, d_rays, n, d_hits, d_frames, static_cast<uint32_t *>(scratch),
+      const int rc = launch_closest_hit_wide(s->d, s->w, d_rays, deal, d_hits, d_frames, static_cast<uint32_t *>(scratch),
                                              static_cast<char *>(scratch) + 256, grid, lds, wide_refill_lanes_of(t),
                                              wide_leaf_lanes_of(t), stream);
       const hipError_t fe = hipFreeAsync(scratch, stream);
@@ -547,9 +549,10 @@ int ptx_intersect_closest_device_noalloc(ptx_scene *scene, const float *d_rays, 
       uint32_t wgrid = wide_query_grid(dev, t, lds, d_frames != nullptr);
       const size_t block = wide_spill_bytes(scene, 1, lds);
       if (block) wgrid = (uint32_t)std::min<size_t>(wgrid, (kNoAllocScratchBytes - 256) / block);
-      wgrid = std::min(wgrid, std::max(1u, (n + 255) / 256));
+      Deal deal{};
+      if (wgrid) wgrid = deal_ids(wgrid, (uint32_t)dev->num_cus, n, deal);
       if (wgrid >= std::min(grid, (uint32_t)dev->num_cus)) {
-         if (launch_closest_hit_wide(scene->d, scene->w, d_rays, n, d_hits, d_frames, work, spill, wgrid, lds,
+         if (launch_closest_hit_wide(scene->d, scene->w, d_rays, deal, d_hits, d_frames, work, spill, wgrid, lds,
                                      wide_refill_lanes_of(t), wide_leaf_lanes_of(t),
                                      static_cast<hipStream_t>(stream)) != 0) {
             (void)hipGetLastError();

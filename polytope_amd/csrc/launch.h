@@ -4,9 +4,35 @@
 #include <hip/hip_runtime_api.h>
 #include <hip/hip_vector_types.h>
 
+#include <algorithm>
+
 #include "ptx_internal.h"
 
 namespace ptx {
+// Blocks per CU that a launch of few ids is spread over (deal_ids): 1 / 2 / 4
+// took 119 / 107 / 115 us for 50,021 rays on 81,920 faces, 342 / 300 / 330 us
+// for a 64x48 thumbnail of 4 samples (82 to 130 and 407 us packed).
+constexpr uint32_t kSpreadBlocks = 2;
+constexpr uint32_t kDealBatch = 64;
+}  // namespace ptx
+
+namespace ptx {
+
+// Grid and batches of a persistent four-wide launch over n ids: `full` blocks
+// (what fits the device) and batches of 64, three quarters of them dealt out
+// statically, when the ids fill it; else every wave gets one batch of its
+// share, from as many blocks as hold the ids at one a lane, or as two waves
+// per SIMD while that leaves a wave at least one id.  A wave of few rays runs
+// fewer phases for lanes other than its own.
+inline uint32_t deal_ids(uint32_t full, uint32_t num_cus, uint64_t n, Deal &d) {
+   const uint64_t packed = (n + 255) / 256, spread = std::min<uint64_t>((n + 3) / 4, kSpreadBlocks * (uint64_t)num_cus);
+   const uint32_t grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(full, std::max(packed, spread)));
+   d.n = (uint32_t)n;
+   d.batch = (uint32_t)std::min<uint64_t>(kDealBatch, std::max<uint64_t>(1, (n + 4ull * grid - 1) / (4ull * grid)));
+   d.batches = (uint32_t)((n + d.batch - 1) / d.batch);
+   d.static_batches = d.batches <= 4 * grid ? d.batches : d.batches - d.batches / 4;
+   return grid;
+}
 
 // windows: the scene's window records (launch_build_windows), or null to step
 // over sc.nodes; root_axis: the root's split axis (used with windows).
@@ -16,7 +42,7 @@ int launch_closest_hit(const DevScene &sc, const float *d_rays, uint32_t n, ptx_
                        const Node64 *windows, uint32_t root_axis, hipStream_t stream);
 // The same over the scene's four-wide form w (w.faces non-null), hits and
 // frames; d_spill: (w.stack - lds_depth) 8-byte entries per resident lane.
-int launch_closest_hit_wide(const DevScene &sc, const WideScene &w, const float *d_rays, uint32_t n, ptx_hit *d_hits,
+int launch_closest_hit_wide(const DevScene &sc, const WideScene &w, const float *d_rays, const Deal &deal, ptx_hit *d_hits,
                             ptx_hit_frame *d_frames, uint32_t *d_work, void *d_spill, uint32_t grid,
                             uint32_t lds_depth, uint32_t refill_min, uint32_t leaf_min, hipStream_t stream);
 int closest_hit_wide_blocks_per_cu(uint32_t lds_depth, bool frames);
@@ -49,13 +75,14 @@ int render_blocks_per_cu(int which);
 // W / wides: the scenes' four-wide forms, which the kernel then steps over
 // (every scene of the launch has one whose stack fits the spill); null = the
 // binary records.
-void launch_primary(const DevScene &S, const WideScene *W, const JobDev &J, uint32_t *work, uint4 *spill,
-                    uint32_t leaf_min, uint32_t grid, hipStream_t st);
+// deal: of the four-wide kernels (deal_ids).
+void launch_primary(const DevScene &S, const WideScene *W, const JobDev &J, const Deal &deal, uint32_t *work,
+                    uint4 *spill, uint32_t leaf_min, uint32_t grid, hipStream_t st);
 // Primary records of every job of a batch in one launch: jobs / scenes are the
 // device tables, offsets (njobs + 1 entries, device) the first pixel id of
 // each job and the total; max_stack bounds every scene's deferred stack.
 void launch_primaries(const JobDev *jobs, const DevScene *scenes, const WideScene *wides, const uint32_t *offsets,
-                      uint32_t njobs, uint32_t *work, uint4 *spill, uint32_t leaf_min, uint32_t max_stack, uint32_t grid,
+                      uint32_t njobs, const Deal &deal, uint32_t *work, uint4 *spill, uint32_t leaf_min, uint32_t max_stack, uint32_t grid,
                       hipStream_t st);
 // Shadow connection of the wavefront form (rounds with next-event jobs):
 // the vertex queue (48 B per entry, one entry per path slot at most), its
@@ -88,7 +115,7 @@ int paths_blocks_per_cu();
 uint32_t paths_max_chunks();
 uint32_t paths_max_scenes();
 void launch_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jobs, const DevScene *scenes,
-                  const WideScene *wides, uint32_t nscenes, float *res, uint32_t *work, uint4 *spill,
+                  const WideScene *wides, uint32_t nscenes, float *res, const Deal &deal, uint32_t *work, uint4 *spill,
                   uint32_t max_stack, uint32_t shade_min, uint32_t leaf_min, float4 *nee_scratch, bool glossy,
                   bool textured, uint32_t grid, hipStream_t st);
 // textured: the scene has textured meshes; cached: start every path from the

@@ -145,6 +145,13 @@ struct Chunk {
    uint32_t job, s0, k, npix, base;
 };
 
+// How a persistent launch's ids are dealt out: `batches` batches of `batch`
+// consecutive ids, the first static_batches of them round robin to the waves,
+// the rest by a counter.
+struct Deal {
+   uint32_t n, batch, batches, static_batches;
+};
+
 // Largest number of chunks in a round of the path-regeneration kernel (its
 // chunk table lives in LDS).
 constexpr uint32_t kMaxRoundChunks = 64;

@@ -566,17 +566,17 @@ struct WidePrimaries {
 
 template <int kLds>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
-k_primary_wide(DevScene S, WideScene W, JobDev J, uint32_t *work, uint2 *spill, uint32_t leaf_min) {
+k_primary_wide(DevScene S, WideScene W, JobDev J, Deal deal, uint32_t *work, uint2 *spill, uint32_t leaf_min) {
    const WidePrimary P{S, W, J};
-   wide_trace<kLds>(P, J.width * J.height, work, spill, kWideRefill, leaf_min, W.stack);
+   wide_trace<kLds>(P, deal, work, spill, kWideRefill, leaf_min, W.stack);
 }
 
 template <int kLds>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
 k_primaries_wide(const JobDev *jobs, const DevScene *scenes, const WideScene *wides, const uint32_t *offsets,
-                 uint32_t njobs, uint32_t *work, uint2 *spill, uint32_t leaf_min, uint32_t max_stack) {
+                 uint32_t njobs, Deal deal, uint32_t *work, uint2 *spill, uint32_t leaf_min, uint32_t max_stack) {
    const WidePrimaries P{jobs, scenes, wides, offsets, njobs};
-   wide_trace<kLds>(P, offsets[njobs], work, spill, kWideRefill, leaf_min, max_stack);
+   wide_trace<kLds>(P, deal, work, spill, kWideRefill, leaf_min, max_stack);
 }
 
 template <int kLds>
@@ -1204,8 +1204,8 @@ struct NeeRecord {
 template <int kLds, bool kNee, bool kGlossy, bool kTex, bool kWide>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
 k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jobs, const DevScene *scenes,
-        const WideScene *wides, uint32_t nscenes, float *res, uint32_t *work, uint4 *spill, uint32_t max_stack,
-        uint32_t shade_min, uint32_t leaf_min, float4 *nee_scratch) {
+        const WideScene *wides, uint32_t nscenes, float *res, Deal deal, uint32_t *work, uint4 *spill,
+        uint32_t max_stack, uint32_t shade_min, uint32_t leaf_min, float4 *nee_scratch) {
    __shared__ uint32_t lds[TraceStack<kLds, kWide>::kWords];
    __shared__ LdsChunk sch[kMaxRoundChunks];
    __shared__ DevScene ssc[kMaxRoundScenes];
@@ -1229,7 +1229,8 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
    const auto st = TraceStack<kLds, kWide>::make(lds, spill, max_stack);
    if constexpr (kWide) st.sentinel();
    RaySource srcq;
-   srcq.init(nslots, work, lane);
+   if constexpr (kWide) srcq.init(deal, work, lane);
+   else srcq.init(nslots, work, lane);
    Trav s;
    s.hit = kNone;
    s.after = 0;
@@ -1670,23 +1671,23 @@ int render_blocks_per_cu(int which) {
    return e == hipSuccess && b > 0 ? b : 1;
 }
 
-void launch_primary(const DevScene &S, const WideScene *W, const JobDev &J, uint32_t *work, uint4 *spill,
-                    uint32_t leaf_min, uint32_t grid, hipStream_t st) {
+void launch_primary(const DevScene &S, const WideScene *W, const JobDev &J, const Deal &deal, uint32_t *work,
+                    uint4 *spill, uint32_t leaf_min, uint32_t grid, hipStream_t st) {
    hipLaunchKernelGGL(dev::k_zero_words, dim3(1), dim3(64), 0, st, work, 8u, (uint32_t *)nullptr, 0u);
    if (W)
-      hipLaunchKernelGGL(dev::k_primary_wide<kRenderLds>, dim3(grid), dim3(256), 0, st, S, *W, J, work,
+      hipLaunchKernelGGL(dev::k_primary_wide<kRenderLds>, dim3(grid), dim3(256), 0, st, S, *W, J, deal, work,
                          reinterpret_cast<uint2 *>(spill), leaf_min);
    else
       hipLaunchKernelGGL(dev::k_primary<kRenderLds>, dim3(grid), dim3(256), 0, st, S, J, work, spill, leaf_min);
 }
 
 void launch_primaries(const JobDev *jobs, const DevScene *scenes, const WideScene *wides, const uint32_t *offsets,
-                      uint32_t njobs, uint32_t *work, uint4 *spill, uint32_t leaf_min, uint32_t max_stack,
+                      uint32_t njobs, const Deal &deal, uint32_t *work, uint4 *spill, uint32_t leaf_min, uint32_t max_stack,
                       uint32_t grid, hipStream_t st) {
    hipLaunchKernelGGL(dev::k_zero_words, dim3(1), dim3(64), 0, st, work, 8u, (uint32_t *)nullptr, 0u);
    if (wides)
       hipLaunchKernelGGL(dev::k_primaries_wide<kRenderLds>, dim3(grid), dim3(256), 0, st, jobs, scenes, wides, offsets,
-                         njobs, work, reinterpret_cast<uint2 *>(spill), leaf_min, max_stack);
+                         njobs, deal, work, reinterpret_cast<uint2 *>(spill), leaf_min, max_stack);
    else
       hipLaunchKernelGGL(dev::k_primaries<kRenderLds>, dim3(grid), dim3(256), 0, st, jobs, scenes, offsets, njobs,
                          work, spill, leaf_min, max_stack);
@@ -1764,12 +1765,12 @@ uint32_t paths_max_scenes() { return dev::kMaxRoundScenes; }
 namespace {
 template <bool W>
 void launch_paths_t(int variant, const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jobs,
-                    const DevScene *scenes, const WideScene *wides, uint32_t nscenes, float *res, uint32_t *work,
-                    uint4 *spill, uint32_t max_stack, uint32_t shade_min, uint32_t leaf_min, float4 *nee_scratch,
+                    const DevScene *scenes, const WideScene *wides, uint32_t nscenes, float *res, const Deal &deal,
+                    uint32_t *work, uint4 *spill, uint32_t max_stack, uint32_t shade_min, uint32_t leaf_min, float4 *nee_scratch,
                     uint32_t grid, hipStream_t st) {
 #define PTX_LAUNCH_PATHS(N, G, T)                                                                                  \
    hipLaunchKernelGGL((dev::k_paths<kRenderLds, N, G, T, W>), dim3(grid), dim3(256), 0, st, chunks, nchunks, nslots, \
-                      jobs, scenes, wides, nscenes, res, work, spill, max_stack, shade_min, leaf_min, nee_scratch)
+                      jobs, scenes, wides, nscenes, res, deal, work, spill, max_stack, shade_min, leaf_min, nee_scratch)
    switch (variant) {
       case 0: PTX_LAUNCH_PATHS(false, false, false); break;
       case 1: PTX_LAUNCH_PATHS(true, false, false); break;
@@ -1785,16 +1786,16 @@ void launch_paths_t(int variant, const Chunk *chunks, uint32_t nchunks, uint32_t
 }  // namespace
 
 void launch_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jobs, const DevScene *scenes,
-                  const WideScene *wides, uint32_t nscenes, float *res, uint32_t *work, uint4 *spill,
+                  const WideScene *wides, uint32_t nscenes, float *res, const Deal &deal, uint32_t *work, uint4 *spill,
                   uint32_t max_stack, uint32_t shade_min, uint32_t leaf_min, float4 *nee_scratch, bool glossy,
                   bool textured, uint32_t grid, hipStream_t st) {
    hipLaunchKernelGGL(dev::k_zero_words, dim3(1), dim3(64), 0, st, work, 8u, (uint32_t *)nullptr, 0u);
    const int v = (nee_scratch ? 1 : 0) | (glossy ? 2 : 0) | (textured ? 4 : 0);
    if (wides)
-      launch_paths_t<true>(v, chunks, nchunks, nslots, jobs, scenes, wides, nscenes, res, work, spill, max_stack,
+      launch_paths_t<true>(v, chunks, nchunks, nslots, jobs, scenes, wides, nscenes, res, deal, work, spill, max_stack,
                            shade_min, leaf_min, nee_scratch, grid, st);
    else
-      launch_paths_t<false>(v, chunks, nchunks, nslots, jobs, scenes, wides, nscenes, res, work, spill, max_stack,
+      launch_paths_t<false>(v, chunks, nchunks, nslots, jobs, scenes, wides, nscenes, res, deal, work, spill, max_stack,
                             shade_min, leaf_min, nee_scratch, grid, st);
 }
 

@@ -334,8 +334,11 @@ std::vector<std::vector<Chunk>> schedule_rounds(const std::vector<RenderJob> &jo
 
 void RenderEngine::trace_primary_of(const JobDev &J, const ptx_scene *scene, uint32_t npix) {
    const bool wide = wide_scene(scene);
-   launch_primary(scene->d, wide ? &scene->w : nullptr, J, words + kWork, spill, leaf_lanes_of(tun, true),
-                  std::min<uint32_t>(wide ? primary_wide_grid : ext_grid, (npix + 255) / 256), stream);
+   Deal deal{};
+   const uint32_t grid = wide ? deal_ids(primary_wide_grid, (uint32_t)dev->num_cus, npix, deal)
+                              : std::min<uint32_t>(ext_grid, (npix + 255) / 256);
+   launch_primary(scene->d, wide ? &scene->w : nullptr, J, deal, words + kWork, spill, leaf_lanes_of(tun, true), grid,
+                  stream);
 }
 
 int RenderEngine::start_job(JobDev &J, const ptx_scene *scene, uint32_t npix, bool trace_primary) {
@@ -365,9 +368,12 @@ int RenderEngine::round(const Chunk *d_round, const std::vector<Chunk> &r, uint3
    }
    if (regen_round((uint32_t)r.size(), nscenes)) {
       const uint32_t shade_min = tun.shade_lanes ? tun.shade_lanes : kDefaultShadeLanes;
-      launch_paths(d_round, (uint32_t)r.size(), nslots, d_jobs, d_scenes, wide ? d_wides : nullptr, nscenes, res,
-                   words + kWork, spill, wide ? wide_cap : stack_cap, shade_min, leaf_lanes_of(tun, true), nee ? nee_scratch : nullptr, glossy, textured,
-                   std::min<uint32_t>(paths_grid, (nslots + 255) / 256), stream);
+      Deal deal{};
+      const uint32_t grid = wide ? deal_ids(paths_grid, (uint32_t)dev->num_cus, nslots, deal)
+                                 : std::min<uint32_t>(paths_grid, (nslots + 255) / 256);
+      launch_paths(d_round, (uint32_t)r.size(), nslots, d_jobs, d_scenes, wide ? d_wides : nullptr, nscenes, res, deal,
+                   words + kWork, spill, wide ? wide_cap : stack_cap, shade_min, leaf_lanes_of(tun, true), nee ? nee_scratch : nullptr, glossy, textured, grid,
+                   stream);
       launch_accumulate(d_round, (uint32_t)r.size(), d_jobs, res, nullptr, shade_grid, stream);
       return PTX_OK;
    }
@@ -482,11 +488,13 @@ int RenderEngine::run_batch(const std::vector<RenderJob> &jobs, const std::vecto
          return set_error(PTX_ERR_HIP, std::string("render batch tables: ") + hipGetErrorString(e));
       }
    }
-   if (one_launch)
-      launch_primaries(d_jobs, d_scenes, wide ? d_wides : nullptr, d_offsets, nj, words + kWork, spill,
-                       leaf_lanes_of(tun, true), wide ? wide_cap : max_stack,
-                       (uint32_t)std::min<uint64_t>(wide ? primary_wide_grid : ext_grid, (total_pixels + 255) / 256),
-                       st);
+   if (one_launch) {
+      Deal deal{};
+      const uint32_t grid = wide ? deal_ids(primary_wide_grid, (uint32_t)dev->num_cus, total_pixels, deal)
+                                 : (uint32_t)std::min<uint64_t>(ext_grid, (total_pixels + 255) / 256);
+      launch_primaries(d_jobs, d_scenes, wide ? d_wides : nullptr, d_offsets, nj, deal, words + kWork, spill,
+                       leaf_lanes_of(tun, true), wide ? wide_cap : max_stack, grid, st);
+   }
    size_t off = 0;
    for (const auto &r : rounds) {
       uint32_t depth = 0;

@@ -147,10 +147,10 @@ struct WideQuery {
 
 template <int kLds, bool kFrames>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8)))
-k_closest_hit_wide(DevScene sc, WideScene w, const float *__restrict__ rays, uint32_t n, ptx_hit *__restrict__ hits,
+k_closest_hit_wide(DevScene sc, WideScene w, const float *__restrict__ rays, Deal deal, ptx_hit *__restrict__ hits,
                    ptx_hit_frame *frames, uint32_t *work, uint2 *spill, uint32_t refill_min, uint32_t leaf_min) {
    const WideQuery<kFrames> q{sc, w, rays, hits, frames};
-   wide_trace<kLds>(q, n, work, spill, refill_min, leaf_min, w.stack);
+   wide_trace<kLds>(q, deal, work, spill, refill_min, leaf_min, w.stack);
 }
 
 // One thread per window: window w of interior node i is win[4 i + 2 w] (the
@@ -269,14 +269,14 @@ int blocks_lds(bool extra, bool windows) {
 namespace {
 
 template <int kLds>
-void launch_wide(const DevScene &sc, const WideScene &w, const float *d_rays, uint32_t n, ptx_hit *d_hits, ptx_hit_frame *d_frames,
+void launch_wide(const DevScene &sc, const WideScene &w, const float *d_rays, const Deal &deal, ptx_hit *d_hits, ptx_hit_frame *d_frames,
                  uint32_t *d_work, uint2 *d_spill, uint32_t grid, uint32_t refill_min, uint32_t leaf_min,
                  hipStream_t stream) {
    if (d_frames)
-      hipLaunchKernelGGL((dev::k_closest_hit_wide<kLds, true>), dim3(grid), dim3(256), 0, stream, sc, w, d_rays, n, d_hits,
+      hipLaunchKernelGGL((dev::k_closest_hit_wide<kLds, true>), dim3(grid), dim3(256), 0, stream, sc, w, d_rays, deal, d_hits,
                          d_frames, d_work, d_spill, refill_min, leaf_min);
    else
-      hipLaunchKernelGGL((dev::k_closest_hit_wide<kLds, false>), dim3(grid), dim3(256), 0, stream, sc, w, d_rays, n,
+      hipLaunchKernelGGL((dev::k_closest_hit_wide<kLds, false>), dim3(grid), dim3(256), 0, stream, sc, w, d_rays, deal,
                          d_hits, d_frames, d_work, d_spill, refill_min, leaf_min);
 }
 
@@ -291,17 +291,17 @@ int blocks_wide(bool frames) {
 
 }  // namespace
 
-int launch_closest_hit_wide(const DevScene &sc, const WideScene &w, const float *d_rays, uint32_t n, ptx_hit *d_hits,
+int launch_closest_hit_wide(const DevScene &sc, const WideScene &w, const float *d_rays, const Deal &deal, ptx_hit *d_hits,
                             ptx_hit_frame *d_frames, uint32_t *d_work, void *d_spill, uint32_t grid,
                             uint32_t lds_depth, uint32_t refill_min, uint32_t leaf_min, hipStream_t stream) {
    hipLaunchKernelGGL(dev::k_zero_u32, dim3(1), dim3(64), 0, stream, d_work, (uint32_t)dev::kWorkWords);
-   if (n == 0) return 0;
+   if (deal.n == 0) return 0;
    uint2 *spill = static_cast<uint2 *>(d_spill);
    switch (lds_depth) {
-      case 8: launch_wide<8>(sc, w, d_rays, n, d_hits, d_frames, d_work, spill, grid, refill_min, leaf_min, stream); break;
-      case 16: launch_wide<16>(sc, w, d_rays, n, d_hits, d_frames, d_work, spill, grid, refill_min, leaf_min, stream); break;
-      case 24: launch_wide<24>(sc, w, d_rays, n, d_hits, d_frames, d_work, spill, grid, refill_min, leaf_min, stream); break;
-      default: launch_wide<12>(sc, w, d_rays, n, d_hits, d_frames, d_work, spill, grid, refill_min, leaf_min, stream); break;
+      case 8: launch_wide<8>(sc, w, d_rays, deal, d_hits, d_frames, d_work, spill, grid, refill_min, leaf_min, stream); break;
+      case 16: launch_wide<16>(sc, w, d_rays, deal, d_hits, d_frames, d_work, spill, grid, refill_min, leaf_min, stream); break;
+      case 24: launch_wide<24>(sc, w, d_rays, deal, d_hits, d_frames, d_work, spill, grid, refill_min, leaf_min, stream); break;
+      default: launch_wide<12>(sc, w, d_rays, deal, d_hits, d_frames, d_work, spill, grid, refill_min, leaf_min, stream); break;
    }
    return hipGetLastError() == hipSuccess ? 0 : -1;
 }

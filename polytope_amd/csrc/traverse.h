@@ -266,7 +266,7 @@ __device__ __forceinline__ bool advance(Trav &s, const Fetched &f, const Stack<k
    return interior_step(s, f.q, st) != kStepDone;
 }
 
-constexpr uint32_t kBatch = 64;        // ids handed to a wave at a time, at most
+constexpr uint32_t kBatch = 64;        // ids handed to a wave at a time, at most (kDealBatch)
 constexpr uint32_t kWorkWords = 8;     // u32 words of work counters a launch clears
 
 // Per-wave source of work ids, in batches of 64 consecutive ids.  The first
@@ -280,45 +280,48 @@ constexpr uint32_t kWorkWords = 8;     // u32 words of work counters a launch cl
 // traversal steps.  When the counter passes the end, the wave is done: no
 // wave ever waits on more than one atomic at the end of a launch.
 struct RaySource {
-   uint32_t n;                    // ids
-   uint32_t batches, static_batches;
+   Deal d;
    uint32_t waves;                // waves in the grid
    uint32_t next;                 // this wave's next static batch
    uint32_t pool_base, pool_left;
    uint32_t prefetch;             // pending dynamic request's result (lane 0)
    bool done;
    __device__ __forceinline__ void init(uint32_t n_ids, uint32_t *work, uint32_t lane) {
-      n = n_ids;
-      batches = (n + kBatch - 1) / kBatch;
-      static_batches = batches - batches / 4;
+      const uint32_t batches = (n_ids + kBatch - 1) / kBatch;
+      init(Deal{n_ids, kBatch, batches, batches - batches / 4}, work, lane);
+   }
+   __device__ __forceinline__ void init(const Deal &deal, uint32_t *work, uint32_t lane) {
+      d = deal;
       waves = gridDim.x * (blockDim.x / 64u);
       next = (blockIdx.x * blockDim.x + threadIdx.x) / 64u;
       pool_base = pool_left = 0;
       prefetch = 0;
-      done = n == 0;
-      if (!done && next >= static_batches) request(work, lane);
+      done = d.n == 0;
+      if (!done && next >= d.static_batches) request(work, lane);
    }
+   // With every batch dealt out statically the counter has nothing to give, and
+   // the small launches that deal so would wait on it for 7 to 20 us.
    __device__ __forceinline__ void request(uint32_t *work, uint32_t lane) {
-      if (lane == 0) prefetch = atomicAdd(&work[0], 1u);
+      if (lane == 0 && d.static_batches != d.batches) prefetch = atomicAdd(&work[0], 1u);
    }
    // Makes pool_left > 0 unless every batch is taken (then done = true).
    __device__ __forceinline__ void refill(uint32_t *work, uint32_t lane) {
       if (pool_left != 0 || done) return;
       uint32_t b;
-      if (next < static_batches) {
+      if (next < d.static_batches) {
          b = next;
          next += waves;
-         if (next >= static_batches) request(work, lane);     // the first dynamic batch, ahead of time
+         if (next >= d.static_batches) request(work, lane);     // the first dynamic batch, ahead of time
       } else {
-         b = static_batches + __builtin_amdgcn_readlane(prefetch, 0);
-         if (b >= batches) {
+         b = d.static_batches + __builtin_amdgcn_readlane(prefetch, 0);
+         if (b >= d.batches) {
             done = true;
             return;
          }
          request(work, lane);
       }
-      pool_base = b * kBatch;
-      pool_left = min(kBatch, n - pool_base);
+      pool_base = b * d.batch;
+      pool_left = min(d.batch, d.n - pool_base);
    }
 };
 

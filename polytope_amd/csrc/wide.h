@@ -478,14 +478,14 @@ __device__ __forceinline__ bool wide_leaf_or_exact(Trav &s, const WideFace *face
 // loads a step: 1,772 against 1,600 us on 2^23 incoherent rays.  Five waves per
 // SIMD spill 24 registers: 1,881 us.
 template <int kLds, class Policy>
-__device__ __forceinline__ void wide_trace(const Policy &P, uint32_t n, uint32_t *work, uint2 *spill,
+__device__ __forceinline__ void wide_trace(const Policy &P, const Deal &deal, uint32_t *work, uint2 *spill,
                                            uint32_t refill_min, uint32_t leaf_min, uint32_t max_stack) {
    __shared__ uint32_t lds[2 * kLds * 256];
    const uint32_t lane = __lane_id();
    const WideStack<kLds> st{lds, reinterpret_cast<u32x2 *>(spill), threadIdx.x,
                             blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, max_stack};
    RaySource src;
-   src.init(n, work, lane);
+   src.init(deal, work, lane);
    constexpr uint32_t kNone = 0xFFFFFFFFu;
    st.sentinel();
    Trav s;
