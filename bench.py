@@ -219,8 +219,8 @@ def render_section(dev, args):
     dev.set_tuning()
     print(f"[bench] batched wavefront: {samples / t_wave / 1e6:.1f} Msamples/s", file=sys.stderr, flush=True)
     # plain: one job per call, one launch per sample; each pixel's primary ray
-    # traced once (the default), and again for every sample (the reference
-    # CUDA path's shape)
+    # traced once, and again for every sample (the reference CUDA path's shape)
+    dev.set_tuning(plain_primary=_abi.PLAIN_CACHED)
     tp = time.perf_counter()
     films_p = [render(scene, c, spp, d, seed) for c, spp, d, seed in jobs]
     t_plain = time.perf_counter() - tp
@@ -246,9 +246,11 @@ def render_section(dev, args):
     tm = time.perf_counter()
     films_m = render_batch(mat_batch)
     t_mat = time.perf_counter() - tm
+    dev.set_tuning(plain_primary=_abi.PLAIN_CACHED)
     tmp = time.perf_counter()
     films_mp = [render(mat_scene, c, spp, d, seed) for c, spp, d, seed in jobs]
     t_mat_plain = time.perf_counter() - tmp
+    dev.set_tuning()
     same_m = all(np.array_equal(a.view(np.uint32), b.view(np.uint32)) for a, b in zip(films_m, films_mp))
     print(f"[bench] textured + glossy: batched {samples / t_mat / 1e6:.1f}, plain {samples / t_mat_plain / 1e6:.1f} "
           f"Msamples/s", file=sys.stderr, flush=True)
@@ -306,7 +308,7 @@ def plain_cpu_render_section(dev, args, threads: int):
     640x480, 16 spp, depth 5): the reference's own TileRunner on the host's cores
     beside the GPU's plain and batched paths on the same scene."""
     import oracle as O
-    from polytope_amd import Scene, render, render_batch
+    from polytope_amd import Scene, _abi, render, render_batch
     from polytope_amd import scenes as S
     meshes, cam, sky = S.plain_render_scene(1, 640, 480)
     spp, depth = 16, 5
@@ -314,10 +316,12 @@ def plain_cpu_render_section(dev, args, threads: int):
     out = {"workload": "ground quad + 3 lat-long spheres (4,802 faces), 640x480, 16 spp, depth 5",
            "samples": samples}
     scene = Scene(dev, meshes, sky)
+    dev.set_tuning(plain_primary=_abi.PLAIN_CACHED)
     render(scene, cam, 1, depth, 1)
     t = time.perf_counter()
     render(scene, cam, spp, depth, 1)
     out["gpu_plain_samples_per_s"] = round(samples / (time.perf_counter() - t), 1)
+    dev.set_tuning()
     render_batch([(scene, cam, 1, depth, 1)])
     t = time.perf_counter()
     render_batch([(scene, cam, spp, depth, 1)])
@@ -354,7 +358,7 @@ def serving_section(dev, args, n_requests: int, rate: float, burst: bool = False
     the continuous-batching server, and the same stream through the plain path:
     one job per render() call, in arrival order, as a caller without the server
     would serve it.  Latency = completion - arrival."""
-    from polytope_amd import Scene, Server, render
+    from polytope_amd import Scene, Server, _abi, render
     from polytope_amd import scenes as S
     scene_defs, reqs = S.serving_requests(n_requests, rate)
     if burst:
@@ -386,6 +390,7 @@ def serving_section(dev, args, n_requests: int, rate: float, burst: bool = False
         out["offered_samples_per_s"] = round(total / max(1e-9, reqs[-1][0]), 1)
     out.update(_latency_stats(lat, total, last - first))
     # the plain path over the same stream
+    dev.set_tuning(plain_primary=_abi.PLAIN_CACHED)
     lat_p = []
     t0 = time.perf_counter()
     for arr, si, cam, spp, depth, seed in reqs:
@@ -395,6 +400,7 @@ def serving_section(dev, args, n_requests: int, rate: float, burst: bool = False
         render(scenes_[si], cam, spp, depth, seed)
         lat_p.append(time.perf_counter() - (t0 + arr))
     span = time.perf_counter() - t0
+    dev.set_tuning()
     out["plain"] = _latency_stats(lat_p, total, span)
     out["server_vs_plain_throughput"] = round(out["throughput_samples_per_s"] / out["plain"]["throughput_samples_per_s"], 3)
     out["server_vs_plain_p50_latency"] = round(out["plain"]["latency_p50_s"] / out["latency_p50_s"], 3)

@@ -242,10 +242,12 @@ int ptx_intersect_closest_device_noalloc(ptx_scene *scene, const float *d_rays, 
                                          ptx_hit *d_hits, ptx_ray_counters *d_counters,
                                          ptx_hit_frame *d_frames, void *stream);
 
-/* Plain GPU render of one job: one launch per sample, each pixel's path in one
- * thread with every bounce inline (the launch shape of the reference's CUDA
- * path); each pixel's primary ray is traced once unless ptx_tuning.plain_primary
- * = RETRACE.  film_rgb = W*H*3 floats on the host (BoxFilter::Output values). */
+/* GPU render of one job.  By default it runs as ptx_render_batch with that one
+ * job (rounds of up to 2^26 path slots).  With one sample a pixel or two of at
+ * most one bounce, with ptx_tuning.plain_primary = CACHED or RETRACE, with render_mode = WAVEFRONT,
+ * or when the path slots find no memory: one launch per sample, each pixel's path in one thread with every
+ * bounce inline (the launch shape of the reference's CUDA path).  Same films.
+ * film_rgb = W*H*3 floats on the host (BoxFilter::Output values). */
 int ptx_render(ptx_scene *scene, const ptx_job_desc *job, float *film_rgb);
 /* Batched render: all jobs' samples are merged into rounds of path slots that
  * share the GPU.  A round is one persistent path-regeneration launch (every
@@ -292,10 +294,12 @@ typedef struct ptx_tuning {
    uint32_t leaf_lanes;      /* traversal: lanes of a wave that must reach a leaf     */
                              /* before the wave runs a leaf step (1..64; 0 = 1 for   */
                              /* ray queries, 16 for rendering)                       */
-   uint32_t plain_primary;   /* ptx_render, PTX_PLAIN_*: CACHED (default) traces each */
-                             /* pixel's primary ray once and starts every sample     */
-                             /* from it; RETRACE traces it again for every sample,   */
-                             /* as the reference's CUDA path does.  Same films.      */
+   uint32_t plain_primary;   /* ptx_render, PTX_PLAIN_*: DEFAULT renders the job as a */
+                             /* batch of one; CACHED and RETRACE take one launch per */
+                             /* sample, CACHED tracing each pixel's primary ray once */
+                             /* and starting every sample from it, RETRACE tracing   */
+                             /* it again for every sample, as the reference's CUDA   */
+                             /* path does.  Same films.                              */
    uint32_t ray_windows;     /* closest-hit queries, PTX_WINDOWS_*: OFF (default)     */
                              /* steps over one node record at a time; ON steps over  */
                              /* window records (a node's record and its first-       */

@@ -157,7 +157,8 @@ class Device:
         """render_mode: 0 auto, 1 path regeneration, 2 wavefront queues;
         shade_lanes: lanes a regeneration wave gathers before it shades;
         leaf_lanes: lanes a traversal wave gathers at leaves before a leaf step;
-        plain_primary: render(), 0/1 primary rays traced once per pixel, 2 traced again every sample;
+        plain_primary: render(), 0 a batch of one job, 1 one launch per sample with primary rays traced once
+        per pixel, 2 the same with them traced again every sample;
         ray_windows: closest-hit queries, 0/2 one node record per step, 1 window records (node + first-visited
         child in one 128-byte block) once the ray queue is drained; same results, slower on MI355X."""
         t = _abi.Tuning(paths_per_wave, block_size, lds_stack, refill_lanes, blocks_per_cu, render_mode, shade_lanes,
@@ -278,8 +279,9 @@ class Scene:
 
 
 def render(scene: Scene, cam: Camera, spp: int, max_depth: int, seed: int, nee: bool = False) -> np.ndarray:
-    """Plain GPU render of one job (ptx_render): one launch per sample, one thread
-    per pixel path.  Returns the (H, W, 3) BoxFilter film (0-255 units)."""
+    """GPU render of one job (ptx_render): a batch of one, or one launch per sample
+    and one thread per pixel path with ``plain_primary`` set.  Returns the (H, W,
+    3) BoxFilter film (0-255 units)."""
     film = np.zeros((cam.height, cam.width, 3), np.float32)
     job = job_desc(cam, spp, max_depth, seed, nee)
     check(load().ptx_render(scene.handle, C.byref(job), film.ctypes.data))

@@ -25,6 +25,7 @@ std::vector<std::vector<Chunk>> schedule_rounds(const std::vector<RenderJob> &jo
 struct RenderEngine {
    static constexpr uint32_t kDefaultPaths = 1u << 22;        // wavefront rounds (232 B per slot)
    static constexpr uint32_t kDefaultRegenPaths = 1u << 30;   // regeneration rounds (12 B per slot)
+   static constexpr uint32_t kDefaultPlainPaths = 1u << 26;   // the same for ptx_render's one job
    static constexpr uint32_t kDefaultShadeLanes = 16;   // lanes a wave gathers before it shades
    // layout of `words`: 8 traversal work words (word 0 counts the dynamic
    // batches handed out), the two queue counts, the bounce index, the
@@ -119,10 +120,13 @@ struct RenderEngine {
    // server's pinned films), its copy there.
    int finish_job(JobDev &J, uint32_t npix, uint32_t spp, float *film_host);
    void free_job(JobDev &J);
-   uint32_t capacity_for(uint64_t total_paths, uint32_t max_npix, bool regen) const;
+   uint32_t capacity_for(uint64_t total_paths, uint32_t max_npix, bool regen, uint32_t regen_paths) const;
+   // regen_paths: path slots of a regeneration round when the tuning names none.
    int run_batch(const std::vector<RenderJob> &jobs, const std::vector<const ptx_scene *> &scenes,
-                 const std::vector<float *> &films_host);
+                 const std::vector<float *> &films_host, uint32_t regen_paths = kDefaultRegenPaths);
+   // ptx_render: a batch of one job, or one launch per sample (run_launches).
    int run_plain(const ptx_scene *scene, const ptx_job_desc &desc, float *film_host);
+   int run_launches(const ptx_scene *scene, const ptx_job_desc &desc, float *film_host);
 };
 
 RenderEngine *engine_of(ptx_device *dev);

@@ -104,3 +104,32 @@ def test_wide_and_binary_queries_agree(name, n):
     finally:
         scene.close()
         dev.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", ["plain", "textured", "nee"])
+@pytest.mark.parametrize("size", [(1, 1, 1, 1), (37, 29, 5, 4), (131, 130, 2, 3)])
+def test_render_forms_agree(case, size):
+    """ptx_render as a batch of one and as one launch per sample, over one
+    pixel, a ragged film and one with the debug pixel: the same bits."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from polytope_amd import Device, Scene, _abi, render
+    w, h, spp, depth = size
+    lights = [((0.0, 5.0, -2.0), (4000.0, 4000.0, 4000.0))] if case == "nee" else None
+    if case == "textured":
+        meshes, cam, sky = S.textured_render_scene(1, w, h)
+    else:
+        meshes, cam, sky = S.plain_render_scene(1, w, h)
+    dev = Device(0)
+    scene = Scene(dev, meshes, sky, lights=lights)
+    try:
+        film = render(scene, cam, spp, depth, 3, nee=bool(lights))
+        for form in (_abi.PLAIN_CACHED, _abi.PLAIN_RETRACE):
+            dev.set_tuning(plain_primary=form)
+            assert np.array_equal(render(scene, cam, spp, depth, 3, nee=bool(lights)).view(np.uint32),
+                                  film.view(np.uint32))
+    finally:
+        scene.close()
+        dev.close()
