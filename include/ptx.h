@@ -244,9 +244,10 @@ int ptx_intersect_closest_device_noalloc(ptx_scene *scene, const float *d_rays, 
 
 /* GPU render of one job.  By default it runs as ptx_render_batch with that one
  * job (rounds of up to 2^26 path slots).  With one sample a pixel or two of at
- * most one bounce, with ptx_tuning.plain_primary = CACHED or RETRACE, with render_mode = WAVEFRONT,
- * or when the path slots find no memory: one launch per sample, each pixel's path in one thread with every
- * bounce inline (the launch shape of the reference's CUDA path).  Same films.
+ * most one bounce, with ptx_tuning.plain_primary = CACHED or RETRACE, with
+ * render_mode = WAVEFRONT, or when the path slots find no memory: one launch
+ * per sample, each pixel's path in one thread with every bounce inline (the
+ * launch shape of the reference's CUDA path).  Same films.
  * film_rgb = W*H*3 floats on the host (BoxFilter::Output values). */
 int ptx_render(ptx_scene *scene, const ptx_job_desc *job, float *film_rgb);
 /* Batched render: all jobs' samples are merged into rounds of path slots that
@@ -290,10 +291,12 @@ typedef struct ptx_tuning {
                              /* 64 scenes runs as consecutive groups of at most 64); */
                              /* WAVEFRONT = path queues, kept as a comparison form   */
    uint32_t shade_lanes;     /* regeneration: lanes of a wave that must wait for a    */
-                             /* shading step before the wave shades (1..64; 0 = 16)  */
+                             /* shading step before the wave shades (1..64; 0 = 32,  */
+                             /* 16 over binary records)                              */
    uint32_t leaf_lanes;      /* traversal: lanes of a wave that must reach a leaf     */
-                             /* before the wave runs a leaf step (1..64; 0 = 1 for   */
-                             /* ray queries, 16 for rendering)                       */
+                             /* before the wave runs a leaf step (1..64; 0 = 24 for  */
+                             /* ray queries and path rounds over the four-wide tree, */
+                             /* over binary records 1 for queries; 16 elsewhere)     */
    uint32_t plain_primary;   /* ptx_render, PTX_PLAIN_*: DEFAULT renders the job as a */
                              /* batch of one; CACHED and RETRACE take one launch per */
                              /* sample, CACHED tracing each pixel's primary ray once */

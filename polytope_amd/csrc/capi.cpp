@@ -603,7 +603,7 @@ int ptx_get_tuning(ptx_device *dev, ptx_tuning *t) {
    if (!t->block_size) t->block_size = 256;
    if (!t->refill_lanes) t->refill_lanes = kDefaultRefillLanes;
    // leaf_lanes stays 0 when unset: each kernel family then uses its own default
-   if (!t->shade_lanes) t->shade_lanes = RenderEngine::kDefaultShadeLanes;
+   if (!t->shade_lanes) t->shade_lanes = RenderEngine::kWideShadeLanes;   // what nearly every scene's kernels take
    return PTX_OK;
 }
 

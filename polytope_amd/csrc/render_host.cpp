@@ -367,12 +367,13 @@ int RenderEngine::round(const Chunk *d_round, const std::vector<Chunk> &r, uint3
       if (rc) return rc;
    }
    if (regen_round((uint32_t)r.size(), nscenes)) {
-      const uint32_t shade_min = tun.shade_lanes ? tun.shade_lanes : kDefaultShadeLanes;
+      const uint32_t shade_min = tun.shade_lanes ? tun.shade_lanes : wide ? kWideShadeLanes : kDefaultShadeLanes;
+      const uint32_t leaf_min = tun.leaf_lanes || !wide ? leaf_lanes_of(tun, true) : kDefaultWideLeafLanes;
       Deal deal{};
       const uint32_t grid = wide ? deal_ids(paths_grid, (uint32_t)dev->num_cus, nslots, deal)
                                  : std::min<uint32_t>(paths_grid, (nslots + 255) / 256);
       launch_paths(d_round, (uint32_t)r.size(), nslots, d_jobs, d_scenes, wide ? d_wides : nullptr, nscenes, res, deal,
-                   words + kWork, spill, wide ? wide_cap : stack_cap, shade_min, leaf_lanes_of(tun, true), nee ? nee_scratch : nullptr, glossy, textured, grid,
+                   words + kWork, spill, wide ? wide_cap : stack_cap, shade_min, leaf_min, nee ? nee_scratch : nullptr, glossy, textured, grid,
                    stream);
       launch_accumulate(d_round, (uint32_t)r.size(), d_jobs, res, nullptr, shade_grid, stream);
       return PTX_OK;

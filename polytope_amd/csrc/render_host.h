@@ -27,6 +27,11 @@ struct RenderEngine {
    static constexpr uint32_t kDefaultRegenPaths = 1u << 30;   // regeneration rounds (12 B per slot)
    static constexpr uint32_t kDefaultPlainPaths = 1u << 26;   // the same for ptx_render's one job
    static constexpr uint32_t kDefaultShadeLanes = 16;   // lanes a wave gathers before it shades
+   // ... and over the four-wide form, whose traversal steps cost half as much
+   // beside the shading's: 12 / 16 / 24 / 32 / 40 lanes 54.2 / 51.3 / 48.8 /
+   // 48.0 / 48.1 ms on 16 jobs of 2.7 M faces, with 24 instead of 16 lanes at
+   // leaves 46.9 (32).
+   static constexpr uint32_t kWideShadeLanes = 32;
    // layout of `words`: 8 traversal work words (word 0 counts the dynamic
    // batches handed out), the two queue counts, the bounce index, the
    // shadow-queue count

@@ -95,7 +95,7 @@ uint32_t lds_depth_of(const ptx_tuning &t);
 // 16 for the render kernels (whose leaf and shading steps share the wave).
 constexpr uint32_t kDefaultLeafLanes = 1;
 constexpr uint32_t kDefaultRenderLeafLanes = 16;
-// Four-wide ray queries: a leaf step runs for the whole wave beside one in nine
+// Four-wide traversals: a leaf step runs for the whole wave beside one in nine
 // node steps, so it waits for 24 lanes (8, 16, 24 and 32 lanes: 1,434, 1,371,
 // 1,348 and 1,344 us on a 4K frame's primary rays, 760, 718, 717 and 720 on
 // 2^21 incoherent ones, 1.3 M faces); new rays for 8 idle lanes (1 %).
