@@ -1246,18 +1246,24 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
    float src[3] = {1.f, 1.f, 1.f};
    float direct[3] = {0.f, 0.f, 0.f};    // next-event sum of the path (kNee)
    float pend[3] = {0.f, 0.f, 0.f};      // the light term a running shadow ray decides (kNee)
-   // the lane's scene arrays: the records its traversal steps over and its faces
+   // The lane's scene: the records its traversal steps over and, over binary
+   // records, its faces.  A four-wide leaf step reads its faces' address from LDS,
+   // and the hit's mesh is read from the face once the traversal has ended: three
+   // registers fewer through the traversal, where this kernel is at its limit of
+   // 128 (next-event variants 60-77 spilled -> 25-55; two next-event jobs with
+   // vertex normals 5.32 -> 4.87 ms, three of five materials 2.89 -> 2.84).
    const std::conditional_t<kWide, WideNode, Node64> *nodes = nullptr;
-   const std::conditional_t<kWide, WideFace, float> *tris = nullptr;
+   const float *tris = nullptr;          // binary records; a four-wide leaf step takes its scene's from LDS
    auto scene_of = [&](uint32_t lane_word) { return sch[lw_chunk(lane_word)].scene; };
    // the 9 corner coordinates of the hit's face
    auto hit_corners = [&](float *v) {
       if constexpr (kWide) {
-         const PTX_GLOBAL f32x4u *p = as_global(reinterpret_cast<const f32x4u *>(tris + s.hit));
+         const WideFace *face = swd[scene_of(mode)].faces + s.hit;
+         const PTX_GLOBAL f32x4u *p = as_global(reinterpret_cast<const f32x4u *>(face));
          const f32x4u a = p[0], b = p[1];
          v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
          v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-         v[8] = as_global(reinterpret_cast<const float *>(tris + s.hit))[8];
+         v[8] = as_global(reinterpret_cast<const float *>(face))[8];
       } else {
          const PTX_GLOBAL float *p = as_global(tris + 9 * (size_t)s.hit);
 #pragma unroll
@@ -1323,7 +1329,7 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
              !__builtin_amdgcn_ballot_w64(tr && (int)s.cur >= 0)) {
             if (leaf) {
                const uint32_t sc = scene_of(mode);
-               wide_leaf_or_exact(s, tris, swd[sc].leaves, binary_of(ssc[sc]), st, !shadow && (mode & kPDbg) != 0,
+               wide_leaf_or_exact(s, swd[sc].faces, swd[sc].leaves, binary_of(ssc[sc]), st, !shadow && (mode & kPDbg) != 0,
                                   shadow);
                if (shadow && s.hit != kNone) s.cur = kNone;      // occluded
             }
@@ -1336,7 +1342,7 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
                write_res(res, slot, fin<kNee>(miss_radiance(ssc[scene_of(mode)], src), direct, mode));
                mode = kPIdle;
             } else {
-               t0 = s.mesh;
+               t0 = as_global(swd[scene_of(mode)].faces + s.hit)->mesh;
                mode = lw_with_state(mode, kTex ? kPShade1 : kPShade2);
             }
             m0 = mode & kPModeMask;
@@ -1619,7 +1625,6 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
             bounce<kGlossy>(M, fr, lin, pixel, sample, b, seed, wout, src);
             if constexpr (kWide) {
                nodes = swd[scene].nodes;
-               tris = swd[scene].faces;
             } else {
                nodes = S.nodes;
                tris = S.tris;
