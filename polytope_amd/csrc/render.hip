@@ -18,7 +18,8 @@
 //             traverse.h fed from a queue) and k_shade (frame, BRDF, compaction
 //             into the next queue).
 // Batched rounds end with k_accumulate, which adds each pixel's samples to its
-// film in sample order; k_finalize scales by 1/spp.
+// film in sample order and scales by 1/spp after the last; the launches per
+// sample end with k_finalize, which does that.
 //
 // All forms run the same arithmetic in the same order, so their films are
 // identical to each other and to the CPU restatement.
@@ -901,9 +902,12 @@ __global__ void __launch_bounds__(256) k_accumulate(const Chunk *chunks, uint32_
       const JobDev &J = jobs[c.job];
       // wavefront form: a next-event job's sample is its terminal radiance plus its next-event sum
       const bool add = direct && (J.flags & PTX_JOB_NEE);
+      const bool last = c.s0 + c.k == J.spp;
+      const float div = 1.0f / (float)J.spp;
       for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < c.npix; p += gridDim.x * blockDim.x) {
          float *film = J.film + 3 * (size_t)p;
-         float ar = film[0], ag = film[1], ab = film[2];
+         float ar = 0.f, ag = 0.f, ab = 0.f;
+         if (c.s0 != 0) { ar = film[0]; ag = film[1]; ab = film[2]; }
          for (uint32_t s = 0; s < c.k; s++) {
             const size_t slot = (size_t)c.base + (size_t)s * c.npix + p;
             const float *r = res + 3 * slot;
@@ -918,6 +922,7 @@ __global__ void __launch_bounds__(256) k_accumulate(const Chunk *chunks, uint32_
             if (sb > 255) sb = 255;
             ar += sr; ag += sg; ab += sb;
          }
+         if (last) { ar *= div; ag *= div; ab *= div; }
          film[0] = ar; film[1] = ag; film[2] = ab;
       }
    }
@@ -946,6 +951,16 @@ __global__ void k_zero_words(uint32_t *a, uint32_t na, uint32_t *b, uint32_t nb)
    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
    if (i < na) a[i] = 0u;
    if (b && i < nb) b[i] = 0u;
+}
+
+__global__ void __launch_bounds__(256) k_copy_words(uint32_t *dst, const uint32_t *src, size_t n) {
+   typedef uint32_t u32x4_ __attribute__((ext_vector_type(4)));
+   const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+   if (4 * i + 4 <= n) {
+      reinterpret_cast<u32x4_ *>(dst)[i] = reinterpret_cast<const u32x4_ *>(src)[i];
+   } else {
+      for (size_t k = 4 * i; k < n; k++) dst[k] = src[k];
+   }
 }
 
 __global__ void k_zero_floats(float *a, size_t n) {
@@ -1676,9 +1691,15 @@ int render_blocks_per_cu(int which) {
    return e == hipSuccess && b > 0 ? b : 1;
 }
 
+namespace {
+void zero_work(uint32_t *work, hipStream_t st) {
+   hipLaunchKernelGGL(dev::k_zero_words, dim3(1), dim3(64), 0, st, work, 8u, (uint32_t *)nullptr, 0u);
+}
+}  // namespace
+
 void launch_primary(const DevScene &S, const WideScene *W, const JobDev &J, const Deal &deal, uint32_t *work,
                     uint4 *spill, uint32_t leaf_min, uint32_t grid, hipStream_t st) {
-   hipLaunchKernelGGL(dev::k_zero_words, dim3(1), dim3(64), 0, st, work, 8u, (uint32_t *)nullptr, 0u);
+   if (!W || counted(deal)) zero_work(work, st);
    if (W)
       hipLaunchKernelGGL(dev::k_primary_wide<kRenderLds>, dim3(grid), dim3(256), 0, st, S, *W, J, deal, work,
                          reinterpret_cast<uint2 *>(spill), leaf_min);
@@ -1689,7 +1710,7 @@ void launch_primary(const DevScene &S, const WideScene *W, const JobDev &J, cons
 void launch_primaries(const JobDev *jobs, const DevScene *scenes, const WideScene *wides, const uint32_t *offsets,
                       uint32_t njobs, const Deal &deal, uint32_t *work, uint4 *spill, uint32_t leaf_min, uint32_t max_stack,
                       uint32_t grid, hipStream_t st) {
-   hipLaunchKernelGGL(dev::k_zero_words, dim3(1), dim3(64), 0, st, work, 8u, (uint32_t *)nullptr, 0u);
+   if (!wides || counted(deal)) zero_work(work, st);
    if (wides)
       hipLaunchKernelGGL(dev::k_primaries_wide<kRenderLds>, dim3(grid), dim3(256), 0, st, jobs, scenes, wides, offsets,
                          njobs, deal, work, reinterpret_cast<uint2 *>(spill), leaf_min, max_stack);
@@ -1739,6 +1760,10 @@ void launch_finalize(float *film, uint32_t npix, uint32_t spp, hipStream_t st) {
 void launch_zero_floats(float *a, size_t n, hipStream_t st) {
    const uint32_t grid = (uint32_t)std::min<size_t>(4096, (n + 255) / 256);
    hipLaunchKernelGGL(dev::k_zero_floats, dim3(std::max(1u, grid)), dim3(256), 0, st, a, n);
+}
+
+void launch_copy_words(uint32_t *dst, const uint32_t *src, size_t n, hipStream_t st) {
+   hipLaunchKernelGGL(dev::k_copy_words, dim3((uint32_t)((n / 4 + 1 + 255) / 256)), dim3(256), 0, st, dst, src, n);
 }
 
 int paths_blocks_per_cu() {
@@ -1794,7 +1819,7 @@ void launch_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const 
                   const WideScene *wides, uint32_t nscenes, float *res, const Deal &deal, uint32_t *work, uint4 *spill,
                   uint32_t max_stack, uint32_t shade_min, uint32_t leaf_min, float4 *nee_scratch, bool glossy,
                   bool textured, uint32_t grid, hipStream_t st) {
-   hipLaunchKernelGGL(dev::k_zero_words, dim3(1), dim3(64), 0, st, work, 8u, (uint32_t *)nullptr, 0u);
+   if (!wides || counted(deal)) zero_work(work, st);
    const int v = (nee_scratch ? 1 : 0) | (glossy ? 2 : 0) | (textured ? 4 : 0);
    if (wides)
       launch_paths_t<true>(v, chunks, nchunks, nslots, jobs, scenes, wides, nscenes, res, deal, work, spill, max_stack,

@@ -148,7 +148,10 @@ void RenderEngine::release() {
    }
    dfree(qa); dfree(qb); dfree(hits); dfree(qs); dfree(direct); dfree(res); dfree(words); dfree(spill);
    dfree(nee_scratch);
-   dfree(d_jobs); dfree(d_offsets); dfree(d_scenes); dfree(d_wides); dfree(d_chunks);
+   dfree(tables);
+   if (tables_host) (void)hipHostFree(tables_host);
+   tables_host = nullptr;
+   tables_host_bytes = 0;
    cap = qcap = 0;
    jobs_cap = scenes_cap = chunks_cap = 0;
    spill_entries = 0;
@@ -210,33 +213,26 @@ int RenderEngine::ensure(uint32_t paths, uint32_t max_stack, uint32_t wide_stack
       graphs_stale = true;
    }
    wide_cap = lds + 2 * (uint32_t)(spill_entries / stride_threads);
-   // a table's capacity is recorded only once its allocation succeeded
-   if (njobs > jobs_cap) {
-      dfree(d_jobs);
-      dfree(d_offsets);
-      jobs_cap = 0;
-      const uint32_t want = std::max(njobs, 64u);
-      if ((rc = dalloc(this, &d_jobs, want))) return rc;
-      if ((rc = dalloc(this, &d_offsets, want + 1))) return rc;
-      jobs_cap = want;
+   if (njobs > jobs_cap || nscenes > scenes_cap || nchunks > chunks_cap) {
+      const uint32_t jc = std::max({njobs, jobs_cap, 64u}), sc = std::max({nscenes, scenes_cap, 16u});
+      const uint32_t cc = std::max({nchunks, chunks_cap, 1024u});
+      dfree(tables);
+      jobs_cap = scenes_cap = chunks_cap = 0;      // recorded only once the allocation succeeded
+      size_t at = 0;
+      auto place = [&](size_t bytes) { const size_t o = at; at = (at + bytes + 255) & ~size_t(255); return o; };
+      const size_t o_jobs = place(jc * sizeof(JobDev)), o_offsets = place((jc + 1) * sizeof(uint32_t));
+      const size_t o_scenes = place(sc * sizeof(DevScene)), o_wides = place(sc * sizeof(WideScene));
+      const size_t o_chunks = place(cc * sizeof(Chunk));
+      if ((rc = dalloc(this, &tables, at))) return rc;
+      d_jobs = reinterpret_cast<JobDev *>(tables + o_jobs);
+      d_offsets = reinterpret_cast<uint32_t *>(tables + o_offsets);
+      d_scenes = reinterpret_cast<DevScene *>(tables + o_scenes);
+      d_wides = reinterpret_cast<WideScene *>(tables + o_wides);
+      d_chunks = reinterpret_cast<Chunk *>(tables + o_chunks);
+      jobs_cap = jc;
+      scenes_cap = sc;
+      chunks_cap = cc;
       graphs_stale = true;
-   }
-   if (nscenes > scenes_cap) {
-      dfree(d_scenes);
-      dfree(d_wides);
-      scenes_cap = 0;
-      const uint32_t want = std::max(nscenes, 16u);
-      if ((rc = dalloc(this, &d_scenes, want))) return rc;
-      if ((rc = dalloc(this, &d_wides, want))) return rc;
-      scenes_cap = want;
-      graphs_stale = true;
-   }
-   if (nchunks > chunks_cap) {
-      dfree(d_chunks);
-      chunks_cap = 0;
-      const uint32_t want = std::max(nchunks, 1024u);
-      if ((rc = dalloc(this, &d_chunks, want))) return rc;
-      chunks_cap = want;
    }
    return PTX_OK;
 }
@@ -353,7 +349,6 @@ int RenderEngine::start_job(JobDev &J, const ptx_scene *scene, uint32_t npix, bo
       free_job(J);
       return set_error(PTX_ERR_OOM, std::string("job film and primary records: ") + hipGetErrorString(e));
    }
-   launch_zero_floats(J.film, (size_t)npix * 3, stream);
    if (trace_primary) trace_primary_of(J, scene, npix);
    return PTX_OK;
 }
@@ -393,13 +388,6 @@ int RenderEngine::round(const Chunk *d_round, const std::vector<Chunk> &r, uint3
       }
    }
    launch_accumulate(d_round, (uint32_t)r.size(), d_jobs, res, nee ? direct : nullptr, shade_grid, stream);
-   return PTX_OK;
-}
-
-int RenderEngine::finish_job(JobDev &J, uint32_t npix, uint32_t spp, float *film_host) {
-   launch_finalize(J.film, npix, spp, stream);
-   if (film_host)
-      PTX_HIP_TRY(hipMemcpyAsync(film_host, J.film, (size_t)npix * 3 * sizeof(float), hipMemcpyDeviceToHost, stream));
    return PTX_OK;
 }
 
@@ -471,23 +459,43 @@ int RenderEngine::run_batch(const std::vector<RenderJob> &jobs, const std::vecto
    std::vector<Chunk> all;
    all.reserve(nchunks);
    for (const auto &r : rounds) all.insert(all.end(), r.begin(), r.end());
-   {
-      // the tables go up before any round; a failed copy still frees every job's buffers
-      hipError_t e = hipMemcpyAsync(d_jobs, jd.data(), nj * sizeof(JobDev), hipMemcpyHostToDevice, st);
-      if (e == hipSuccess)
-         e = hipMemcpyAsync(d_scenes, sd.data(), sd.size() * sizeof(DevScene), hipMemcpyHostToDevice, st);
-      if (e == hipSuccess && wide)
-         e = hipMemcpyAsync(d_wides, wd.data(), wd.size() * sizeof(WideScene), hipMemcpyHostToDevice, st);
-      if (e == hipSuccess && !all.empty())
-         e = hipMemcpyAsync(d_chunks, all.data(), all.size() * sizeof(Chunk), hipMemcpyHostToDevice, st);
-      if (e == hipSuccess && one_launch)
-         e = hipMemcpyAsync(d_offsets, offsets.data(), (nj + 1) * sizeof(uint32_t), hipMemcpyHostToDevice, st);
-      if (e != hipSuccess) {
-         (void)hipGetLastError();
-         (void)hipStreamSynchronize(st);
-         cleanup();
-         return set_error(PTX_ERR_HIP, std::string("render batch tables: ") + hipGetErrorString(e));
+   // the tables go up before any round, in one launch out of their pinned
+   // mirror (the call ends with the stream idle, so the mirror is free again)
+   const size_t up = (size_t)(reinterpret_cast<char *>(d_chunks + all.size()) - tables);
+   std::vector<char> pageable;
+   if (tables_host_bytes < up) {
+      if (tables_host) (void)hipHostFree(tables_host);
+      tables_host = nullptr;
+      tables_host_bytes = 0;
+      if (hipHostMalloc(reinterpret_cast<void **>(&tables_host), 2 * up, hipHostMallocDefault) == hipSuccess) {
+         tables_host_bytes = 2 * up;
+      } else {
+         (void)hipGetLastError();      // no pinned memory: an ordinary copy
+         tables_host = nullptr;
+         pageable.resize(up);
       }
+   }
+   char *mirror = tables_host ? tables_host : pageable.data();
+   auto fill = [&](const void *d_at, const void *src, size_t bytes) {
+      if (bytes) std::memcpy(mirror + (static_cast<const char *>(d_at) - tables), src, bytes);
+   };
+   fill(d_jobs, jd.data(), nj * sizeof(JobDev));
+   fill(d_offsets, offsets.data(), (nj + 1) * sizeof(uint32_t));
+   fill(d_scenes, sd.data(), sd.size() * sizeof(DevScene));
+   fill(d_wides, wd.data(), wd.size() * sizeof(WideScene));
+   fill(d_chunks, all.data(), all.size() * sizeof(Chunk));
+   hipError_t e = hipSuccess;
+   if (tables_host) {
+      launch_copy_words(reinterpret_cast<uint32_t *>(tables), reinterpret_cast<const uint32_t *>(mirror), up / 4, st);
+      e = hipGetLastError();
+   } else {
+      e = hipMemcpyAsync(tables, mirror, up, hipMemcpyHostToDevice, st);
+   }
+   if (e != hipSuccess) {
+      (void)hipGetLastError();
+      (void)hipStreamSynchronize(st);
+      cleanup();              // a failed copy still frees every job's buffers
+      return set_error(PTX_ERR_HIP, std::string("render batch tables: ") + hipGetErrorString(e));
    }
    if (one_launch) {
       Deal deal{};
@@ -515,17 +523,12 @@ int RenderEngine::run_batch(const std::vector<RenderJob> &jobs, const std::vecto
    }
    // films back through the pinned staging, several host threads at once
    std::vector<Span> films;
-   for (uint32_t j = 0; j < nj; j++) {
-      if ((rc = finish_job(jd[j], jobs[j].npix, jobs[j].desc.spp, nullptr))) {
-         (void)hipStreamSynchronize(st);
-         cleanup();
-         return rc;
-      }
+   for (uint32_t j = 0; j < nj; j++)
       if (films_host[j])
          films.push_back(Span{reinterpret_cast<char *>(films_host[j]), reinterpret_cast<char *>(jd[j].film),
                               (size_t)jobs[j].npix * 3 * sizeof(float)});
-   }
    rc = download_host(dev, st, films);
+   if (rc) (void)hipStreamSynchronize(st);      // the tables' mirror is free again on every way out
    cleanup();
    return rc;
 }

@@ -55,6 +55,13 @@ struct RenderEngine {
    size_t spill_entries = 0;
    uint32_t stack_cap = 0;                  // binary stack levels the spill holds
    uint32_t wide_cap = 0;                   // four-wide stack entries it holds
+   // The round tables, one device allocation: jobs, offsets, scenes, four-wide
+   // forms, chunks.  A batch fills a pinned mirror of it and one launch brings
+   // all of them up (a copy each, from pageable memory, took about 10 us of
+   // host time apiece, five of them before a batch's first ray).
+   char *tables = nullptr;
+   char *tables_host = nullptr;             // pinned mirror, made by the first batch
+   size_t tables_host_bytes = 0;
    JobDev *d_jobs = nullptr;
    uint32_t *d_offsets = nullptr;           // jobs_cap + 1 entries: first primary-ray id of each job
    uint32_t jobs_cap = 0;
@@ -108,9 +115,10 @@ struct RenderEngine {
    // per-bounce graphs.
    int ensure_queues(uint32_t need);
    ShadowArgs shadow_args() const { return ShadowArgs{qs, words + kCountS, direct, connect_grid}; }
-   // Allocates the job's film and primary records, zeroes the film and, with
-   // trace_primary, traces the primary hits (a batch traces every job's in
-   // one launch instead).  J.film / J.primary are set.
+   // Allocates the job's film and primary records and, with trace_primary,
+   // traces the primary hits (a batch traces every job's in one launch
+   // instead).  J.film / J.primary are set; the film holds nothing until its
+   // job's first chunk has been added to it.
    int start_job(JobDev &J, const ptx_scene *scene, uint32_t npix, bool trace_primary = true);
    // The job's primary records, traced on the engine's stream.
    void trace_primary_of(const JobDev &J, const ptx_scene *scene, uint32_t npix);
@@ -121,9 +129,6 @@ struct RenderEngine {
    // wide: wide_scene() of every scene of the round.
    int round(const Chunk *d_round, const std::vector<Chunk> &r, uint32_t depth, uint32_t nscenes, bool nee,
              bool glossy, bool textured, bool wide);
-   // Queues the film's finalisation and, when film_host is not NULL (the
-   // server's pinned films), its copy there.
-   int finish_job(JobDev &J, uint32_t npix, uint32_t spp, float *film_host);
    void free_job(JobDev &J);
    uint32_t capacity_for(uint64_t total_paths, uint32_t max_npix, bool regen, uint32_t regen_paths) const;
    // regen_paths: path slots of a regeneration round when the tuning names none.

@@ -378,7 +378,7 @@ void ptx_server::loop() {
                j.inflight++;
             }
          }
-         // jobs whose last chunk is in this round: finalise and copy the film behind it
+         // jobs whose last chunk is in this round: copy the film behind it
          for (auto &pj : r.parts) {
             JobState &j = *pj.first;
             if (j.next_sample < j.desc.spp || r.rc != PTX_OK) continue;
@@ -387,7 +387,10 @@ void ptx_server::loop() {
             j.film = take_film(j.film_bytes);
             j.done_ev = take_event();
             int rc = j.film && j.done_ev ? PTX_OK : set_error(PTX_ERR_OOM, "server: pinned film or event");
-            if (rc == PTX_OK) rc = eng.finish_job(j.jd, j.npix, j.desc.spp, j.film);
+            if (rc == PTX_OK && hipMemcpyAsync(j.film, j.jd.film, j.film_bytes, hipMemcpyDeviceToHost, stream) != hipSuccess) {
+               (void)hipGetLastError();
+               rc = set_error(PTX_ERR_HIP, "server: film download");
+            }
             if (rc == PTX_OK && hipEventRecord(j.done_ev, stream) != hipSuccess) {
                (void)hipGetLastError();
                rc = PTX_ERR_HIP;

@@ -294,8 +294,8 @@ int blocks_wide(bool frames) {
 int launch_closest_hit_wide(const DevScene &sc, const WideScene &w, const float *d_rays, const Deal &deal, ptx_hit *d_hits,
                             ptx_hit_frame *d_frames, uint32_t *d_work, void *d_spill, uint32_t grid,
                             uint32_t lds_depth, uint32_t refill_min, uint32_t leaf_min, hipStream_t stream) {
-   hipLaunchKernelGGL(dev::k_zero_u32, dim3(1), dim3(64), 0, stream, d_work, (uint32_t)dev::kWorkWords);
    if (deal.n == 0) return 0;
+   if (counted(deal)) hipLaunchKernelGGL(dev::k_zero_u32, dim3(1), dim3(64), 0, stream, d_work, (uint32_t)dev::kWorkWords);
    uint2 *spill = static_cast<uint2 *>(d_spill);
    switch (lds_depth) {
       case 8: launch_wide<8>(sc, w, d_rays, deal, d_hits, d_frames, d_work, spill, grid, refill_min, leaf_min, stream); break;

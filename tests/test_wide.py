@@ -133,3 +133,70 @@ def test_render_forms_agree(case, size):
     finally:
         scene.close()
         dev.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("extra", [-1, 0, 1, 64])
+def test_launches_with_and_without_the_batch_counter_agree(extra):
+    """Ids that one block per CU deals out in batches of 64 without the
+    counter, which no kernel clears then, and the first that need it, each
+    behind a launch that leaves the counter's scratch dirty."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from polytope_amd import Device, Scene
+    verts, faces = _scene("slivers")
+    meshes = [S.MeshData(verts, faces)]
+    n = 4 * 64 * torch.cuda.get_device_properties(0).multi_processor_count + extra
+    lo, hi = S.scene_bounds(meshes)
+    rays = S.rays_incoherent(np.asarray(lo) - 0.2, np.asarray(hi) + 0.2, 3 * n, 5)
+    dev = Device(0)
+    scene = Scene(dev, meshes)
+    dev.set_tuning(blocks_per_cu=1)
+    r = torch.from_numpy(rays).cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def query(m: int, counters: bool):
+        h = torch.full((m, 6), -7, dtype=torch.int32, device="cuda")
+        c = torch.zeros((m, 3), dtype=torch.int32, device="cuda")
+        scene.intersect_device(r.data_ptr(), m, h.data_ptr(), c.data_ptr() if counters else 0, 0, stream)
+        torch.cuda.synchronize()
+        return h.cpu().numpy()
+
+    try:
+        whole = query(3 * n, True)
+        for _ in range(2):
+            assert np.array_equal(query(3 * n, False), whole)
+            assert np.array_equal(query(n, False), whole[:n])
+    finally:
+        scene.close()
+        dev.close()
+
+
+@pytest.mark.gpu
+def test_batch_tables_grow_and_films_span_rounds():
+    """Batches of 2, 70 and 2 jobs over one engine (its tables grow once) whose
+    films are summed over several rounds and in one: the films of one launch
+    per sample."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from polytope_amd import Device, Scene, _abi, render, render_batch
+    dev = Device(0)
+    scenes, jobs, want = [], [], []
+    try:
+        dev.set_tuning(plain_primary=_abi.PLAIN_CACHED)
+        for w, h in ((17, 9), (32, 8)):
+            meshes, cam, sky = S.plain_render_scene(1, w, h)
+            scenes.append(Scene(dev, meshes, sky))
+            jobs.append((scenes[-1], cam, 5, 3, 3))
+            want.append(render(*jobs[-1]).view(np.uint32))
+        for paths in (0, 700):
+            dev.set_tuning(paths_per_wave=paths)
+            for n in (2, 70, 2):
+                for i, film in enumerate(render_batch([jobs[i % 2] for i in range(n)])):
+                    assert np.array_equal(film.view(np.uint32), want[i % 2])
+    finally:
+        for s in scenes:
+            s.close()
+        dev.close()
