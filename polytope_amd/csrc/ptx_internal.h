@@ -38,8 +38,8 @@ static_assert(sizeof(Node64) == 64, "Node64 is 64 bytes");
 constexpr uint32_t kLeafBit = 0x80000000u;
 
 // Four-wide form of the tree (wide.h): up to four descendants of a binary
-// node, their boxes in steps of 2^exponent from the node's low corner, rounded
-// outwards.  planes: low and high x, low and high y, low and high z, child k in
+// node, their boxes in steps of 2^(exponent - 24) from the node's low corner,
+// rounded outwards (a plane's byte read as a half is 2^-24 times its steps).  planes: low and high x, low and high y, low and high z, child k in
 // byte k.  later[q], q = octant of the rays whose z direction is not negative
 // (bit a set: direction a negative): bits 4 k .. 4 k + 3 = the children visited
 // after child k; the octant with every sign flipped visits in reverse.  Only

@@ -1185,9 +1185,23 @@ __device__ __forceinline__ void p_begin(const DevScene &S, uint32_t wroot, Trav 
    }
 }
 
+// Three floats of a lane, in registers or in LDS (one plane of the block's lanes
+// per component).
+template <bool kInLds>
+struct LaneVec3 {
+   float v[3];
+   __device__ __forceinline__ float &operator[](uint32_t k) { return v[k]; }
+   __device__ __forceinline__ float operator[](uint32_t k) const { return v[k]; }
+};
+template <>
+struct LaneVec3<true> {
+   float *p;
+   __device__ __forceinline__ float &operator[](uint32_t k) const { return p[k * 256]; }
+};
+
 // Terminal radiance of a path plus its next-event sum (paths of next-event jobs).
-template <bool kNee>
-__device__ __forceinline__ Radiance fin(Radiance R, const float direct[3], uint32_t lane_word) {
+template <bool kNee, class Sum>
+__device__ __forceinline__ Radiance fin(Radiance R, const Sum &direct, uint32_t lane_word) {
    if (kNee && (lane_word & kPNee)) {
       R.r = R.r + direct[0];
       R.g = R.g + direct[1];
@@ -1198,9 +1212,9 @@ __device__ __forceinline__ Radiance fin(Radiance R, const float direct[3], uint3
 
 // Starts the traversal of ray s.r in scene S; returns the next state, or kPIdle
 // after writing the miss result when the root box is missed.
-template <bool kNee, bool kWide>
+template <bool kNee, bool kWide, class Sum>
 __device__ __forceinline__ uint32_t p_root(const DevScene &S, uint32_t wroot, Trav &s, float *res, uint32_t slot,
-                                           const float src[3], const float direct[3], uint32_t lane_word) {
+                                           const float src[3], const Sum &direct, uint32_t lane_word) {
    p_begin<kWide>(S, wroot, s);
    if (s.cur != kNone) return kPTrace;
    write_res(res, slot, fin<kNee>(miss_radiance(S, src), direct, lane_word));
@@ -1259,7 +1273,13 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
    // Shade1 -> Shade2 of a textured hit keeps the texel's address and the texture
    // record's flags in ray words a found hit no longer needs (origin, 1 / d)
    float src[3] = {1.f, 1.f, 1.f};
-   float direct[3] = {0.f, 0.f, 0.f};    // next-event sum of the path (kNee)
+   // Next-event sum of the path (kNee).  In LDS beside the four-wide stack, where
+   // a block has 4 KB left of a fourth of the CU's 160 KB (the binary form none).
+   LaneVec3<kNee && kWide> direct{};
+   if constexpr (kNee && kWide) {
+      __shared__ float sums[3 * 256];
+      direct.p = sums + threadIdx.x;
+   }
    float pend[3] = {0.f, 0.f, 0.f};      // the light term a running shadow ray decides (kNee)
    // The lane's scene: the records its traversal steps over and, over binary
    // records, its faces.  A four-wide leaf step reads its faces' address from LDS,

@@ -21,7 +21,8 @@ namespace ptx {
 namespace {
 
 constexpr uint32_t kWide = 4;
-constexpr float kLimit = 1e18f;                // kWideLimit of wide.h
+constexpr float kLimit = 1e16f;                // kWideLimit of wide.h
+constexpr int kStepExponent = 24;              // kWideStep of wide.h
 constexpr uint32_t kIndexEnd = 0x1FFFFFFEu;    // leaf indices stay below the reserved references
 constexpr uint32_t kMaxNodes = 1u << 26;       // 32-bit byte offsets into the node array
 constexpr uint32_t kLeafHeader = kLeafBit, kLeafOne = kLeafBit | (1u << 29), kLeafTwo = kLeafBit | (2u << 29);
@@ -214,7 +215,7 @@ bool build_wide(const HostBvh &bvh, const HostImage &img, unsigned threads, Wide
                while (extent * pow2(-e) > 255.0) e++;
             }
             o.org[a] = lo;
-            o.exponent[a] = (int8_t)e;
+            o.exponent[a] = (int8_t)(e + kStepExponent);
             const double inv = pow2(-e);
             for (uint32_t k = 0; k < kWide; k++) {
                uint8_t &p0 = o.planes[2 * a][k], &p1 = o.planes[2 * a + 1][k];

@@ -200,3 +200,38 @@ def test_batch_tables_grow_and_films_span_rounds():
         for s in scenes:
             s.close()
         dev.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [1e-15, 4e15, 2e16, 3e17])
+def test_scenes_at_the_edges_of_the_wide_ranges_agree(scale):
+    """Extents far below one, just inside and past the limit of the four-wide
+    test's range, with directions whose reciprocals lie on both sides of it."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from polytope_amd import Device, Scene
+    verts, faces = _scene("sphere")
+    lo, hi = S.scene_bounds([S.MeshData(verts, faces)])
+    n = 4001
+    rays = S.rays_incoherent(np.asarray(lo) - 0.2, np.asarray(hi) + 0.2, n, 9)
+    rays[:, :3] *= np.float32(scale)
+    for i, d in enumerate((3e-16, -5e-17, 1e-18, 1e20)):
+        rays[i::9, 3 + i % 3] = d
+    meshes = [S.MeshData((verts * np.float32(scale)).astype(np.float32), faces)]
+    dev = Device(0)
+    scene = Scene(dev, meshes)
+    r = torch.from_numpy(rays).cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+    out = []
+    try:
+        for counters in (True, False):
+            h = torch.full((n, 6), -7, dtype=torch.int32, device="cuda")
+            c = torch.zeros((n, 3), dtype=torch.int32, device="cuda")
+            scene.intersect_device(r.data_ptr(), n, h.data_ptr(), c.data_ptr() if counters else 0, 0, stream)
+            torch.cuda.synchronize()
+            out.append(h.cpu().numpy())
+        assert np.array_equal(*out)
+    finally:
+        scene.close()
+        dev.close()
