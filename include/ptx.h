@@ -296,7 +296,7 @@ typedef struct ptx_tuning {
    uint32_t leaf_lanes;      /* traversal: lanes of a wave that must reach a leaf     */
                              /* before the wave runs a leaf step (1..64; 0 = 24 for  */
                              /* ray queries and path rounds over the four-wide tree, */
-                             /* over binary records 1 for queries; 16 elsewhere)     */
+                             /* 16 elsewhere)                                        */
    uint32_t plain_primary;   /* ptx_render, PTX_PLAIN_*: DEFAULT renders the job as a */
                              /* batch of one; CACHED and RETRACE take one launch per */
                              /* sample, CACHED tracing each pixel's primary ray once */

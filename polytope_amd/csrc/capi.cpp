@@ -162,9 +162,6 @@ size_t wide_spill_bytes(const ptx_scene *s, uint32_t grid, uint32_t lds) {
 uint32_t wide_refill_lanes_of(const ptx_tuning &t) {
    return t.refill_lanes ? std::min(64u, t.refill_lanes) : kDefaultWideRefillLanes;
 }
-uint32_t wide_leaf_lanes_of(const ptx_tuning &t) {
-   return t.leaf_lanes ? std::min(64u, t.leaf_lanes) : kDefaultWideLeafLanes;
-}
 
 }  // namespace
 
@@ -181,23 +178,24 @@ int run_closest_hit(ptx_scene *s, const float *d_rays, uint32_t n, ptx_hit *d_hi
       PTX_HIP_TRY(pool_malloc(dev, &scratch, 256 + wide_spill_bytes(s, grid, lds), stream));
       const int rc = launch_closest_hit_wide(s->d, s->w, d_rays, deal, d_hits, d_frames, static_cast<uint32_t *>(scratch),
                                              static_cast<char *>(scratch) + 256, grid, lds, wide_refill_lanes_of(t),
-                                             wide_leaf_lanes_of(t), stream);
+                                             leaf_lanes_of(t), stream);
       const hipError_t fe = hipFreeAsync(scratch, stream);
       if (rc != 0) return set_error(PTX_ERR_HIP, "closest-hit launch failed");
       if (fe != hipSuccess) return set_error(PTX_ERR_HIP, std::string("hipFreeAsync: ") + hipGetErrorString(fe));
       return PTX_OK;
    }
    const Node64 *win = n ? scene_windows(s, t) : nullptr;
-   uint32_t grid = closest_hit_grid(dev, t, lds, d_counters != nullptr || d_frames != nullptr, win != nullptr);
-   const uint32_t needed_blocks = (n + 255) / 256;
-   grid = std::max(1u, std::min(grid, needed_blocks));
+   Deal deal;
+   const uint32_t grid =
+         deal_ids(closest_hit_grid(dev, t, lds, d_counters != nullptr || d_frames != nullptr, win != nullptr),
+                  (uint32_t)dev->num_cus, n, deal);
    void *scratch = nullptr;
    PTX_HIP_TRY(pool_malloc(dev, &scratch, closest_hit_scratch_bytes(s, grid, lds), stream));
    uint32_t *work = static_cast<uint32_t *>(scratch);
    uint4 *spill = reinterpret_cast<uint4 *>(static_cast<char *>(scratch) + 256);
    const uint32_t refill = refill_lanes_of(t);
    const uint32_t leaf = leaf_lanes_of(t);
-   const int rc = launch_closest_hit(s->d, d_rays, n, d_hits, d_counters, d_frames, work, spill, grid, lds, refill, leaf,
+   const int rc = launch_closest_hit(s->d, d_rays, deal, d_hits, d_counters, d_frames, work, spill, grid, lds, refill, leaf,
                                      win, s->root_axis, stream);
    const hipError_t fe = hipFreeAsync(scratch, stream);
    if (rc != 0) return set_error(PTX_ERR_HIP, "closest-hit launch failed");
@@ -540,6 +538,7 @@ int ptx_intersect_closest_device_noalloc(ptx_scene *scene, const float *d_rays, 
                                 std::to_string(kNoAllocScratchBytes) + "; use ptx_intersect_closest_device");
       grid = (uint32_t)std::min<size_t>(grid, fit);
    }
+   const uint32_t grid_max = grid;
    grid = std::max(1u, std::min(grid, (n + 255) / 256));
    PTX_HIP_TRY(hipSetDevice(dev->ordinal));
    uint32_t *work = static_cast<uint32_t *>(dev->noalloc_scratch);
@@ -553,7 +552,7 @@ int ptx_intersect_closest_device_noalloc(ptx_scene *scene, const float *d_rays, 
       if (wgrid) wgrid = deal_ids(wgrid, (uint32_t)dev->num_cus, n, deal);
       if (wgrid >= std::min(grid, (uint32_t)dev->num_cus)) {
          if (launch_closest_hit_wide(scene->d, scene->w, d_rays, deal, d_hits, d_frames, work, spill, wgrid, lds,
-                                     wide_refill_lanes_of(t), wide_leaf_lanes_of(t),
+                                     wide_refill_lanes_of(t), leaf_lanes_of(t),
                                      static_cast<hipStream_t>(stream)) != 0) {
             (void)hipGetLastError();
             return set_error(PTX_ERR_HIP, "closest-hit launch failed");
@@ -562,8 +561,10 @@ int ptx_intersect_closest_device_noalloc(ptx_scene *scene, const float *d_rays, 
       }
    }
    const uint32_t refill = refill_lanes_of(t);
+   Deal deal{};
+   grid = deal_ids(grid_max, (uint32_t)dev->num_cus, n, deal);
    // the work counters are cleared by a kernel at the head of the launch (no memset)
-   if (launch_closest_hit(scene->d, d_rays, n, d_hits, d_counters, d_frames, work, spill, grid, lds, refill,
+   if (launch_closest_hit(scene->d, d_rays, deal, d_hits, d_counters, d_frames, work, spill, grid, lds, refill,
                           leaf_lanes_of(t), win, scene->root_axis, static_cast<hipStream_t>(stream)) != 0) {
       (void)hipGetLastError();
       return set_error(PTX_ERR_HIP, "closest-hit launch failed");

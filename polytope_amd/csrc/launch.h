@@ -18,7 +18,7 @@ constexpr uint32_t kDealBatch = 64;
 
 namespace ptx {
 
-// Grid and batches of a persistent four-wide launch over n ids: `full` blocks
+// Grid and batches of a persistent launch over n ids: `full` blocks
 // (what fits the device) and batches of 64, three quarters of them dealt out
 // statically, when the ids fill it; else every wave gets one batch of its
 // share, from as many blocks as hold the ids at one a lane, or as two waves
@@ -41,7 +41,7 @@ inline bool counted(const Deal &d) { return d.static_batches < d.batches; }
 
 // windows: the scene's window records (launch_build_windows), or null to step
 // over sc.nodes; root_axis: the root's split axis (used with windows).
-int launch_closest_hit(const DevScene &sc, const float *d_rays, uint32_t n, ptx_hit *d_hits,
+int launch_closest_hit(const DevScene &sc, const float *d_rays, const Deal &deal, ptx_hit *d_hits,
                        ptx_ray_counters *d_counters, ptx_hit_frame *d_frames, uint32_t *d_work, uint4 *d_spill,
                        uint32_t grid, uint32_t lds_depth, uint32_t refill_min, uint32_t leaf_min,
                        const Node64 *windows, uint32_t root_axis, hipStream_t stream);

@@ -363,7 +363,7 @@ int RenderEngine::round(const Chunk *d_round, const std::vector<Chunk> &r, uint3
    }
    if (regen_round((uint32_t)r.size(), nscenes)) {
       const uint32_t shade_min = tun.shade_lanes ? tun.shade_lanes : wide ? kWideShadeLanes : kDefaultShadeLanes;
-      const uint32_t leaf_min = tun.leaf_lanes || !wide ? leaf_lanes_of(tun, true) : kDefaultWideLeafLanes;
+      const uint32_t leaf_min = leaf_lanes_of(tun, !wide);
       Deal deal{};
       const uint32_t grid = wide ? deal_ids(paths_grid, (uint32_t)dev->num_cus, nslots, deal)
                                  : std::min<uint32_t>(paths_grid, (nslots + 255) / 256);

@@ -90,16 +90,16 @@ const char *last_error_cstr();
 ptx_tuning tuning_of(const ptx_device *dev);
 void set_tuning(ptx_device *dev, const ptx_tuning &t);
 uint32_t lds_depth_of(const ptx_tuning &t);
-// Lanes of a wave that gather at leaves before the wave runs a leaf step:
-// measured best 1 for ray queries (leaf and interior steps are balanced) and
-// 16 for the render kernels (whose leaf and shading steps share the wave).
-constexpr uint32_t kDefaultLeafLanes = 1;
+// Lanes of a wave that gather at leaves before the wave runs a leaf step, which
+// runs for the whole wave: ray queries and path rounds over the four-wide tree
+// wait for 24, with one leaf step in nine node steps (8, 16, 24 and 32 lanes:
+// 1,434, 1,371, 1,348 and 1,344 us on a 4K frame's primary rays, 760, 718, 717
+// and 720 on 2^21 incoherent ones, 1.3 M faces; over the binary records with
+// counters 1,657, 1,514, 1,490 and 1,497, and 774, 726, 721 and 728).  The
+// other render kernels, whose leaf and shading steps share the wave, take 16.
+constexpr uint32_t kDefaultLeafLanes = 24;
 constexpr uint32_t kDefaultRenderLeafLanes = 16;
-// Four-wide traversals: a leaf step runs for the whole wave beside one in nine
-// node steps, so it waits for 24 lanes (8, 16, 24 and 32 lanes: 1,434, 1,371,
-// 1,348 and 1,344 us on a 4K frame's primary rays, 760, 718, 717 and 720 on
-// 2^21 incoherent ones, 1.3 M faces); new rays for 8 idle lanes (1 %).
-constexpr uint32_t kDefaultWideLeafLanes = 24;
+// New rays of a four-wide query's wave: for 8 idle lanes (1 %).
 constexpr uint32_t kDefaultWideRefillLanes = 8;
 // Idle lanes a ray-query wave waits for before it takes new rays: 2, 4 and 8
 // measured 2,377-2,383 Mrays/s against 2,342 for 1 and 2,349 for 16 (2^21

@@ -52,8 +52,6 @@ __device__ __forceinline__ void write_result(const Trav &s, const DevScene &sc, 
 // split axis when it is interior) instead of its Node64 records.
 template <bool kExtra, bool kWin>
 struct RayQuery {
-   struct Ctx {};
-   static constexpr bool kStaged = true;
    static constexpr bool kWindows = kWin;
    DevScene sc;
    const float *rays;
@@ -67,21 +65,15 @@ struct RayQuery {
 #pragma unroll
       for (int k = 0; k < 6; k++) f.q[k] = rp[k];
    }
-   __device__ __forceinline__ int start(uint32_t, const Fetched &f, Ctx &, Trav &s) const {
+   __device__ __forceinline__ void start(const Fetched &f, Trav &s) const {
       make_ray(s.r, f.q[0], f.q[1], f.q[2], f.q[3], f.q[4], f.q[5]);
-      return 0;
    }
-   __device__ __forceinline__ void load2(Ctx &, Fetched &) const {}
-   __device__ __forceinline__ void start2(Ctx &, const Fetched &, Trav &) const {}
-   __device__ __forceinline__ void begin_root(Ctx &, Trav &s) const {
-      begin(s, sc.root_box, sc.root_ref, sc.root_count);
-   }
+   __device__ __forceinline__ void begin_root(Trav &s) const { begin(s, sc.root_box, sc.root_ref, sc.root_count); }
    __device__ __forceinline__ uint32_t root_count() const { return root_cnt; }
-   __device__ __forceinline__ const Node64 *nodes(const Ctx &) const { return sc.nodes; }
+   __device__ __forceinline__ const Node64 *nodes() const { return sc.nodes; }
    __device__ __forceinline__ const Node64 *windows() const { return win; }
-   __device__ __forceinline__ const float *tris(const Ctx &) const { return sc.tris; }
-   __device__ __forceinline__ bool debug_pixel(const Ctx &) const { return false; }
-   __device__ __forceinline__ void finish(uint32_t id, const Ctx &, const Trav &s) const {
+   __device__ __forceinline__ const float *tris() const { return sc.tris; }
+   __device__ __forceinline__ void finish(uint32_t id, const Trav &s) const {
       write_result<kExtra>(s, sc, id, hits, counters, frames);
    }
 };
@@ -93,11 +85,11 @@ struct RayQuery {
 // and keep four waves rather than spill.
 template <int kLds, bool kExtra, bool kWin>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kExtra || kWin ? 4 : 5, 8)))
-k_closest_hit(DevScene sc, const float *__restrict__ rays, uint32_t n, ptx_hit *__restrict__ hits,
+k_closest_hit(DevScene sc, const float *__restrict__ rays, Deal deal, ptx_hit *__restrict__ hits,
               ptx_ray_counters *counters, ptx_hit_frame *frames, uint32_t *work, uint4 *spill, uint32_t refill_min,
               uint32_t leaf_min, const Node64 *win, uint32_t root_cnt) {
    const RayQuery<kExtra, kWin> q{sc, rays, hits, counters, frames, win, root_cnt};
-   persistent_trace<kLds>(q, n, work, spill, refill_min, leaf_min, sc.max_stack);
+   query_trace<kLds>(q, deal, work, spill, refill_min, leaf_min, sc.max_stack);
 }
 
 // The four-wide form (hits, and frames when asked for): the reference's
@@ -224,28 +216,28 @@ int noalloc_scratch_address(int ordinal, void **ptr) {
 namespace {
 
 template <int kLds, bool kWin>
-void launch_form(const DevScene &sc, const float *d_rays, uint32_t n, ptx_hit *d_hits, ptx_ray_counters *d_counters,
+void launch_form(const DevScene &sc, const float *d_rays, const Deal &deal, ptx_hit *d_hits, ptx_ray_counters *d_counters,
                  ptx_hit_frame *d_frames, uint32_t *d_work, uint4 *d_spill, uint32_t grid, uint32_t refill_min,
                  uint32_t leaf_min, const Node64 *win, uint32_t root_cnt, hipStream_t stream) {
    if (d_counters || d_frames)
-      hipLaunchKernelGGL((dev::k_closest_hit<kLds, true, kWin>), dim3(grid), dim3(256), 0, stream, sc, d_rays, n,
+      hipLaunchKernelGGL((dev::k_closest_hit<kLds, true, kWin>), dim3(grid), dim3(256), 0, stream, sc, d_rays, deal,
                          d_hits, d_counters, d_frames, d_work, d_spill, refill_min, leaf_min, win, root_cnt);
    else
-      hipLaunchKernelGGL((dev::k_closest_hit<kLds, false, kWin>), dim3(grid), dim3(256), 0, stream, sc, d_rays, n,
+      hipLaunchKernelGGL((dev::k_closest_hit<kLds, false, kWin>), dim3(grid), dim3(256), 0, stream, sc, d_rays, deal,
                          d_hits, d_counters, d_frames, d_work, d_spill, refill_min, leaf_min, win, root_cnt);
 }
 
 template <int kLds>
-void launch_lds(const DevScene &sc, const float *d_rays, uint32_t n, ptx_hit *d_hits, ptx_ray_counters *d_counters,
+void launch_lds(const DevScene &sc, const float *d_rays, const Deal &deal, ptx_hit *d_hits, ptx_ray_counters *d_counters,
                 ptx_hit_frame *d_frames, uint32_t *d_work, uint4 *d_spill, uint32_t grid, uint32_t refill_min,
                 uint32_t leaf_min, const Node64 *win, uint32_t root_axis, hipStream_t stream) {
    if (win) {
       // the root's count slot: its face count when it is a leaf, else its split axis
       const uint32_t root_cnt = (sc.root_ref & kLeafBit) ? sc.root_count : root_axis;
-      launch_form<kLds, true>(sc, d_rays, n, d_hits, d_counters, d_frames, d_work, d_spill, grid, refill_min,
+      launch_form<kLds, true>(sc, d_rays, deal, d_hits, d_counters, d_frames, d_work, d_spill, grid, refill_min,
                               leaf_min, win, root_cnt, stream);
    } else {
-      launch_form<kLds, false>(sc, d_rays, n, d_hits, d_counters, d_frames, d_work, d_spill, grid, refill_min,
+      launch_form<kLds, false>(sc, d_rays, deal, d_hits, d_counters, d_frames, d_work, d_spill, grid, refill_min,
                                leaf_min, nullptr, sc.root_count, stream);
    }
 }
@@ -315,27 +307,27 @@ int closest_hit_wide_blocks_per_cu(uint32_t lds_depth, bool frames) {
    }
 }
 
-int launch_closest_hit(const DevScene &sc, const float *d_rays, uint32_t n, ptx_hit *d_hits,
+int launch_closest_hit(const DevScene &sc, const float *d_rays, const Deal &deal, ptx_hit *d_hits,
                        ptx_ray_counters *d_counters, ptx_hit_frame *d_frames, uint32_t *d_work, uint4 *d_spill,
                        uint32_t grid, uint32_t lds_depth, uint32_t refill_min, uint32_t leaf_min,
                        const Node64 *windows, uint32_t root_axis, hipStream_t stream) {
-   hipLaunchKernelGGL(dev::k_zero_u32, dim3(1), dim3(64), 0, stream, d_work, (uint32_t)dev::kWorkWords);
-   if (n == 0) return 0;
+   if (deal.n == 0) return 0;
+   if (counted(deal)) hipLaunchKernelGGL(dev::k_zero_u32, dim3(1), dim3(64), 0, stream, d_work, (uint32_t)dev::kWorkWords);
    switch (lds_depth) {
       case 8:
-         launch_lds<8>(sc, d_rays, n, d_hits, d_counters, d_frames, d_work, d_spill, grid, refill_min, leaf_min,
+         launch_lds<8>(sc, d_rays, deal, d_hits, d_counters, d_frames, d_work, d_spill, grid, refill_min, leaf_min,
                        windows, root_axis, stream);
          break;
       case 16:
-         launch_lds<16>(sc, d_rays, n, d_hits, d_counters, d_frames, d_work, d_spill, grid, refill_min, leaf_min,
+         launch_lds<16>(sc, d_rays, deal, d_hits, d_counters, d_frames, d_work, d_spill, grid, refill_min, leaf_min,
                         windows, root_axis, stream);
          break;
       case 24:
-         launch_lds<24>(sc, d_rays, n, d_hits, d_counters, d_frames, d_work, d_spill, grid, refill_min, leaf_min,
+         launch_lds<24>(sc, d_rays, deal, d_hits, d_counters, d_frames, d_work, d_spill, grid, refill_min, leaf_min,
                         windows, root_axis, stream);
          break;
       default:
-         launch_lds<12>(sc, d_rays, n, d_hits, d_counters, d_frames, d_work, d_spill, grid, refill_min, leaf_min,
+         launch_lds<12>(sc, d_rays, deal, d_hits, d_counters, d_frames, d_work, d_spill, grid, refill_min, leaf_min,
                         windows, root_axis, stream);
          break;
    }

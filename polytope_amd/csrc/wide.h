@@ -539,14 +539,15 @@ __device__ __forceinline__ void wide_trace(const Policy &P, const Deal &deal, ui
    typename Policy::Words gw{};
    uint32_t base = 0, left = 0, off = 0;
    while (true) {
-      // lanes whose ray has ended write its result and take a new one
-      if (id != kNone && s.cur == kNone) {
-         P.finish(id, words, s);
-         id = kNone;
-      }
-      uint64_t idle = __builtin_amdgcn_ballot_w64(id == kNone);
-      if ((uint32_t)__popcll(idle) >= refill_min && !(src.done && left == 0)) {
-         while (idle) {
+      // lanes without a ray to step: write what has ended and take new rays,
+      // when enough wait or, at the end, when all have ended
+      uint64_t idle = __builtin_amdgcn_ballot_w64(s.cur == kNone);
+      if ((uint32_t)__popcll(idle) >= (src.done && left == 0 ? 64u : refill_min)) {
+         if (id != kNone && s.cur == kNone) {
+            P.finish(id, words, s);
+            id = kNone;
+         }
+         while (idle && !(src.done && left == 0)) {
             if (left == 0) {
                src.refill(work, lane);
                if (src.done) break;
@@ -591,12 +592,11 @@ __device__ __forceinline__ void wide_trace(const Policy &P, const Deal &deal, ui
             off += take;
             left -= take;
          }
-         idle = __builtin_amdgcn_ballot_w64(id == kNone);
+         if (!__builtin_amdgcn_ballot_w64(id != kNone) && src.done && left == 0) break;
+         idle = __builtin_amdgcn_ballot_w64(s.cur == kNone);
       }
-      if (!~idle && src.done && left == 0) break;
       // node steps until enough lanes are at leaves or have ended
       const bool last = src.done && left == 0;
-      const uint32_t idle_max = (uint32_t)__popcll(idle) + refill_min;
       const uint32_t leaf_now = wide_gather(leaf_min, 64u - (uint32_t)__popcll(idle));
       while (true) {
          const bool node = (int)s.cur >= 0;
@@ -604,7 +604,7 @@ __device__ __forceinline__ void wide_trace(const Policy &P, const Deal &deal, ui
          if (node) wide_node_step(s, P.nodes(words), st);
          const uint32_t ended = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(s.cur == kNone));
          const uint32_t held = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64((int)s.cur < 0)) - ended;
-         if (held >= leaf_now || (!last && ended >= idle_max)) break;
+         if (held >= leaf_now || (!last && ended >= refill_min)) break;
       }
       const bool leaf = (int)s.cur < 0 && s.cur != kNone;
       const uint32_t held = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(leaf));

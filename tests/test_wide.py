@@ -235,3 +235,45 @@ def test_scenes_at_the_edges_of_the_wide_ranges_agree(scale):
     finally:
         scene.close()
         dev.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 64, 65, 20_011])
+def test_counters_do_not_depend_on_the_gathering(n):
+    """Hits, counters and frames of the binary form with every lane, one lane
+    and the defaults gathered at leaves and at refills, over node and window
+    records: the same words, and the hits of the four-wide form."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from polytope_amd import Device, Scene, _abi
+    verts, faces = _scene("sphere")
+    meshes = [S.MeshData(verts, faces)]
+    lo, hi = S.scene_bounds(meshes)
+    rays = _edge_rays(S.rays_incoherent(np.asarray(lo) - 0.2, np.asarray(hi) + 0.2, n, 9), verts)
+    dev = Device(0)
+    scene = Scene(dev, meshes)
+    r = torch.from_numpy(rays).cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def query(counters: bool):
+        h = torch.full((n, 6), -7, dtype=torch.int32, device="cuda")
+        c = torch.full((n, 3), -7, dtype=torch.int32, device="cuda")
+        f = torch.full((n, 15), -7, dtype=torch.int32, device="cuda")
+        scene.intersect_device(r.data_ptr(), n, h.data_ptr(), c.data_ptr() if counters else 0, f.data_ptr(), stream)
+        torch.cuda.synchronize()
+        return [x.cpu().numpy() for x in (h, c, f)]
+
+    try:
+        first = query(True)
+        for windows in (_abi.WINDOWS_OFF, _abi.WINDOWS_ON):
+            for lanes in (1, 64):
+                dev.set_tuning(leaf_lanes=lanes, refill_lanes=lanes, ray_windows=windows, blocks_per_cu=1)
+                for a, b in zip(query(True), first):
+                    assert np.array_equal(a, b)
+        dev.set_tuning(leaf_lanes=64, refill_lanes=64)
+        wide = query(False)
+        assert np.array_equal(wide[0], first[0]) and np.array_equal(wide[2], first[2])
+    finally:
+        scene.close()
+        dev.close()
