@@ -145,7 +145,7 @@ namespace {
 
 // Queries for hits or frames take the four-wide form; the counters count
 // binary boxes, and ray_windows = ON asks for the window records.
-bool wide_query(const ptx_scene *s, const ptx_tuning &t, const ptx_ray_counters *counters) {
+bool wide_query(const ptx_scene *s, const ptx_tuning &t, bool counters) {
    return s->w.faces && !counters && t.ray_windows != PTX_WINDOWS_ON;
 }
 
@@ -165,42 +165,56 @@ uint32_t wide_refill_lanes_of(const ptx_tuning &t) {
 
 }  // namespace
 
+QueryLaunch::QueryLaunch(ptx_scene *s, uint32_t n, bool counters, bool frames, const ptx_tuning &t)
+    : scene(s), tun(t), lds(lds_depth_of(t)), wide(wide_query(s, t, counters)) {
+   ptx_device *dev = s->dev;
+   Deal deal;
+   if (wide) {
+      full = wide_query_grid(dev, t, lds, frames);
+      bytes = 256 + wide_spill_bytes(s, deal_ids(full, (uint32_t)dev->num_cus, n, deal), lds);
+   } else {
+      win = n ? scene_windows(s, t) : nullptr;
+      full = closest_hit_grid(dev, t, lds, counters || frames, win != nullptr);
+      bytes = closest_hit_scratch_bytes(s, deal_ids(full, (uint32_t)dev->num_cus, n, deal), lds);
+   }
+}
+
+int QueryLaunch::take_scratch(hipStream_t stream) {
+   PTX_HIP_TRY(pool_malloc(scene->dev, &scratch, bytes, stream));
+   return PTX_OK;
+}
+
+int QueryLaunch::give_scratch(hipStream_t stream) {
+   const hipError_t e = hipFreeAsync(scratch, stream);
+   scratch = nullptr;
+   if (e != hipSuccess) return set_error(PTX_ERR_HIP, std::string("hipFreeAsync: ") + hipGetErrorString(e));
+   return PTX_OK;
+}
+
+int QueryLaunch::launch(const float *d_rays, uint32_t n, ptx_hit *d_hits, ptx_ray_counters *d_counters,
+                        ptx_hit_frame *d_frames, hipStream_t stream) {
+   ptx_scene *s = scene;
+   Deal deal;
+   const uint32_t grid = deal_ids(full, (uint32_t)s->dev->num_cus, n, deal);
+   uint32_t *work = static_cast<uint32_t *>(scratch);
+   char *spill = static_cast<char *>(scratch) + 256;
+   const int rc =
+         wide ? launch_closest_hit_wide(s->d, s->w, d_rays, deal, d_hits, d_frames, work, spill, grid, lds,
+                                        wide_refill_lanes_of(tun), leaf_lanes_of(tun), stream)
+              : launch_closest_hit(s->d, d_rays, deal, d_hits, d_counters, d_frames, work,
+                                   reinterpret_cast<uint4 *>(spill), grid, lds, refill_lanes_of(tun),
+                                   leaf_lanes_of(tun), win, s->root_axis, stream);
+   return rc ? set_error(PTX_ERR_HIP, "closest-hit launch failed") : PTX_OK;
+}
+
 // Closest-hit launch with stack-spill scratch taken from the stream-ordered allocator.
 int run_closest_hit(ptx_scene *s, const float *d_rays, uint32_t n, ptx_hit *d_hits, ptx_ray_counters *d_counters,
                     ptx_hit_frame *d_frames, hipStream_t stream, const ptx_tuning &t) {
-   ptx_device *dev = s->dev;
-   const uint32_t lds = lds_depth_of(t);
-   if (wide_query(s, t, d_counters)) {
-      Deal deal;
-      const uint32_t grid =
-            deal_ids(wide_query_grid(dev, t, lds, d_frames != nullptr), (uint32_t)dev->num_cus, n, deal);
-      void *scratch = nullptr;
-      PTX_HIP_TRY(pool_malloc(dev, &scratch, 256 + wide_spill_bytes(s, grid, lds), stream));
-      const int rc = launch_closest_hit_wide(s->d, s->w, d_rays, deal, d_hits, d_frames, static_cast<uint32_t *>(scratch),
-                                             static_cast<char *>(scratch) + 256, grid, lds, wide_refill_lanes_of(t),
-                                             leaf_lanes_of(t), stream);
-      const hipError_t fe = hipFreeAsync(scratch, stream);
-      if (rc != 0) return set_error(PTX_ERR_HIP, "closest-hit launch failed");
-      if (fe != hipSuccess) return set_error(PTX_ERR_HIP, std::string("hipFreeAsync: ") + hipGetErrorString(fe));
-      return PTX_OK;
-   }
-   const Node64 *win = n ? scene_windows(s, t) : nullptr;
-   Deal deal;
-   const uint32_t grid =
-         deal_ids(closest_hit_grid(dev, t, lds, d_counters != nullptr || d_frames != nullptr, win != nullptr),
-                  (uint32_t)dev->num_cus, n, deal);
-   void *scratch = nullptr;
-   PTX_HIP_TRY(pool_malloc(dev, &scratch, closest_hit_scratch_bytes(s, grid, lds), stream));
-   uint32_t *work = static_cast<uint32_t *>(scratch);
-   uint4 *spill = reinterpret_cast<uint4 *>(static_cast<char *>(scratch) + 256);
-   const uint32_t refill = refill_lanes_of(t);
-   const uint32_t leaf = leaf_lanes_of(t);
-   const int rc = launch_closest_hit(s->d, d_rays, deal, d_hits, d_counters, d_frames, work, spill, grid, lds, refill, leaf,
-                                     win, s->root_axis, stream);
-   const hipError_t fe = hipFreeAsync(scratch, stream);
-   if (rc != 0) return set_error(PTX_ERR_HIP, "closest-hit launch failed");
-   if (fe != hipSuccess) return set_error(PTX_ERR_HIP, std::string("hipFreeAsync: ") + hipGetErrorString(fe));
-   return PTX_OK;
+   QueryLaunch q(s, n, d_counters != nullptr, d_frames != nullptr, t);
+   if (int rc = q.take_scratch(stream)) return rc;
+   const int rc = q.launch(d_rays, n, d_hits, d_counters, d_frames, stream);
+   const int free_rc = q.give_scratch(stream);
+   return rc ? rc : free_rc;
 }
 
 }  // namespace ptx
@@ -544,7 +558,7 @@ int ptx_intersect_closest_device_noalloc(ptx_scene *scene, const float *d_rays, 
    uint32_t *work = static_cast<uint32_t *>(dev->noalloc_scratch);
    uint4 *spill = reinterpret_cast<uint4 *>(static_cast<char *>(dev->noalloc_scratch) + 256);
    // the four-wide form wherever its spill takes no fewer blocks
-   if (wide_query(scene, t, d_counters)) {
+   if (wide_query(scene, t, d_counters != nullptr)) {
       uint32_t wgrid = wide_query_grid(dev, t, lds, d_frames != nullptr);
       const size_t block = wide_spill_bytes(scene, 1, lds);
       if (block) wgrid = (uint32_t)std::min<size_t>(wgrid, (kNoAllocScratchBytes - 256) / block);

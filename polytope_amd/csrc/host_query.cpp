@@ -29,6 +29,12 @@ HostQueryStaging::~HostQueryStaging() {
    (void)hipSetDevice(ordinal);
    for (hipEvent_t &e : events)
       if (e) (void)hipEventDestroy(e);
+   for (uint32_t i = 0; i < kMaxParts; i++) {
+      if (sent[i]) (void)hipEventDestroy(sent[i]);
+      if (done[i]) (void)hipEventDestroy(done[i]);
+   }
+   if (up) (void)hipStreamDestroy(up);
+   if (down) (void)hipStreamDestroy(down);
    if (pinned) (void)hipHostFree(pinned);
    if (d_buf) (void)hipFree(d_buf);
 }
@@ -36,6 +42,12 @@ HostQueryStaging::~HostQueryStaging() {
 namespace {
 
 constexpr size_t kSlot = HostQueryStaging::kSlotBytes;
+// Rays of a part, at least, and parts a worker sends before the first comes
+// back.  2^20 + 17 rays on 327,680 faces: 1.84 ms in one part, 1.49 in four of
+// 2^18 (one or three ahead: 1.72 and 1.51), 2.00 in eight of 2^17, whose copies
+// and launches cost more than the overlap gives; the link needs 0.88 both ways.
+constexpr uint32_t kPartRays = 1u << 18;
+constexpr uint32_t kAhead = 2;
 
 // Host threads for one call: half the cores this process may run on, at most
 // kMaxWorkers (four threads copy pageable to pinned memory at 60-75 GB/s,
@@ -66,25 +78,36 @@ std::vector<Piece> share(const std::vector<Span> &spans, uint32_t w, uint32_t wo
    return out;
 }
 
-// State one call's workers share.  Phase 0: host spans to the device; the
-// calling thread runs `between` (the launch) once every worker has queued
-// its copies; phase 1: device spans back to the host; -1: a step failed, the
-// rest is skipped.
+// The host spans that go up before a part's launch and the device spans that
+// come back after it.
+struct Part {
+   std::vector<Span> in, out;
+};
+
+// State one call's workers share.  The calling thread launches a part
+// (`between`) once every worker has queued its copies; a worker queues a part's
+// copies up, then copies the part before it back.  A failed step ends the call:
+// the rest is skipped.  A call of one part copies on the launch's stream, a
+// call of several on the staging's own, one for each direction.
 struct HostCall {
    HostQueryStaging *st;
    hipStream_t stream;
    int ordinal;
    uint32_t workers = 1;
-   std::vector<Span> in, out;
+   std::vector<Part> parts;
    std::mutex mu;
    std::condition_variable cv;
-   uint32_t arrived = 0;
-   int phase = 0;
+   uint32_t arrived[HostQueryStaging::kMaxParts] = {};
+   uint32_t launched = 0;             // parts whose hits may be waited for
+   bool stop = false;
    std::string error;
 
+   bool several() const { return parts.size() > 1; }
    void fail(const std::string &m) {
       std::lock_guard<std::mutex> lock(mu);
       if (error.empty()) error = m;
+      stop = true;
+      cv.notify_all();
    }
    bool ok(hipError_t e, const char *what) {
       if (e == hipSuccess) return true;
@@ -92,66 +115,98 @@ struct HostCall {
       fail(std::string(what) + ": " + hipGetErrorString(e));
       return false;
    }
-   char *slot(uint32_t w, uint32_t k) const { return st->pinned + (2 * size_t(w) + (k & 1)) * kSlot; }
-   hipEvent_t event(uint32_t w, uint32_t k) const { return st->events[2 * w + (k & 1)]; }
+   // slot and event k of a worker's two in one direction
+   char *slot(uint32_t w, uint32_t back, uint32_t k) const {
+      return st->pinned + (4 * size_t(w) + 2 * back + (k & 1)) * kSlot;
+   }
+   hipEvent_t event(uint32_t w, uint32_t back, uint32_t k) const { return st->events[4 * w + 2 * back + (k & 1)]; }
 
-   // Worker w's share going up: copy a piece into a slot, then queue its DMA;
-   // a slot is refilled once the DMA that read it has finished.
-   bool send(uint32_t w) {
-      const std::vector<Piece> ps = share(in, w, workers);
-      for (uint32_t k = 0; k < ps.size(); k++) {
-         if (k >= 2 && !ok(hipEventSynchronize(event(w, k)), "hipEventSynchronize")) return false;
-         std::memcpy(slot(w, k), ps[k].host, ps[k].len);
-         if (!ok(hipMemcpyAsync(ps[k].dev, slot(w, k), ps[k].len, hipMemcpyHostToDevice, stream), "hipMemcpyAsync"))
-            return false;
-         if (!ok(hipEventRecord(event(w, k), stream), "hipEventRecord")) return false;
+   // Worker w's share of a part going up: copy a piece into a slot, then queue
+   // its DMA; a slot is refilled once the DMA that read it has finished.  used:
+   // pieces this worker has sent in the call.
+   bool send(uint32_t w, const Part &part, uint32_t &used) {
+      const hipStream_t s = several() ? st->up : stream;
+      for (const Piece &p : share(part.in, w, workers)) {
+         const uint32_t k = used++;
+         if (k >= 2 && !ok(hipEventSynchronize(event(w, 0, k)), "hipEventSynchronize")) return false;
+         std::memcpy(slot(w, 0, k), p.host, p.len);
+         if (!ok(hipMemcpyAsync(p.dev, slot(w, 0, k), p.len, hipMemcpyHostToDevice, s), "hipMemcpyAsync")) return false;
+         if (!ok(hipEventRecord(event(w, 0, k), s), "hipEventRecord")) return false;
       }
       return true;
    }
 
-   // Worker w's share coming back: the DMA of piece k + 1 is queued before
-   // piece k is copied out of its slot.
-   bool receive(uint32_t w) {
-      const std::vector<Piece> ps = share(out, w, workers);
-      auto queue = [&](uint32_t k) {
-         return ok(hipMemcpyAsync(slot(w, k), ps[k].dev, ps[k].len, hipMemcpyDeviceToHost, stream), "hipMemcpyAsync") &&
-                ok(hipEventRecord(event(w, k), stream), "hipEventRecord");
-      };
+   // Worker w's share of a part coming back: the DMA of piece k + 1 is queued
+   // before piece k is copied out of its slot.
+   bool receive(uint32_t w, uint32_t c) {
+      const std::vector<Piece> ps = share(parts[c].out, w, workers);
       if (ps.empty()) return true;
+      hipStream_t s = stream;
+      if (several()) {
+         s = st->down;
+         if (!ok(hipEventSynchronize(st->done[c]), "hipEventSynchronize")) return false;
+      }
+      auto queue = [&](uint32_t k) {
+         return ok(hipMemcpyAsync(slot(w, 1, k), ps[k].dev, ps[k].len, hipMemcpyDeviceToHost, s), "hipMemcpyAsync") &&
+                ok(hipEventRecord(event(w, 1, k), s), "hipEventRecord");
+      };
       if (!queue(0)) return false;
       for (uint32_t k = 0; k < ps.size(); k++) {
          if (k + 1 < ps.size() && !queue(k + 1)) return false;
-         if (!ok(hipEventSynchronize(event(w, k)), "hipEventSynchronize")) return false;
-         std::memcpy(ps[k].host, slot(w, k), ps[k].len);
+         if (!ok(hipEventSynchronize(event(w, 1, k)), "hipEventSynchronize")) return false;
+         std::memcpy(ps[k].host, slot(w, 1, k), ps[k].len);
       }
       return true;
    }
 
    void worker(uint32_t w) {
-      bool good = ok(hipSetDevice(ordinal), "hipSetDevice") && send(w);
-      std::unique_lock<std::mutex> lock(mu);
-      if (!good && error.empty()) error = "host copy failed";
-      arrived++;
-      cv.notify_all();
-      cv.wait(lock, [&] { return phase != 0; });
-      if (phase < 0) return;
-      lock.unlock();
-      receive(w);
+      if (!ok(hipSetDevice(ordinal), "hipSetDevice")) return;
+      uint32_t used = 0;
+      // up to kAhead parts go up before the first comes back
+      for (uint32_t c = 0; c < parts.size() + kAhead; c++) {
+         if (c < parts.size()) {
+            if (!send(w, parts[c], used)) return;
+            std::lock_guard<std::mutex> lock(mu);
+            arrived[c]++;
+            cv.notify_all();
+         }
+         if (c < kAhead) continue;
+         {
+            std::unique_lock<std::mutex> lock(mu);
+            cv.wait(lock, [&] { return stop || launched > c - kAhead; });
+            if (stop) return;
+         }
+         if (!receive(w, c - kAhead)) return;
+      }
+   }
+
+   // Launches part c behind its rays.
+   template <class F>
+   int launch(uint32_t c, F &between) {
+      if (!several()) return between(c);
+      if (!ok(hipEventRecord(st->sent[c], st->up), "hipEventRecord") ||
+          !ok(hipStreamWaitEvent(stream, st->sent[c], 0), "hipStreamWaitEvent"))
+         return PTX_ERR_HIP;
+      if (const int rc = between(c)) return rc;
+      return ok(hipEventRecord(st->done[c], stream), "hipEventRecord") ? PTX_OK : PTX_ERR_HIP;
    }
 
    // The whole call on the calling thread and up to `workers` threads.
    template <class F>
    int run(F between) {
       size_t in_bytes = 0, out_bytes = 0;
-      for (const Span &a : in) in_bytes += a.bytes;
-      for (const Span &a : out) out_bytes += a.bytes;
+      for (const Part &p : parts) {
+         for (const Span &a : p.in) in_bytes += a.bytes;
+         for (const Span &a : p.out) out_bytes += a.bytes;
+      }
       const size_t pieces = (std::max(in_bytes, out_bytes) + kSlot - 1) / kSlot;
       workers = uint32_t(std::min<size_t>(host_workers(), std::max<size_t>(1, pieces)));
       int rc = PTX_OK;
       if (workers == 1) {
-         if (send(0)) {
-            rc = between();
-            if (rc == PTX_OK) receive(0);
+         uint32_t used = 0;
+         for (uint32_t c = 0; c < parts.size() + kAhead && rc == PTX_OK && !stop; c++) {
+            if (c < parts.size() && send(0, parts[c], used)) rc = launch(c, between);
+            if (c >= kAhead && rc == PTX_OK && !stop) receive(0, c - kAhead);
          }
       } else {
          std::vector<std::thread> ts;
@@ -161,24 +216,27 @@ struct HostCall {
          } catch (const std::exception &) {
             fail("could not start the host copy threads");
          }
-         std::unique_lock<std::mutex> lock(mu);
-         // threads that did not start never arrive: count them as arrived
-         arrived += workers - uint32_t(ts.size());
-         cv.wait(lock, [&] { return arrived == workers; });
-         if (error.empty()) {
-            lock.unlock();
-            rc = between();
-            lock.lock();
+         for (uint32_t c = 0; c < parts.size(); c++) {
+            {
+               std::unique_lock<std::mutex> lock(mu);
+               cv.wait(lock, [&] { return stop || arrived[c] == workers; });
+               if (stop) break;
+            }
+            rc = launch(c, between);
+            std::lock_guard<std::mutex> lock(mu);
+            if (rc == PTX_OK) launched = c + 1;
+            else stop = true;
+            cv.notify_all();
+            if (stop) break;
          }
-         phase = (rc == PTX_OK && error.empty()) ? 1 : -1;
-         cv.notify_all();
-         lock.unlock();
          for (std::thread &th : ts) th.join();
       }
       // every queued copy has finished before the slots serve another call
-      const hipError_t se = hipStreamSynchronize(stream);
-      if (rc != PTX_OK) return rc;
+      hipError_t se = several() ? hipStreamSynchronize(st->up) : hipSuccess;
+      const hipError_t ss = hipStreamSynchronize(stream), sd = several() ? hipStreamSynchronize(st->down) : hipSuccess;
+      if (se == hipSuccess) se = ss != hipSuccess ? ss : sd;
       if (!error.empty()) return set_error(PTX_ERR_HIP, error);
+      if (rc != PTX_OK) return rc;
       if (se != hipSuccess) {
          (void)hipGetLastError();
          return set_error(PTX_ERR_HIP, std::string("hipStreamSynchronize: ") + hipGetErrorString(se));
@@ -196,10 +254,15 @@ int ensure_staging(ptx_device *dev, size_t need) {
    if (!st.ready) {
       // what an earlier failed call made is kept and not made again
       if (!st.pinned)
-         PTX_HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&st.pinned), 2 * HostQueryStaging::kMaxWorkers * kSlot,
+         PTX_HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&st.pinned), 4 * HostQueryStaging::kMaxWorkers * kSlot,
                                    hipHostMallocDefault));
       for (hipEvent_t &e : st.events)
          if (!e) PTX_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+      for (uint32_t i = 0; i < HostQueryStaging::kMaxParts; i++)
+         for (hipEvent_t *e : {&st.sent[i], &st.done[i]})
+            if (!*e) PTX_HIP_TRY(hipEventCreateWithFlags(e, hipEventDisableTiming));
+      for (hipStream_t *s : {&st.up, &st.down})
+         if (!*s) PTX_HIP_TRY(hipStreamCreateWithFlags(s, hipStreamNonBlocking));
       st.ready = true;
    }
    if (need > st.d_cap) {
@@ -227,15 +290,34 @@ int intersect_host(ptx_scene *s, const float *rays, uint32_t n, ptx_hit *hits, p
    call.stream = dev->stream;
    call.ordinal = dev->ordinal;
    char *d_hits = st.d_buf + b_rays, *d_cnt = counters ? d_hits + b_hits : nullptr;
-   call.in.push_back(Span{reinterpret_cast<char *>(const_cast<float *>(rays)), st.d_buf, size_t(n) * 24});
-   call.out.push_back(Span{reinterpret_cast<char *>(hits), d_hits, size_t(n) * sizeof(ptx_hit)});
-   if (counters)
-      call.out.push_back(Span{reinterpret_cast<char *>(counters), d_cnt, size_t(n) * sizeof(ptx_ray_counters)});
+   const uint32_t np = std::clamp<uint32_t>(n / kPartRays, 1u, HostQueryStaging::kMaxParts);
+   // parts of whole batches, the last one taking the rest
+   const uint32_t each = n / np & ~63u;
+   auto first = [&](uint32_t c) { return size_t(c) * each; };
+   auto count = [&](uint32_t c) { return c + 1 < np ? each : n - (np - 1) * each; };
+   for (uint32_t c = 0; c < np; c++) {
+      const size_t f = first(c), m = count(c);
+      Part p;
+      p.in.push_back(Span{reinterpret_cast<char *>(const_cast<float *>(rays + 6 * f)), st.d_buf + f * 24, m * 24});
+      p.out.push_back(Span{reinterpret_cast<char *>(hits + f), d_hits + f * sizeof(ptx_hit), m * sizeof(ptx_hit)});
+      if (counters)
+         p.out.push_back(Span{reinterpret_cast<char *>(counters + f), d_cnt + f * sizeof(ptx_ray_counters),
+                              m * sizeof(ptx_ray_counters)});
+      call.parts.push_back(std::move(p));
+   }
+   // one scratch for all parts, which run one after another: given back between
+   // them it made the next launch wait for the one before
    const ptx_tuning t = tuning_of(dev);
-   return call.run([&] {
-      return run_closest_hit(s, reinterpret_cast<const float *>(st.d_buf), n, reinterpret_cast<ptx_hit *>(d_hits),
-                             reinterpret_cast<ptx_ray_counters *>(d_cnt), nullptr, call.stream, t);
+   QueryLaunch q(s, n, d_cnt != nullptr, false, t);
+   if (int rc = q.take_scratch(call.stream)) return rc;
+   const int rc = call.run([&](uint32_t c) {
+      const size_t f = first(c);
+      return q.launch(reinterpret_cast<const float *>(st.d_buf + f * 24), count(c),
+                      reinterpret_cast<ptx_hit *>(d_hits) + f,
+                      d_cnt ? reinterpret_cast<ptx_ray_counters *>(d_cnt) + f : nullptr, nullptr, call.stream);
    });
+   const int free_rc = q.give_scratch(call.stream);
+   return rc ? rc : free_rc;
 }
 
 int download_host(ptx_device *dev, hipStream_t stream, const std::vector<Span> &spans) {
@@ -244,8 +326,8 @@ int download_host(ptx_device *dev, hipStream_t stream, const std::vector<Span> &
    call.st = dev->host_query.get();
    call.stream = stream;
    call.ordinal = dev->ordinal;
-   call.out = spans;
-   return call.run([] { return int(PTX_OK); });
+   call.parts.push_back(Part{{}, spans});
+   return call.run([](uint32_t) { return int(PTX_OK); });
 }
 
 }  // namespace ptx

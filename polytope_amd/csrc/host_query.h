@@ -22,12 +22,15 @@ namespace ptx {
 struct HostQueryStaging {
    static constexpr size_t kSlotBytes = size_t(2) << 20;  // one pinned chunk
    static constexpr uint32_t kMaxWorkers = 4;             // host threads of one call
+   static constexpr uint32_t kMaxParts = 4;               // parts of one query in flight
    int ordinal = 0;
    char *d_buf = nullptr;
    size_t d_cap = 0;
-   char *pinned = nullptr;                  // kMaxWorkers x 2 slots of kSlotBytes
-   hipEvent_t events[2 * kMaxWorkers] = {};  // one per slot: its last copy
-   bool ready = false;                      // pinned slots and events exist
+   char *pinned = nullptr;                  // per worker two slots going up, two coming back
+   hipEvent_t events[4 * kMaxWorkers] = {};  // one per slot: its last copy
+   hipEvent_t sent[kMaxParts] = {}, done[kMaxParts] = {};   // a part's rays are up, its hits written
+   hipStream_t up = nullptr, down = nullptr;  // the copies of a query in parts
+   bool ready = false;                      // pinned slots, events and streams exist
    ~HostQueryStaging();
 };
 

@@ -119,6 +119,24 @@ const Node64 *scene_windows(ptx_scene *s, const ptx_tuning &t);
 // The window records if already built (never allocates), else null.
 const Node64 *built_windows(ptx_scene *s, const ptx_tuning &t);
 size_t closest_hit_scratch_bytes(const ptx_scene *s, uint32_t grid, uint32_t lds);
+// The form, grid and scratch of closest-hit launches of at most n rays each,
+// which run one after another on one stream between take_scratch and
+// give_scratch.
+struct QueryLaunch {
+   ptx_scene *scene;
+   ptx_tuning tun;
+   uint32_t lds;
+   bool wide;
+   const Node64 *win = nullptr;
+   uint32_t full = 0;                 // blocks that fit the device
+   size_t bytes = 0;
+   void *scratch = nullptr;
+   QueryLaunch(ptx_scene *s, uint32_t n, bool counters, bool frames, const ptx_tuning &t);
+   int take_scratch(hipStream_t stream);
+   int give_scratch(hipStream_t stream);
+   int launch(const float *d_rays, uint32_t n, ptx_hit *d_hits, ptx_ray_counters *d_counters, ptx_hit_frame *d_frames,
+              hipStream_t stream);
+};
 int run_closest_hit(ptx_scene *s, const float *d_rays, uint32_t n, ptx_hit *d_hits, ptx_ray_counters *d_counters,
                     ptx_hit_frame *d_frames, hipStream_t stream, const ptx_tuning &t);
 void device_retain(ptx_device *dev);

@@ -277,3 +277,34 @@ def test_counters_do_not_depend_on_the_gathering(n):
     finally:
         scene.close()
         dev.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [(1 << 18) - 1, (1 << 19) - 1, (1 << 19) + 33, 5 * (1 << 18) + 1])
+def test_host_queries_in_parts_agree(n):
+    """Host queries of one part, two and four (sizes around where they split),
+    with and without counters: the words of the device query."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from polytope_amd import Device, Scene
+    verts, faces = _scene("sphere")
+    meshes = [S.MeshData(verts, faces)]
+    lo, hi = S.scene_bounds(meshes)
+    rays = S.rays_incoherent(np.asarray(lo) - 0.2, np.asarray(hi) + 0.2, n, 9)
+    dev = Device(0)
+    scene = Scene(dev, meshes)
+    r = torch.from_numpy(rays).cuda()
+    h = torch.full((n, 6), -7, dtype=torch.int32, device="cuda")
+    c = torch.zeros((n, 3), dtype=torch.int32, device="cuda")
+    try:
+        scene.intersect_device(r.data_ptr(), n, h.data_ptr(), c.data_ptr(), 0, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        for _ in range(2):
+            hits, cnt = scene.intersect(rays, counters=True)
+            assert np.array_equal(hits.view(np.int32).reshape(n, 6), h.cpu().numpy())
+            assert np.array_equal(cnt.view(np.int32).reshape(n, 3), c.cpu().numpy())
+            assert np.array_equal(scene.intersect(rays).view(np.int32).reshape(n, 6), h.cpu().numpy())
+    finally:
+        scene.close()
+        dev.close()
