@@ -78,11 +78,11 @@ struct RayQuery {
    }
 };
 
-// The hits-only node-record form is held to at most 96 VGPRs, five waves per
-// SIMD (with a 12- or 8-entry LDS stack five blocks fit a CU's LDS too): four
-// blocks per CU ran 2,154 against 2,307-2,326 Mrays/s with five on 2^21
-// incoherent rays.  The counters/frames and window forms need more registers
-// and keep four waves rather than spill.
+// The hits-only node-record form (scenes without a four-wide form) is held to
+// five waves per SIMD (with a 12- or 8-entry LDS stack five blocks fit a CU's
+// LDS too): four ran 2,154 against 2,307-2,326 Mrays/s with five on 2^21
+// incoherent rays.  The counters/frames and window forms keep four, which is
+// the better number on small launches (query_trace).
 template <int kLds, bool kExtra, bool kWin>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kExtra || kWin ? 4 : 5, 8)))
 k_closest_hit(DevScene sc, const float *__restrict__ rays, Deal deal, ptx_hit *__restrict__ hits,
