@@ -398,38 +398,6 @@ int ptx_scene_create(ptx_device *dev, const ptx_scene_desc *desc, ptx_scene **ou
    if ((rc = upload(s.get(), img.tris, &s->d.tris)) != PTX_OK) return rc;
    if ((rc = upload(s.get(), s->bvh.pairs, &s->d.pairs)) != PTX_OK) return rc;
    if ((rc = upload(s.get(), img.meshes, &s->d.meshes)) != PTX_OK) return rc;
-   // the four-wide faces from the triangles and ids just uploaded, while the
-   // host still builds the nodes; a scene whose four-wide form finds no device
-   // memory does without it
-   const size_t kept = s->allocations.size(), face_bytes = size_t(img.num_tris) * sizeof(WideFace);
-   const uint64_t kept_bytes = s->info.device_bytes;
-   void *faces = nullptr;
-   if (face_bytes && hipMalloc(&faces, face_bytes) == hipSuccess) {
-      s->allocations.push_back(faces);
-      s->info.device_bytes += face_bytes;
-      if (launch_build_wide_faces(s->d.tris, s->d.pairs, img.num_tris, static_cast<WideFace *>(faces), nullptr) != 0) {
-         (void)hipGetLastError();
-         return set_error(PTX_ERR_HIP, "four-wide face records");
-      }
-   } else {
-      (void)hipGetLastError();
-      faces = nullptr;
-   }
-   const bool built = (wide_built.valid() ? wide_built.get() : make_wide()) && faces;
-   if (built && upload(s.get(), wide.nodes, &s->w.nodes) == PTX_OK &&
-       upload(s.get(), wide.leaves, &s->w.leaves) == PTX_OK) {
-      s->w.faces = static_cast<const WideFace *>(faces);
-      s->w.root = wide.root;
-      s->w.stack = wide.stack;
-   } else {
-      (void)hipGetLastError();
-      s->w = WideScene{};
-   }
-   if (faces) PTX_HIP_TRY(hipStreamSynchronize(nullptr));
-   if (!s->w.faces) {
-      for (; s->allocations.size() > kept; s->allocations.pop_back()) (void)hipFree(s->allocations.back());
-      s->info.device_bytes = kept_bytes;
-   }
    if (s->has_texture) {
       // one texture record per leaf-ordered triangle, then the texel pool (each
       // texture that a mesh uses, once), in one allocation
@@ -470,6 +438,38 @@ int ptx_scene_create(ptx_device *dev, const ptx_scene_desc *desc, ptx_scene **ou
          std::copy(desc->lights[i].intensity, desc->lights[i].intensity + 3, &lights[6 * i + 3]);
       }
       if ((rc = upload(s.get(), lights, &s->d.lights)) != PTX_OK) return rc;
+   }
+   // the four-wide form last, out of the memory that everything a scene cannot
+   // do without has left: one that finds none is dropped.  Its faces come from
+   // the triangles and ids just uploaded, while the host still builds the nodes
+   const size_t kept = s->allocations.size(), face_bytes = size_t(img.num_tris) * sizeof(WideFace);
+   const uint64_t kept_bytes = s->info.device_bytes;
+   void *faces = nullptr;
+   if (face_bytes && hipMalloc(&faces, face_bytes) == hipSuccess) {
+      s->allocations.push_back(faces);
+      s->info.device_bytes += face_bytes;
+      if (launch_build_wide_faces(s->d.tris, s->d.pairs, img.num_tris, static_cast<WideFace *>(faces), nullptr) != 0) {
+         (void)hipGetLastError();
+         return set_error(PTX_ERR_HIP, "four-wide face records");
+      }
+   } else {
+      (void)hipGetLastError();
+      faces = nullptr;
+   }
+   const bool built = (wide_built.valid() ? wide_built.get() : make_wide()) && faces;
+   if (built && upload(s.get(), wide.nodes, &s->w.nodes) == PTX_OK &&
+       upload(s.get(), wide.leaves, &s->w.leaves) == PTX_OK) {
+      s->w.faces = static_cast<const WideFace *>(faces);
+      s->w.root = wide.root;
+      s->w.stack = wide.stack;
+   } else {
+      (void)hipGetLastError();
+      s->w = WideScene{};
+   }
+   if (faces) PTX_HIP_TRY(hipStreamSynchronize(nullptr));
+   if (!s->w.faces) {
+      for (; s->allocations.size() > kept; s->allocations.pop_back()) (void)hipFree(s->allocations.back());
+      s->info.device_bytes = kept_bytes;
    }
    s->d.num_lights = desc->num_lights;
    std::copy(img.root_box, img.root_box + 6, s->d.root_box);
