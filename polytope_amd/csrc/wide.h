@@ -17,9 +17,11 @@
 //
 // The one case in which boxes do not nest as tests: a direction component of
 // -0 makes the reference's slab selections accept a box that is flat in that
-// axis at the origin's coordinate inside boxes they reject.  Such a ray, and
-// rays with NaN or all-zero directions, are traced again or at once over the
-// binary records in the reference's own steps (exact_trace).
+// axis at the origin's coordinate inside boxes they reject.  Such a ray is
+// traced again over the binary records in the reference's own steps
+// (exact_trace).  Rays with NaN, infinite or all-zero components nest: a NaN
+// slab value leaves the fold as it was in every box, and an infinite one moves
+// with the plane as a finite one does.
 #pragma once
 
 #include "traverse.h"
@@ -60,7 +62,7 @@ namespace dev {
 constexpr uint32_t kRayAxisShift = 3, kRayAxisMask = 3u;
 constexpr uint32_t kRaySlow = 1u << 5;     // child tests with the exact slab
 constexpr uint32_t kRayMinus = 1u << 6;    // some 1 / direction is -inf
-constexpr uint32_t kRayHard = 1u << 7;     // traced over the binary records
+constexpr uint32_t kRayHard = 1u << 7;     // an accepted face's t may be NaN: a component is not finite, or all are 0
 // 16 * the octant's entry of WideNode::later, in bits 8-13
 constexpr uint32_t kRayLaterShift = 8;
 constexpr uint32_t kLaterFlip = 0x7BDEu;   // every pair of different children
@@ -179,7 +181,7 @@ PTX_HD bool wide_child_slow(const WidePlanes &p, int k, const Ray &r, float gx, 
    wide_slow_axis(p.nx, p.fx, k, gx, ex, r.ox, r.ix, near, far);
    wide_slow_axis(p.ny, p.fy, k, gy, ey, r.oy, r.iy, near, far);
    wide_slow_axis(p.nz, p.fz, k, gz, ez, r.oz, r.iz, near, far);
-   return near <= wide_bound(far * kSlabScale) && near <= wide_bound(fminf(kInf, min_t));
+   return near <= wide_bound(far * kSlabScale) && near <= wide_bound(min_t);     // never past a NaN min_t
 }
 
 // Whether a leaf box that passed is flat at the origin's coordinate in an
@@ -453,6 +455,8 @@ __device__ __forceinline__ bool wide_leaf_step(Trav &s, const WideFace *faces, c
          }
       }
    }
+   // no box passes a NaN MinT: what is deferred need not be popped one by one
+   if (done && (s.r.nk & kRayHard) && s.min_t != s.min_t) s.sp = 1;
    return done ? wide_pop(s, st) : true;
 }
 
@@ -466,7 +470,7 @@ __device__ __forceinline__ uint32_t wide_gather(uint32_t most, uint32_t holding)
 }
 
 // The state a traversal starts from: s.r set up and classified, min_t = tmax.
-__device__ __forceinline__ void wide_begin(Trav &s, const float *root_box, uint32_t root, float tmax = kInf) {
+PTX_HD void wide_begin(Trav &s, const float *root_box, uint32_t root, float tmax = kInf) {
    s.min_t = tmax;
    s.hit = 0xFFFFFFFFu;
    s.mesh = s.face = 0xFFFFFFFFu;
@@ -476,7 +480,7 @@ __device__ __forceinline__ void wide_begin(Trav &s, const float *root_box, uint3
    s.hu = s.hv = s.hw = 0.f;
    float near, far;
    slab(root_box[0], root_box[1], root_box[2], root_box[3], root_box[4], root_box[5], s.r, near, far);
-   s.cur = (s.r.nk & kRayHard) ? kWideExact : near <= far && near <= s.min_t ? root : 0xFFFFFFFFu;
+   s.cur = near <= far && near <= s.min_t ? root : 0xFFFFFFFFu;
 }
 
 // One leaf step, or the whole traversal over the binary records for a ray that

@@ -308,3 +308,62 @@ def test_host_queries_in_parts_agree(n):
     finally:
         scene.close()
         dev.close()
+
+
+def test_rays_without_finite_directions_step_over_the_wide_tree(tmp_path):
+    """No ray starts over the binary records: a lane whose direction is zero or
+    NaN traced there alone held its wave for the whole of it."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not Path(hipcc).exists():
+        pytest.skip("hipcc not found")
+    exe = tmp_path / "wide_hard_check"
+    csrc = ROOT / "polytope_amd" / "csrc"
+    subprocess.run([hipcc, "-O2", "-std=c++17", "-ffp-contract=off", "-x", "hip", "--offload-arch=gfx950",
+                    "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                    f"-I{csrc}", f"-I{ROOT / 'include'}", str(ROOT / "tests" / "wide_hard_check.cpp"),
+                    *(str(csrc / f) for f in ("wide_build.cpp", "bvh_build.cpp", "scene.cpp")), "-lpthread",
+                    "-o", str(exe)], check=True, capture_output=True, timeout=300)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stdout
+    assert " 0 mismatches" in out.stdout
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("share", [1, 2, 64])
+def test_idle_lanes_marked_by_their_directions_agree(share):
+    """Every share-th ray without a direction, one in sixteen of those NaN or
+    infinite, as a program marks the idle lanes of a batch: the hits of the
+    binary form."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from polytope_amd import Device, Scene
+    verts, faces = _scene("sphere")
+    meshes = [S.MeshData(verts, faces)]
+    n = 20_011
+    lo, hi = S.scene_bounds(meshes)
+    rays = S.rays_incoherent(lo, hi, n, 9)
+    rays[::share, 3:] = 0.0
+    rays[::2 * share, 3] = -0.0
+    rays[::16 * share, 4] = np.nan
+    rays[7 * share::16 * share, 5] = -np.inf
+    dev = Device(0)
+    scene = Scene(dev, meshes)
+    r = torch.from_numpy(rays).cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+    out = []
+    try:
+        for counters in (True, False):
+            h = torch.full((n, 6), -7, dtype=torch.int32, device="cuda")
+            c = torch.zeros((n, 3), dtype=torch.int32, device="cuda")
+            f = torch.full((n, 15), -7.0, dtype=torch.float32, device="cuda")
+            scene.intersect_device(r.data_ptr(), n, h.data_ptr(), c.data_ptr() if counters else 0, f.data_ptr(), stream)
+            torch.cuda.synchronize()
+            out.append((h.cpu().numpy(), f.cpu().numpy()))
+        (h0, f0), (h1, f1) = out
+        assert np.array_equal(h0[:, :2], h1[:, :2])
+        assert np.array_equal(h0[:, 2:].view(np.float32), h1[:, 2:].view(np.float32), equal_nan=True)
+        assert np.array_equal(f0, f1, equal_nan=True)
+    finally:
+        scene.close()
+        dev.close()
