@@ -35,18 +35,60 @@ double now_s() {
 
 namespace {
 
-template <class T, class A>
-int upload(ptx_scene *s, const std::vector<T, A> &v, const T **dst) {
-   *dst = nullptr;
-   if (v.empty()) return PTX_OK;
-   void *p = nullptr;
-   PTX_HIP_TRY(hipMalloc(&p, v.size() * sizeof(T)));
-   s->allocations.push_back(p);
-   PTX_HIP_TRY(hipMemcpy(p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
-   s->info.device_bytes += v.size() * sizeof(T);
-   *dst = static_cast<const T *>(p);
-   return PTX_OK;
-}
+// Arrays of a scene that go up together, in one allocation (each costs about
+// 7 us, and its free more) and, while they are small, in one copy.
+struct Uploads {
+   static constexpr size_t kOneCopy = 256 << 10;
+   struct Item {
+      const void *src;          // null: only the room
+      size_t bytes;
+      const void **dst;
+   };
+   ptx_scene *scene;
+   std::vector<Item> items;
+   template <class T>
+   void add(const T *src, size_t n, const T **dst) {
+      *dst = nullptr;
+      if (n) items.push_back(Item{src, n * sizeof(T), reinterpret_cast<const void **>(dst)});
+   }
+   template <class T, class A>
+   void add(const std::vector<T, A> &v, const T **dst) {
+      add(v.data(), v.size(), dst);
+   }
+   // Makes them and leaves the list empty.
+   int run() {
+      std::vector<Item> list;
+      list.swap(items);
+      auto place = [](size_t bytes) { return (bytes + 255) & ~size_t(255); };
+      size_t all = 0;
+      bool whole = true;
+      for (const Item &i : list) {
+         all += place(i.bytes);
+         whole = whole && i.src;
+      }
+      if (all == 0) return PTX_OK;
+      char *p = nullptr;
+      PTX_HIP_TRY(hipMalloc(reinterpret_cast<void **>(&p), all));
+      scene->allocations.push_back(p);
+      scene->info.device_bytes += all;
+      const bool one = whole && all <= kOneCopy;
+      std::vector<char> block(one ? all : 0);
+      size_t at = 0;
+      for (const Item &i : list) {
+         if (one) std::memcpy(&block[at], i.src, i.bytes);
+         else if (i.src) PTX_HIP_TRY(hipMemcpy(p + at, i.src, i.bytes, hipMemcpyHostToDevice));
+         *i.dst = p + at;
+         at += place(i.bytes);
+      }
+      if (one) PTX_HIP_TRY(hipMemcpy(p, block.data(), all, hipMemcpyHostToDevice));
+      return PTX_OK;
+   }
+};
+
+// Faces up to which a scene's four-wide form is built by the calling thread and
+// its face records with it: a thread, a kernel and the wait for it take 35 us,
+// the form of 1,280 faces 40.
+constexpr uint32_t kWideBeside = 2048;
 
 }  // namespace
 
@@ -385,19 +427,24 @@ int ptx_scene_create(ptx_device *dev, const ptx_scene_desc *desc, ptx_scene **ou
    auto make_wide = [&] {
       try {
          return build_wide(s->bvh, img, desc->build_threads, wide);
-      } catch (const std::bad_alloc &) {         // no memory for it: the scene does without
+      } catch (const std::exception &) {         // no memory for it: the scene does without
          return false;
       }
    };
    std::future<bool> wide_built;
-   try {
-      wide_built = std::async(std::launch::async, make_wide);
-   } catch (const std::system_error &) {         // no thread to be had: built below by this one
+   if (img.num_tris > kWideBeside) {
+      try {
+         wide_built = std::async(std::launch::async, make_wide);
+      } catch (const std::exception &) {         // no thread to be had: built below by this one
+      }
    }
-   if ((rc = upload(s.get(), img.nodes, &s->d.nodes)) != PTX_OK) return rc;
-   if ((rc = upload(s.get(), img.tris, &s->d.tris)) != PTX_OK) return rc;
-   if ((rc = upload(s.get(), s->bvh.pairs, &s->d.pairs)) != PTX_OK) return rc;
-   if ((rc = upload(s.get(), img.meshes, &s->d.meshes)) != PTX_OK) return rc;
+   Uploads up{s.get(), {}};
+   up.add(img.nodes, &s->d.nodes);
+   up.add(img.tris, &s->d.tris);
+   up.add(s->bvh.pairs, &s->d.pairs);
+   up.add(img.meshes, &s->d.meshes);
+   std::vector<uint32_t> blob;
+   const uint32_t *dev_blob = nullptr;
    if (s->has_texture) {
       // one texture record per leaf-ordered triangle, then the texel pool (each
       // texture that a mesh uses, once), in one allocation
@@ -411,7 +458,7 @@ int ptx_scene_create(ptx_device *dev, const ptx_scene_desc *desc, ptx_scene **ou
          pool += size_t(desc->textures[t].width) * desc->textures[t].height;
       }
       if (pool > 0xFFFFFFFFull) return set_error(PTX_ERR_INVALID, "a scene's textures exceed 2^32 texels");
-      std::vector<uint32_t> blob(nt * (sizeof(TexTri) / 4) + pool, 0u);
+      blob.assign(nt * (sizeof(TexTri) / 4) + pool, 0u);
       TexTri *rec = reinterpret_cast<TexTri *>(blob.data());
       for (size_t k = 0; k < nt; k++) {
          const uint32_t mi = s->bvh.pairs[2 * k], face = s->bvh.pairs[2 * k + 1];
@@ -426,48 +473,46 @@ int ptx_scene_create(ptx_device *dev, const ptx_scene_desc *desc, ptx_scene **ou
          if (first[t] >= 0)
             std::memcpy(&blob[nt * (sizeof(TexTri) / 4) + first[t]], desc->textures[t].rgba,
                         size_t(desc->textures[t].width) * desc->textures[t].height * 4);
-      const uint32_t *dev_blob = nullptr;
-      if ((rc = upload(s.get(), blob, &dev_blob)) != PTX_OK) return rc;
-      s->d.tex_tris = reinterpret_cast<const TexTri *>(dev_blob);
+      up.add(blob, &dev_blob);
    }
-   if ((rc = upload(s.get(), img.normals, &s->d.normals)) != PTX_OK) return rc;
-   if (desc->num_lights) {
-      std::vector<float> lights(6 * (size_t)desc->num_lights);
-      for (uint32_t i = 0; i < desc->num_lights; i++) {
-         std::copy(desc->lights[i].position, desc->lights[i].position + 3, &lights[6 * i]);
-         std::copy(desc->lights[i].intensity, desc->lights[i].intensity + 3, &lights[6 * i + 3]);
-      }
-      if ((rc = upload(s.get(), lights, &s->d.lights)) != PTX_OK) return rc;
+   up.add(img.normals, &s->d.normals);
+   std::vector<float> lights(6 * (size_t)desc->num_lights);
+   for (uint32_t i = 0; i < desc->num_lights; i++) {
+      std::copy(desc->lights[i].position, desc->lights[i].position + 3, &lights[6 * i]);
+      std::copy(desc->lights[i].intensity, desc->lights[i].intensity + 3, &lights[6 * i + 3]);
    }
+   up.add(lights, &s->d.lights);
+   if ((rc = up.run()) != PTX_OK) return rc;
+   s->d.tex_tris = reinterpret_cast<const TexTri *>(dev_blob);
    // the four-wide form last, out of the memory that everything a scene cannot
-   // do without has left: one that finds none is dropped.  Its faces come from
-   // the triangles and ids just uploaded, while the host still builds the nodes
-   const size_t kept = s->allocations.size(), face_bytes = size_t(img.num_tris) * sizeof(WideFace);
+   // do without has left: one that finds none is dropped.  Its faces are made
+   // here for a few, else on the device from the triangles and ids just uploaded
+   const size_t kept = s->allocations.size();
    const uint64_t kept_bytes = s->info.device_bytes;
-   void *faces = nullptr;
-   if (face_bytes && hipMalloc(&faces, face_bytes) == hipSuccess) {
-      s->allocations.push_back(faces);
-      s->info.device_bytes += face_bytes;
-      if (launch_build_wide_faces(s->d.tris, s->d.pairs, img.num_tris, static_cast<WideFace *>(faces), nullptr) != 0) {
-         (void)hipGetLastError();
-         return set_error(PTX_ERR_HIP, "four-wide face records");
-      }
-   } else {
-      (void)hipGetLastError();
-      faces = nullptr;
+   const bool built = wide_built.valid() ? wide_built.get() : make_wide();
+   std::vector<WideFace> few(img.num_tris <= kWideBeside ? img.num_tris : 0);
+   for (size_t k = 0; k < few.size(); k++) {
+      std::copy(&img.tris[9 * k], &img.tris[9 * k] + 9, few[k].v);
+      few[k].mesh = s->bvh.pairs[2 * k];
+      few[k].face = s->bvh.pairs[2 * k + 1];
+      few[k].pad = 0;
    }
-   const bool built = (wide_built.valid() ? wide_built.get() : make_wide()) && faces;
-   if (built && upload(s.get(), wide.nodes, &s->w.nodes) == PTX_OK &&
-       upload(s.get(), wide.leaves, &s->w.leaves) == PTX_OK) {
-      s->w.faces = static_cast<const WideFace *>(faces);
+   up.add(few.empty() ? nullptr : few.data(), img.num_tris, &s->w.faces);
+   up.add(wide.nodes, &s->w.nodes);
+   up.add(wide.leaves, &s->w.leaves);
+   if (built && up.run() == PTX_OK) {
       s->w.root = wide.root;
       s->w.stack = wide.stack;
+      if (few.empty()) {
+         if (launch_build_wide_faces(s->d.tris, s->d.pairs, img.num_tris, const_cast<WideFace *>(s->w.faces),
+                                     nullptr) != 0) {
+            (void)hipGetLastError();
+            return set_error(PTX_ERR_HIP, "four-wide face records");
+         }
+         PTX_HIP_TRY(hipStreamSynchronize(nullptr));
+      }
    } else {
-      (void)hipGetLastError();
       s->w = WideScene{};
-   }
-   if (faces) PTX_HIP_TRY(hipStreamSynchronize(nullptr));
-   if (!s->w.faces) {
       for (; s->allocations.size() > kept; s->allocations.pop_back()) (void)hipFree(s->allocations.back());
       s->info.device_bytes = kept_bytes;
    }

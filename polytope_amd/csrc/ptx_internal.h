@@ -5,6 +5,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -158,6 +159,23 @@ constexpr uint32_t kMaxRoundChunks = 64;
 
 // ---------------------------------------------------------------- host-side scene
 
+// A vector whose resize leaves new elements unset: large arrays that several
+// threads fill are then first touched by those threads.
+template <class T>
+struct UnsetAlloc : std::allocator<T> {
+   template <class U>
+   struct rebind {
+      using other = UnsetAlloc<U>;
+   };
+   template <class U, class... A>
+   void construct(U *p, A &&...a) {
+      if constexpr (sizeof...(A) == 0) ::new (static_cast<void *>(p)) U;
+      else ::new (static_cast<void *>(p)) U(std::forward<A>(a)...);
+   }
+};
+template <class T>
+using UnsetVector = std::vector<T, UnsetAlloc<T>>;
+
 struct HostBvh {
    std::vector<ptx_bvh_node> nodes;       // reference compact layout
    std::vector<uint32_t> pairs;           // 2 per leaf entry (mesh, face)
@@ -165,9 +183,9 @@ struct HostBvh {
 
 struct WorldMesh {
    uint32_t nf = 0;
-   std::vector<float> wv;                 // 9 floats per face (world v0, v1, v2)
+   UnsetVector<float> wv;                 // 9 floats per face (world v0, v1, v2)
    bool has_normals = false;
-   std::vector<float> wn;                 // 9 floats per face (world corner normals)
+   UnsetVector<float> wn;                 // 9 floats per face (world corner normals)
    std::vector<float> uv;                 // textured: 6 floats per face (u, v of corners 0, 1, 2)
    int32_t texture = -1;                  // textured: index into the scene's texture table
    MeshRec rec{};

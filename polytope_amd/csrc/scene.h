@@ -32,23 +32,6 @@ struct HostQueryStaging;
 
 namespace ptx {
 
-// A vector whose resize leaves new elements unset: large arrays that several
-// threads fill are then first touched by those threads.
-template <class T>
-struct UnsetAlloc : std::allocator<T> {
-   template <class U>
-   struct rebind {
-      using other = UnsetAlloc<U>;
-   };
-   template <class U, class... A>
-   void construct(U *p, A &&...a) {
-      if constexpr (sizeof...(A) == 0) ::new (static_cast<void *>(p)) U;
-      else ::new (static_cast<void *>(p)) U(std::forward<A>(a)...);
-   }
-};
-template <class T>
-using UnsetVector = std::vector<T, UnsetAlloc<T>>;
-
 struct HostImage {
    UnsetVector<Node64> nodes;
    UnsetVector<float> tris;
@@ -65,9 +48,10 @@ struct HostImage {
 int layout_scene(const std::vector<WorldMesh> &meshes, const HostBvh &bvh, HostImage &img, unsigned threads = 0);
 
 // f(lo, hi) over [0, n) on up to `threads` host threads (0 = all cores, at most
-// 16), none with fewer than `least` items; the calling thread takes a share.
-template <class F>
-void host_ranges(size_t n, unsigned threads, size_t least, F f) {
+// 16), none with fewer than `least` items; the calling thread takes a share,
+// after beside(), which needs nothing of f.
+template <class F, class G>
+void host_ranges(size_t n, unsigned threads, size_t least, F f, G beside) {
    if (threads == 0) threads = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
    const size_t parts = std::max<size_t>(1, std::min<size_t>(threads, n / std::max<size_t>(1, least)));
    std::vector<std::thread> ts;
@@ -79,8 +63,13 @@ void host_ranges(size_t n, unsigned threads, size_t least, F f) {
          f(n * t / parts, n * (t + 1) / parts);
       }
    }
+   beside();
    f(size_t(0), n / parts);
    for (std::thread &t : ts) t.join();
+}
+template <class F>
+void host_ranges(size_t n, unsigned threads, size_t least, F f) {
+   host_ranges(n, threads, least, f, [] {});
 }
 
 double now_s();

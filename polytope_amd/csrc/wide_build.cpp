@@ -25,20 +25,22 @@ constexpr float kLimit = 1e16f;                // kWideLimit of wide.h
 constexpr int kStepExponent = 24;              // kWideStep of wide.h
 constexpr uint32_t kIndexEnd = 0x1FFFFFFEu;    // leaf indices stay below the reserved references
 constexpr uint32_t kMaxNodes = 1u << 26;       // 32-bit byte offsets into the node array
+// Nodes that a thread checks or builds at least: about 0.1 ms of either.
+constexpr size_t kCheckNodes = 8192, kBuildNodes = 2048;
 constexpr uint32_t kLeafHeader = kLeafBit, kLeafOne = kLeafBit | (1u << 29), kLeafTwo = kLeafBit | (2u << 29);
 
 // later[] bits of a pair of children i < j (tree order) whose paths part at a
 // node split on axis a: octants with a clear visit j after i, the others i
 // after j (octants 0-3 have z clear).
 struct PairTable {
-   uint16_t bits[3][kWide][kWide][4];
+   uint64_t bits[3][kWide][kWide];                // later[0] in the low 16 bits
    PairTable() {
       std::memset(bits, 0, sizeof(bits));
       for (uint32_t a = 0; a < 3; a++)
          for (uint32_t i = 0; i < kWide; i++)
             for (uint32_t j = i + 1; j < kWide; j++)
                for (uint32_t o = 0; o < 4; o++)
-                  bits[a][i][j][o] = (uint16_t)((o >> a & 1u) ? 1u << (4 * j + i) : 1u << (4 * i + j));
+                  bits[a][i][j] |= uint64_t((o >> a & 1u) ? 1u << (4 * j + i) : 1u << (4 * i + j)) << (16 * o);
    }
 };
 
@@ -50,18 +52,29 @@ double diff(double a, double b, bool up) {
    return s;
 }
 
-// Whether the corners of leaf b's faces (v) span its box exactly.
+// Three of a point's coordinates and whatever follows them in memory.
+typedef float Lanes __attribute__((vector_size(16)));
+typedef int Mask __attribute__((vector_size(16)));
+inline Lanes lanes(const float *p) {
+   Lanes x;
+   std::memcpy(&x, p, sizeof x);
+   return x;
+}
+inline bool all3(Mask m) { return (m[0] & m[1] & m[2]) != 0; }
+
+// Whether the corners of leaf b's kFaces faces (v, and four bytes behind) span
+// its box exactly, none of them NaN (those a minimum skips).
+template <int kFaces>
 bool corners_span(const ptx_bvh_node &b, const float *v) {
-   float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-   for (size_t i = 0; i < 3 * size_t(b.num_faces); i++)
-      for (int k = 0; k < 3; k++) {
-         if (!(std::fabs(v[3 * i + k]) < kLimit)) return false;
-         lo[k] = std::min(lo[k], v[3 * i + k]);
-         hi[k] = std::max(hi[k], v[3 * i + k]);
-      }
-   for (int k = 0; k < 3; k++)
-      if (lo[k] != b.p0[k] || hi[k] != b.p1[k]) return false;
-   return true;
+   Lanes lo = lanes(v), hi = lo;
+   Mask ok = lo == lo;
+   for (int i = 1; i < 3 * kFaces; i++) {
+      const Lanes x = lanes(v + 3 * i);
+      lo = x < lo ? x : lo;
+      hi = x > hi ? x : hi;
+      ok &= x == x;
+   }
+   return all3(ok & (lo == lanes(b.p0)) & (hi == lanes(b.p1)));
 }
 
 // 2^e for e in the normal range.
@@ -70,6 +83,13 @@ double pow2(int e) {
    double x;
    std::memcpy(&x, &bits, 8);
    return x;
+}
+
+// floor(log2(x)) of a normal x > 0.
+int floor_log2(double x) {
+   uint64_t bits;
+   std::memcpy(&bits, &x, 8);
+   return int(bits >> 52) - 1023;
 }
 
 // Subtree costs of the cut: cost[i - 1] = the least area sum when the subtree
@@ -122,46 +142,52 @@ bool build_wide(const HostBvh &bvh, const HostImage &img, unsigned threads, Wide
    // leaves need no header: of one or two faces whose corners span the box.
    UnsetVector<uint8_t> plain(nn);
    std::atomic<bool> nest{true};
-   host_ranges(nn, threads, 65536, [&](size_t lo, size_t hi) {
+   auto check = [&](size_t lo, size_t hi) {
       bool good = true;
       for (size_t i = lo; i < hi && good; i++) {
          const ptx_bvh_node &b = nodes[i];
-         for (int k = 0; k < 3; k++) good &= b.p0[k] <= b.p1[k] && b.p0[k] > -kLimit && b.p1[k] < kLimit;
+         const Lanes p0 = lanes(b.p0), p1 = lanes(b.p1);
+         good &= all3((p0 <= p1) & (p0 > -kLimit) & (p1 < kLimit));
          if (b.num_faces) {
-            plain[i] = b.num_faces <= 2 && corners_span(b, &img.tris[9 * size_t(b.offset)]);
+            const float *v = &img.tris[9 * size_t(b.offset)];
+            plain[i] = b.num_faces == 1 ? corners_span<1>(b, v) : b.num_faces == 2 && corners_span<2>(b, v);
             continue;
          }
-         for (const size_t c : {i + 1, i + b.offset})
-            for (int k = 0; k < 3; k++) good &= nodes[c].p0[k] >= b.p0[k] && nodes[c].p1[k] <= b.p1[k];
+         const ptx_bvh_node &l = nodes[i + 1], &h = nodes[i + b.offset];
+         good &= all3((lanes(l.p0) >= p0) & (lanes(l.p1) <= p1) & (lanes(h.p0) >= p0) & (lanes(h.p1) <= p1));
       }
       if (!good) nest = false;
-   });
-   if (!nest) return false;
-   // the cut, from the last node to the first (children follow their parents)
+   };
+   // beside it the cut, from the last node to the first (children follow their
+   // parents; of boxes that do not nest it is any cut)
    UnsetVector<Cut> cut(nn);
-   for (size_t q = nn; q-- > 0;) {
-      const ptx_bvh_node &b = nodes[q];
-      Cut &c = cut[q];
-      if (b.num_faces) {
-         c = Cut{{0.f, 0.f, 0.f}, 0, 0, 0};
-         continue;
+   auto cuts = [&] {
+      for (size_t q = nn; q-- > 0;) {
+         const ptx_bvh_node &b = nodes[q];
+         Cut &c = cut[q];
+         if (b.num_faces) {
+            c = Cut{{0.f, 0.f, 0.f}, 0, 0, 0};
+            continue;
+         }
+         const Cut &l = cut[q + 1], &r = cut[q + b.offset];
+         const float d2 = l.cost[0] + r.cost[0];
+         const float d3a = l.cost[0] + r.cost[1], d3b = l.cost[1] + r.cost[0];
+         const float d4a = l.cost[0] + r.cost[2], d4b = l.cost[1] + r.cost[1], d4c = l.cost[2] + r.cost[0];
+         const float d3 = std::min(d3a, d3b);
+         float d4 = d4b;
+         c.split4 = 2;
+         if (d4a < d4) { d4 = d4a; c.split4 = 1; }
+         if (d4c < d4) { d4 = d4c; c.split4 = 3; }
+         const float x = b.p1[0] - b.p0[0], y = b.p1[1] - b.p0[1], z = b.p1[2] - b.p0[2];
+         c.cost[0] = d4 + (x * y + y * z + z * x);
+         c.split3 = c.cost[0] <= d3 ? 0 : d3a <= d3b ? 1 : 2;
+         c.split2 = c.cost[0] <= d2 ? 0 : 1;
+         c.cost[1] = std::min(c.cost[0], d2);
+         c.cost[2] = std::min(c.cost[0], d3);
       }
-      const Cut &l = cut[q + 1], &r = cut[q + b.offset];
-      const float d2 = l.cost[0] + r.cost[0];
-      const float d3a = l.cost[0] + r.cost[1], d3b = l.cost[1] + r.cost[0];
-      const float d4a = l.cost[0] + r.cost[2], d4b = l.cost[1] + r.cost[1], d4c = l.cost[2] + r.cost[0];
-      const float d3 = std::min(d3a, d3b);
-      float d4 = d4b;
-      c.split4 = 2;
-      if (d4a < d4) { d4 = d4a; c.split4 = 1; }
-      if (d4c < d4) { d4 = d4c; c.split4 = 3; }
-      const float x = b.p1[0] - b.p0[0], y = b.p1[1] - b.p0[1], z = b.p1[2] - b.p0[2];
-      c.cost[0] = d4 + (x * y + y * z + z * x);
-      c.split3 = c.cost[0] <= d3 ? 0 : d3a <= d3b ? 1 : 2;
-      c.split2 = c.cost[0] <= d2 ? 0 : 1;
-      c.cost[1] = std::min(c.cost[0], d2);
-      c.cost[2] = std::min(c.cost[0], d3);
-   }
+   };
+   host_ranges(nn, threads, kCheckNodes, check, cuts);
+   if (!nest) return false;
    // wide nodes in tree order
    UnsetVector<uint32_t> index(nn), roots;
    WideLeaf empty;
@@ -196,7 +222,7 @@ bool build_wide(const HostBvh &bvh, const HostImage &img, unsigned threads, Wide
    static const PairTable pairs;
    out.nodes.resize(roots.size());
    std::vector<uint8_t> count(roots.size());
-   host_ranges(roots.size(), threads, 8192, [&](size_t first, size_t last) {
+   host_ranges(roots.size(), threads, kBuildNodes, [&](size_t first, size_t last) {
       Gather g{nodes, cut};
       for (size_t w = first; w < last; w++) {
          g.root(roots[w]);
@@ -210,8 +236,7 @@ bool build_wide(const HostBvh &bvh, const HostImage &img, unsigned threads, Wide
             const double extent = diff(box.p1[a], lo, true);
             int e = -60;
             if (extent > 0) {
-               (void)std::frexp(extent / 255.0, &e);
-               e = std::max(e - 1, -60);
+               e = std::max(floor_log2(extent / 255.0), -60);
                while (extent * pow2(-e) > 255.0) e++;
             }
             o.org[a] = lo;
@@ -232,10 +257,10 @@ bool build_wide(const HostBvh &bvh, const HostImage &img, unsigned threads, Wide
          }
          o.used = (uint8_t)((1u << g.n) - 1u);
          for (uint32_t k = 0; k < kWide; k++) o.ref[k] = k < g.n ? index[g.child[k]] : kLeafHeader;
-         std::memset(o.later, 0, sizeof(o.later));
+         uint64_t later = 0;
          for (uint32_t i = 0; i < g.n; i++)
-            for (uint32_t j = i + 1; j < g.n; j++)
-               for (uint32_t q = 0; q < 4; q++) o.later[q] |= pairs.bits[g.axis[i][j]][i][j][q];
+            for (uint32_t j = i + 1; j < g.n; j++) later |= pairs.bits[g.axis[i][j]][i][j];
+         std::memcpy(o.later, &later, sizeof(o.later));
          count[w] = (uint8_t)g.n;
       }
    });

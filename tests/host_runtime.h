@@ -7,6 +7,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -24,7 +25,8 @@ struct Launch {
 struct State {
    std::mutex mu;
    std::map<void *, size_t> device;            // live device allocations
-   size_t used = 0, peak = 0, limit = SIZE_MAX;
+   size_t used = 0, limit = SIZE_MAX;
+   uint32_t allocations = 0, copies = 0;        // made so far
    int blocks_per_cu = 4;                      // every kernel's occupancy
    std::map<const void *, std::string> names;  // kernels by host function
    std::vector<Launch> launches;
@@ -48,7 +50,7 @@ inline hipError_t take(void **p, size_t bytes) {
    *p = std::aligned_alloc(256, (bytes + 255) / 256 * 256);
    s.device[*p] = bytes;
    s.used += bytes;
-   s.peak = std::max(s.peak, s.used);
+   s.allocations++;
    return hipSuccess;
 }
 inline hipError_t give(void *p) {
@@ -137,6 +139,7 @@ hipError_t hipHostFree(void *p) {
    return hipSuccess;
 }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) {
+   state().copies++;
    std::memcpy(d, s, n);
    return hipSuccess;
 }

@@ -1,15 +1,17 @@
 // Host check of ptx_scene_create at every memory limit: a scene with corner
 // normals, a texture and a light is created wherever the arrays that it cannot
 // do without fit, with its four-wide form only where that fits too, and no
-// limit leaves an allocation behind.  Prints the failures; exit 1 on any.
+// limit leaves an allocation behind.  A creation makes two allocations and, of
+// a small scene, two copies and no launch.  Prints the failures; exit 1 on any.
 #include <cmath>
 #include <cstdio>
 
 #include "host_runtime.h"
 #include "ptx.h"
 
-int main() {
-   constexpr uint32_t kSide = 24, kVerts = (kSide + 1) * (kSide + 1), kFaces = 2 * kSide * kSide, kTex = 16;
+// A sheet of 2 side^2 faces; returns the number of failures.
+static int check(uint32_t kSide) {
+   const uint32_t kVerts = (kSide + 1) * (kSide + 1), kFaces = 2 * kSide * kSide, kTex = 16;
    std::vector<float> x(kVerts), y(kVerts), z(kVerts), up(kVerts, 1.f), flat(kVerts, 0.f), u(kVerts), v(kVerts);
    for (uint32_t i = 0; i < kVerts; i++) {
       x[i] = float(i % (kSide + 1));
@@ -53,18 +55,30 @@ int main() {
    const size_t base = rt.used;
    ptx_scene *scene = nullptr;
    ptx_scene_info info{};
+   const uint32_t allocations = rt.allocations, copies = rt.copies;
+   const size_t launches = rt.launches.size();
    if (ptx_scene_create(dev, &desc, &scene) != PTX_OK) return std::printf("no scene: %s\n", ptx_last_error()), 1;
+   int bad = 0;
+   const uint32_t a = rt.allocations - allocations, c = rt.copies - copies, l = uint32_t(rt.launches.size() - launches);
+   if (a != 2 || (kFaces <= 1152 ? c != 2 || l != 0 : l != 1))
+      std::printf("%u faces: %u allocations, %u copies, %u launches\n", kFaces, a, c, l), bad++;
    (void)ptx_scene_get_info(scene, &info);
    const size_t whole = rt.used - base;
-   // records, triangles with their padding, ids, mesh record, texture records and texels, corner normals, light
-   const size_t need = size_t(info.num_interior) * 64 + size_t(kFaces) * 36 + 128 + size_t(info.num_pairs) * 8 + 36 +
-                       size_t(kFaces) * 32 + 4 * kTex * kTex + size_t(kFaces) * 36 + 24;
-   int bad = 0;
-   if (info.device_bytes != whole || whole <= need)
-      std::printf("%zu bytes used, %zu told, %zu needed\n", whole, (size_t)info.device_bytes, need), bad++;
+   // records, triangles with their padding, ids, mesh record, texture records and texels, corner normals,
+   // light; seven arrays, which may be padded to 256 bytes each
+   const size_t least = size_t(info.num_interior) * 64 + size_t(kFaces) * 36 + 128 + size_t(info.num_pairs) * 8 + 36 +
+                        size_t(kFaces) * 32 + 4 * kTex * kTex + size_t(kFaces) * 36 + 24;
+   if (info.device_bytes != whole) std::printf("%zu bytes used, %zu told\n", whole, (size_t)info.device_bytes), bad++;
+   ptx_scene_destroy(scene);
+   // what it takes without the form: at the largest limit that the whole misses
+   rt.limit = base + whole - 1;
+   if (ptx_scene_create(dev, &desc, &scene) != PTX_OK) return std::printf("refused: %s\n", ptx_last_error()), 1;
+   const size_t need = rt.used - base;
+   if (need < least || need > least + 7 * 256) std::printf("%zu bytes without the form, %zu needed\n", need, least), bad++;
    ptx_scene_destroy(scene);
    uint32_t with = 0, without = 0, refused = 0;
-   for (size_t limit = 0; limit <= whole; limit += limit + 1009 < whole ? 1009 : std::max<size_t>(1, whole - limit)) {
+   const size_t step = whole / 211 + 1;
+   for (size_t limit = 0; limit <= whole; limit += limit + step < whole ? step : std::max<size_t>(1, whole - limit)) {
       rt.limit = base + limit;
       scene = nullptr;
       const int rc = ptx_scene_create(dev, &desc, &scene);
@@ -85,6 +99,13 @@ int main() {
    }
    rt.limit = SIZE_MAX;
    ptx_device_close(dev);
-   std::printf("%u scenes with the four-wide form, %u without, %u refused, %d failures\n", with, without, refused, bad);
-   return bad || !with || !without || !refused;
+   std::printf("%u scenes with the four-wide form, %u without, %u refused\n", with, without, refused);
+   return bad + (!with || !without || !refused);
+}
+
+int main() {
+   int bad = 0;
+   for (uint32_t side : {4u, 24u, 48u}) bad += check(side);      // 32, 1,152 and 4,608 faces
+   std::printf("%d failures\n", bad);
+   return bad != 0;
 }

@@ -33,4 +33,4 @@ def run_check(tmp_path, name: str) -> str:
 
 
 def test_scene_creation_at_every_memory_limit(tmp_path):
-    assert " 0 failures" in run_check(tmp_path, "scene_memory_check")
+    assert "\n0 failures" in run_check(tmp_path, "scene_memory_check")
