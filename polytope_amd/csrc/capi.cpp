@@ -495,16 +495,18 @@ int ptx_scene_create(ptx_device *dev, const ptx_scene_desc *desc, ptx_scene **ou
       std::copy(&img.tris[9 * k], &img.tris[9 * k] + 9, few[k].v);
       few[k].mesh = s->bvh.pairs[2 * k];
       few[k].face = s->bvh.pairs[2 * k + 1];
-      few[k].pad = 0;
+      few[k].flat = k < wide.flat.size() ? wide.flat[k] : 0u;
    }
    up.add(few.empty() ? nullptr : few.data(), img.num_tris, &s->w.faces);
    up.add(wide.nodes, &s->w.nodes);
    up.add(wide.leaves, &s->w.leaves);
+   const uint8_t *flat = nullptr;
+   if (few.empty()) up.add(wide.flat, &flat);
    if (built && up.run() == PTX_OK) {
       s->w.root = wide.root;
       s->w.stack = wide.stack;
       if (few.empty()) {
-         if (launch_build_wide_faces(s->d.tris, s->d.pairs, img.num_tris, const_cast<WideFace *>(s->w.faces),
+         if (launch_build_wide_faces(s->d.tris, s->d.pairs, flat, img.num_tris, const_cast<WideFace *>(s->w.faces),
                                      nullptr) != 0) {
             (void)hipGetLastError();
             return set_error(PTX_ERR_HIP, "four-wide face records");

@@ -59,8 +59,9 @@ int closest_hit_blocks_per_cu(uint32_t lds_depth, bool extra, bool windows);
 int launch_build_windows(const Node64 *nodes, uint32_t n_int, Node64 *win, hipStream_t stream);
 
 // Face records of the four-wide form from the scene's np leaf-ordered triangles
-// and ids.
-int launch_build_wide_faces(const float *tris, const uint32_t *pairs, uint32_t np, WideFace *out, hipStream_t stream);
+// and ids and their flat words (or null for none).
+int launch_build_wide_faces(const float *tris, const uint32_t *pairs, const uint8_t *flat, uint32_t np, WideFace *out,
+                            hipStream_t stream);
 
 // Size of the per-device static scratch of the no-allocation closest-hit entry
 // point: 256 bytes of work counters, then the deferred-stack spill.

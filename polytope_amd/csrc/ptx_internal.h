@@ -56,11 +56,13 @@ struct alignas(64) WideNode {
 };
 static_assert(sizeof(WideNode) == 64, "WideNode is 64 bytes");
 
-// A face as the four-wide traversal reads it, at its leaf-ordered index.
+// A face as the four-wide traversal reads it, at its leaf-ordered index.  flat,
+// of a leaf's first face: the axes (bit a) in which the leaf's box is flat and
+// the smallest box above it that is not holds its coordinate strictly inside.
 struct alignas(16) WideFace {
    float v[9];               // world v0, v1, v2
    uint32_t mesh, face;      // the reference's ids
-   uint32_t pad;
+   uint32_t flat;
 };
 static_assert(sizeof(WideFace) == 48, "WideFace layout");
 

@@ -161,8 +161,9 @@ __global__ void k_build_windows(const Node64 *__restrict__ nodes, uint32_t n_int
    win[2 * t + 1] = b;
 }
 
-__global__ void k_build_wide_faces(const float *__restrict__ tris, const uint32_t *__restrict__ pairs, uint32_t np,
-                                   WideFace *__restrict__ out) {
+// flat: WideFace::flat of every face, or null where no leaf is flat.
+__global__ void k_build_wide_faces(const float *__restrict__ tris, const uint32_t *__restrict__ pairs,
+                                   const uint8_t *__restrict__ flat, uint32_t np, WideFace *__restrict__ out) {
    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
    if (p >= np) return;
    WideFace f;
@@ -170,7 +171,7 @@ __global__ void k_build_wide_faces(const float *__restrict__ tris, const uint32_
    for (int k = 0; k < 9; k++) f.v[k] = tris[9 * (size_t)p + k];
    f.mesh = pairs[2 * (size_t)p];
    f.face = pairs[2 * (size_t)p + 1];
-   f.pad = 0;
+   f.flat = flat ? flat[p] : 0u;
    out[p] = f;
 }
 
@@ -343,9 +344,11 @@ int closest_hit_blocks_per_cu(uint32_t lds_depth, bool extra, bool windows) {
    }
 }
 
-int launch_build_wide_faces(const float *tris, const uint32_t *pairs, uint32_t np, WideFace *out, hipStream_t stream) {
+int launch_build_wide_faces(const float *tris, const uint32_t *pairs, const uint8_t *flat, uint32_t np, WideFace *out,
+                            hipStream_t stream) {
    if (np == 0) return 0;
-   hipLaunchKernelGGL(dev::k_build_wide_faces, dim3((np + 255) / 256), dim3(256), 0, stream, tris, pairs, np, out);
+   hipLaunchKernelGGL(dev::k_build_wide_faces, dim3((np + 255) / 256), dim3(256), 0, stream, tris, pairs, flat, np,
+                      out);
    return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -17,8 +17,13 @@
 //
 // The one case in which boxes do not nest as tests: a direction component of
 // -0 makes the reference's slab selections accept a box that is flat in that
-// axis at the origin's coordinate inside boxes they reject.  Such a ray is
-// traced again over the binary records in the reference's own steps
+// axis at the origin's coordinate c inside boxes they reject, those with c on
+// their face.  Of the boxes above such a leaf those that are flat too pass, and
+// of the others the smallest decides: c inside it is inside all of them, and c on
+// its face is rejected there, its interval starting or ending at infinity.  So
+// whether the leaf is visited is known beforehand (WideFace::flat), but for a
+// ray whose other axes leave the interval's end at infinity (kRayLoose): that
+// is traced again over the binary records in the reference's own steps
 // (exact_trace).  Rays with NaN, infinite or all-zero components nest: a NaN
 // slab value leaves the fold as it was in every box, and an infinite one moves
 // with the plane as a finite one does.
@@ -63,6 +68,7 @@ constexpr uint32_t kRayAxisShift = 3, kRayAxisMask = 3u;
 constexpr uint32_t kRaySlow = 1u << 5;     // child tests with the exact slab
 constexpr uint32_t kRayMinus = 1u << 6;    // some 1 / direction is -inf
 constexpr uint32_t kRayHard = 1u << 7;     // an accepted face's t may be NaN: a component is not finite, or all are 0
+constexpr uint32_t kRayLoose = 1u << 14;   // kRayMinus, and no axis bounds every box's interval
 // 16 * the octant's entry of WideNode::later, in bits 8-13
 constexpr uint32_t kRayLaterShift = 8;
 constexpr uint32_t kLaterFlip = 0x7BDEu;   // every pair of different children
@@ -77,7 +83,12 @@ PTX_HD void wide_ray(Ray &r) {
                       r.oy == r.oy && r.oz == r.oz && ax > 0.f && ay > 0.f && az > 0.f;
    if (plain) return;
    uint32_t f = kRaySlow;
-   if (r.ix == -kInf || r.iy == -kInf || r.iz == -kInf) f |= kRayMinus;
+   if (r.ix == -kInf || r.iy == -kInf || r.iz == -kInf) {
+      const bool bounded = (ax < kWideLimit && __builtin_fabsf(r.ox) < kWideLimit) ||
+                           (ay < kWideLimit && __builtin_fabsf(r.oy) < kWideLimit) ||
+                           (az < kWideLimit && __builtin_fabsf(r.oz) < kWideLimit);
+      f |= bounded ? kRayMinus : kRayMinus | kRayLoose;
+   }
    const bool nan = !(r.ix == r.ix && r.iy == r.iy && r.iz == r.iz && r.ox == r.ox && r.oy == r.oy && r.oz == r.oz);
    const bool all_inf = ax == kInf && ay == kInf && az == kInf;
    if (nan || all_inf || !(ax > 0.f && ay > 0.f && az > 0.f) || mo == kInf) f |= kRayHard;
@@ -184,11 +195,11 @@ PTX_HD bool wide_child_slow(const WidePlanes &p, int k, const Ray &r, float gx, 
    return near <= wide_bound(far * kSlabScale) && near <= wide_bound(min_t);     // never past a NaN min_t
 }
 
-// Whether a leaf box that passed is flat at the origin's coordinate in an
-// axis of direction -0: the one test that its ancestors need not pass.
-PTX_HD bool wide_flat(float b0, float b1, float b2, float b3, float b4, float b5, const Ray &r) {
-   return (r.ix == -kInf && b0 == r.ox && b3 == r.ox) || (r.iy == -kInf && b1 == r.oy && b4 == r.oy) ||
-          (r.iz == -kInf && b2 == r.oz && b5 == r.oz);
+// The axes of direction -0 in which a leaf box that passed is flat at the
+// origin's coordinate: the one test that its ancestors need not pass.
+PTX_HD uint32_t wide_flat(float b0, float b1, float b2, float b3, float b4, float b5, const Ray &r) {
+   return (r.ix == -kInf && b0 == r.ox && b3 == r.ox ? 1u : 0u) | (r.iy == -kInf && b1 == r.oy && b4 == r.oy ? 2u : 0u) |
+          (r.iz == -kInf && b2 == r.oz && b5 == r.oz ? 4u : 0u);
 }
 
 // ---------------------------------------------------------------- traversal
@@ -382,6 +393,15 @@ __device__ __forceinline__ bool wide_node_step(Trav &s, const WideNode *nodes, c
    return wide_pop(s, st);
 }
 
+// What a leaf that passed under a direction component of -0 is: visited, not
+// reached by the reference, or for the ray to be traced again.
+enum : uint32_t { kFlatVisit = 0, kFlatSkip = 1, kFlatAgain = 2 };
+__device__ __forceinline__ uint32_t wide_flat_leaf(uint32_t axes, const Ray &r, const WideFace *first) {
+   if (axes == 0) return kFlatVisit;
+   if (r.nk & kRayLoose) return kFlatAgain;
+   return axes & ~as_global(first)->flat ? kFlatSkip : kFlatVisit;
+}
+
 // One leaf step: a header's box, or up to two faces, the first of a one- or
 // two-face leaf after its box, which is the corners' own (the builder checks
 // that).  Returns false when the traversal has ended.
@@ -397,9 +417,13 @@ __device__ __forceinline__ bool wide_leaf_step(Trav &s, const WideFace *faces, c
       float near, far;
       slab(b0, b1, b2, b3, b4, b5, s.r, near, far);
       if (near <= far && near <= s.min_t && count != 0) {
-         s.cur = (s.r.nk & kRayMinus) && wide_flat(b0, b1, b2, b3, b4, b5, s.r) ? kWideExact : kWideRaw | first;
-         s.cnt = count;
-         done = false;
+         uint32_t what = kFlatVisit;
+         if (s.r.nk & kRayMinus) what = wide_flat_leaf(wide_flat(b0, b1, b2, b3, b4, b5, s.r), s.r, faces + first);
+         if (what != kFlatSkip) {
+            s.cur = what == kFlatAgain ? kWideExact : kWideRaw | first;
+            s.cnt = count;
+            done = false;
+         }
       }
    } else {
       const uint32_t n = kind == kWideRaw ? s.cnt : kind == kWideTwo ? 2u : 1u;
@@ -424,9 +448,13 @@ __device__ __forceinline__ bool wide_leaf_step(Trav &s, const WideFace *faces, c
          float near, far;
          slab(x0, y0, z0, x1, y1, z1, s.r, near, far);
          in = near <= far && near <= s.min_t;
-         if (in && (s.r.nk & kRayMinus) && wide_flat(x0, y0, z0, x1, y1, z1, s.r)) {
-            s.cur = kWideExact;
-            in = done = false;
+         if (in && (s.r.nk & kRayMinus)) {
+            const uint32_t what = wide_flat_leaf(wide_flat(x0, y0, z0, x1, y1, z1, s.r), s.r, faces + idx);
+            in = what == kFlatVisit;
+            if (what == kFlatAgain) {
+               s.cur = kWideExact;
+               done = false;
+            }
          }
       }
       if (in) {

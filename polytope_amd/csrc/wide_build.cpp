@@ -61,6 +61,7 @@ inline Lanes lanes(const float *p) {
    return x;
 }
 inline bool all3(Mask m) { return (m[0] & m[1] & m[2]) != 0; }
+inline bool any3(Mask m) { return (m[0] | m[1] | m[2]) != 0; }
 
 // Whether the corners of leaf b's kFaces faces (v, and four bytes behind) span
 // its box exactly, none of them NaN (those a minimum skips).
@@ -75,6 +76,42 @@ bool corners_span(const ptx_bvh_node &b, const float *v) {
       ok &= x == x;
    }
    return all3(ok & (lo == lanes(b.p0)) & (hi == lanes(b.p1)));
+}
+
+// WideFace::flat of every face: down the tree, a box that is flat in an axis
+// takes its parent's answer if that is flat too, else whether the parent holds
+// the coordinate strictly inside.  False when two boxes above one leaf, or two
+// leaves of one face, give different answers (trees a caller brings).
+bool flat_leaves(const std::vector<ptx_bvh_node> &nodes, size_t faces, UnsetVector<uint8_t> &out) {
+   constexpr uint8_t kNot = 0xFF;
+   std::vector<uint8_t> inside(nodes.size(), kNot);
+   inside[0] = 7;
+   out.assign(faces, kNot);
+   bool same = true;
+   for (size_t i = 0; i < nodes.size(); i++) {
+      const ptx_bvh_node &b = nodes[i];
+      if (inside[i] == kNot) continue;          // a node that nothing refers to
+      if (b.num_faces) {
+         uint8_t axes = 0;
+         for (int a = 0; a < 3; a++) axes |= b.p0[a] == b.p1[a] ? inside[i] & 1u << a : 0u;
+         uint8_t &f = out[b.offset];
+         same &= f == kNot || f == axes;
+         f = axes;
+         continue;
+      }
+      for (const size_t c : {i + 1, i + b.offset}) {
+         uint8_t in = 0;
+         for (int a = 0; a < 3; a++) {
+            const float x = nodes[c].p0[a];
+            if (x == nodes[c].p1[a] && (b.p0[a] == b.p1[a] ? inside[i] >> a & 1u : b.p0[a] < x && x < b.p1[a]))
+               in |= uint8_t(1u << a);
+         }
+         same &= inside[c] == kNot || inside[c] == in;
+         inside[c] = in;
+      }
+   }
+   for (uint8_t &f : out) f = f == kNot ? 0 : f;
+   return same;
 }
 
 // 2^e for e in the normal range.
@@ -141,14 +178,15 @@ bool build_wide(const HostBvh &bvh, const HostImage &img, unsigned threads, Wide
    // the equality of the leaves visited rests on.  In the same pass, which
    // leaves need no header: of one or two faces whose corners span the box.
    UnsetVector<uint8_t> plain(nn);
-   std::atomic<bool> nest{true};
+   std::atomic<bool> nest{true}, flat{false};
    auto check = [&](size_t lo, size_t hi) {
-      bool good = true;
+      bool good = true, some = false;
       for (size_t i = lo; i < hi && good; i++) {
          const ptx_bvh_node &b = nodes[i];
          const Lanes p0 = lanes(b.p0), p1 = lanes(b.p1);
          good &= all3((p0 <= p1) & (p0 > -kLimit) & (p1 < kLimit));
          if (b.num_faces) {
+            some |= any3(p0 == p1);
             const float *v = &img.tris[9 * size_t(b.offset)];
             plain[i] = b.num_faces == 1 ? corners_span<1>(b, v) : b.num_faces == 2 && corners_span<2>(b, v);
             continue;
@@ -157,6 +195,7 @@ bool build_wide(const HostBvh &bvh, const HostImage &img, unsigned threads, Wide
          good &= all3((lanes(l.p0) >= p0) & (lanes(l.p1) <= p1) & (lanes(h.p0) >= p0) & (lanes(h.p1) <= p1));
       }
       if (!good) nest = false;
+      if (some) flat = true;
    };
    // beside it the cut, from the last node to the first (children follow their
    // parents; of boxes that do not nest it is any cut)
@@ -188,6 +227,7 @@ bool build_wide(const HostBvh &bvh, const HostImage &img, unsigned threads, Wide
    };
    host_ranges(nn, threads, kCheckNodes, check, cuts);
    if (!nest) return false;
+   if (flat && !flat_leaves(nodes, np, out.flat)) return false;
    // wide nodes in tree order
    UnsetVector<uint32_t> index(nn), roots;
    WideLeaf empty;

@@ -9,6 +9,7 @@ namespace ptx {
 struct WideImage {
    UnsetVector<WideNode> nodes;
    std::vector<WideLeaf> leaves;    // leaf 0 is empty
+   UnsetVector<uint8_t> flat;       // WideFace::flat of every face, or nothing where no leaf is flat
    uint32_t root = 0;               // wide node or leaf reference
    uint32_t stack = 1;              // 8-byte stack entries a lane needs
 };

@@ -367,3 +367,65 @@ def test_idle_lanes_marked_by_their_directions_agree(share):
     finally:
         scene.close()
         dev.close()
+
+
+def test_rays_in_the_planes_of_flat_leaves_step_over_the_wide_tree(tmp_path):
+    """Under a direction component of -0 a flat leaf at the origin's coordinate
+    is visited or not by the boxes above it, without a second traversal."""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not Path(hipcc).exists():
+        pytest.skip("hipcc not found")
+    exe = tmp_path / "wide_flat_check"
+    csrc = ROOT / "polytope_amd" / "csrc"
+    subprocess.run([hipcc, "-O2", "-std=c++17", "-ffp-contract=off", "-x", "hip", "--offload-arch=gfx950",
+                    "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                    f"-I{csrc}", f"-I{ROOT / 'include'}", str(ROOT / "tests" / "wide_flat_check.cpp"),
+                    *(str(csrc / f) for f in ("wide_build.cpp", "bvh_build.cpp", "scene.cpp")), "-lpthread",
+                    "-o", str(exe)], check=True, capture_output=True, timeout=300)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stdout
+    assert " 0 mismatches" in out.stdout
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("side", [1, 6, 40])
+@pytest.mark.parametrize("n", [65, 20_011])
+def test_rays_in_the_plane_of_a_floor_agree(side, n):
+    """A floor of 2 side^2 triangles (face records made by the host, from 40 on
+    by the device) below a sphere, rays that start on it with -0 and 0 as their
+    vertical component and rays from its corners: the words of the binary form."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from polytope_amd import Device, Scene
+    g = np.linspace(-4, 4, side + 1, dtype=np.float32)
+    x, z = np.meshgrid(g, g)
+    floor = np.stack([x, 0 * x, z], -1).reshape(-1, 3)
+    i = np.arange(side * (side + 1)).reshape(side, side + 1)[:, :side].ravel()
+    quads = np.concatenate([np.stack([i, i + 1, i + side + 1], 1), np.stack([i + 1, i + side + 2, i + side + 1], 1)])
+    v, f = S.icosphere(2, radius=1.0, center=(0.0, 1.0, 0.0), noise=0.05, seed=3)
+    meshes = [S.MeshData(floor, quads.astype(np.uint32)), S.MeshData(v, f)]
+    rays = S.rays_incoherent((-5.0, -0.5, -5.0), (5.0, 2.0, 5.0), n, 9)
+    rays[::2, 1] = 0.0
+    rays[::2, 4] = -0.0
+    rays[::6, 4] = 0.0
+    rays[::10, 0] = -4.0
+    rays[::14, 3] = -0.0
+    rays[::22, 3:] = -0.0
+    dev = Device(0)
+    scene = Scene(dev, meshes)
+    r = torch.from_numpy(rays).cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+    out = []
+    try:
+        for counters in (True, False):
+            h = torch.full((n, 6), -7, dtype=torch.int32, device="cuda")
+            c = torch.zeros((n, 3), dtype=torch.int32, device="cuda")
+            scene.intersect_device(r.data_ptr(), n, h.data_ptr(), c.data_ptr() if counters else 0, 0, stream)
+            torch.cuda.synchronize()
+            out.append(h.cpu().numpy())
+        assert np.array_equal(out[0][:, :2], out[1][:, :2])
+        assert np.array_equal(out[0][:, 2:].view(np.float32), out[1][:, 2:].view(np.float32), equal_nan=True)
+    finally:
+        scene.close()
+        dev.close()
