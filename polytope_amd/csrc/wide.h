@@ -402,31 +402,34 @@ __device__ __forceinline__ uint32_t wide_flat_leaf(uint32_t axes, const Ray &r, 
    return axes & ~as_global(first)->flat ? kFlatSkip : kFlatVisit;
 }
 
-// One leaf step: a header's box, or up to two faces, the first of a one- or
-// two-face leaf after its box, which is the corners' own (the builder checks
-// that).  Returns false when the traversal has ended.
+// One leaf step: up to two faces, the first of a leaf after its box, which is
+// its header's or, for a one- or two-face leaf, the corners' own (the builder
+// checks that).  Returns false when the traversal has ended.
 template <int kLds>
 __device__ __forceinline__ bool wide_leaf_step(Trav &s, const WideFace *faces, const WideLeaf *leaves,
                                                const WideStack<kLds> &st, bool debug_pixel) {
-   const uint32_t kind = s.cur & ~kWideIndex, idx = s.cur & kWideIndex;
+   const uint32_t kind = s.cur & ~kWideIndex;
+   uint32_t idx = s.cur & kWideIndex, n = kind == kWideRaw ? s.cnt : kind == kWideTwo ? 2u : 1u;
    bool done = true;                                // this leaf is: go on with the next deferred child
+   bool in = true;
    if (kind == kWideHeader) {
       const PTX_GLOBAL WideLeaf *l = as_global(leaves + idx);
       const float b0 = l->box[0], b1 = l->box[1], b2 = l->box[2], b3 = l->box[3], b4 = l->box[4], b5 = l->box[5];
-      const uint32_t first = l->first, count = l->count;
+      idx = l->first;
+      n = l->count;
       float near, far;
       slab(b0, b1, b2, b3, b4, b5, s.r, near, far);
-      if (near <= far && near <= s.min_t && count != 0) {
-         uint32_t what = kFlatVisit;
-         if (s.r.nk & kRayMinus) what = wide_flat_leaf(wide_flat(b0, b1, b2, b3, b4, b5, s.r), s.r, faces + first);
-         if (what != kFlatSkip) {
-            s.cur = what == kFlatAgain ? kWideExact : kWideRaw | first;
-            s.cnt = count;
+      in = near <= far && near <= s.min_t && n != 0;
+      if (in && (s.r.nk & kRayMinus)) {
+         const uint32_t what = wide_flat_leaf(wide_flat(b0, b1, b2, b3, b4, b5, s.r), s.r, faces + idx);
+         in = what == kFlatVisit;
+         if (what == kFlatAgain) {
+            s.cur = kWideExact;
             done = false;
          }
       }
-   } else {
-      const uint32_t n = kind == kWideRaw ? s.cnt : kind == kWideTwo ? 2u : 1u;
+   }
+   if (in) {
       typedef float f32x4 __attribute__((ext_vector_type(4)));
       const PTX_GLOBAL f32x4 *p = as_global(reinterpret_cast<const f32x4 *>(faces + idx));
       const f32x4 a = p[0], b = p[1], c = p[2];
@@ -436,8 +439,7 @@ __device__ __forceinline__ bool wide_leaf_step(Trav &s, const WideFace *faces, c
          e = p[4];
          g = p[5];
       }
-      bool in = true;
-      if (kind != kWideRaw) {
+      if (kind == kWideOne || kind == kWideTwo) {
          // vertices: (a.xyz, a.w b.xy, b.zw c.x), (d.xyz, d.w e.xy, e.zw g.x)
          float x0 = fminf(fminf(a.x, a.w), b.z), x1 = fmaxf(fmaxf(a.x, a.w), b.z);
          float y0 = fminf(fminf(a.y, b.x), b.w), y1 = fmaxf(fmaxf(a.y, b.x), b.w);
@@ -476,9 +478,9 @@ __device__ __forceinline__ bool wide_leaf_step(Trav &s, const WideFace *faces, c
             }
             s.after++;
          }
-         if (kind == kWideRaw && n > 2) {              // more faces in this leaf: the next step goes on
-            s.cur += 2;
-            s.cnt -= 2;
+         if (n > 2) {                                  // more faces in this leaf: the next step goes on
+            s.cur = kWideRaw | (idx + 2);
+            s.cnt = n - 2;
             done = false;
          }
       }

@@ -429,3 +429,50 @@ def test_rays_in_the_plane_of_a_floor_agree(side, n):
     finally:
         scene.close()
         dev.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("copies", [1, 2, 3, 4, 7])
+@pytest.mark.parametrize("widen", [0.0, 0.01])
+def test_leaves_of_any_number_of_faces_agree(copies, widen):
+    """Leaves of one face to more than two steps' worth, whose boxes are their
+    corners' or (in a tree the caller brings) wider: the words of the binary
+    form, in queries and in a render."""
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from polytope_amd import Device, Scene, _abi, build_bvh, render
+    verts, faces = S.icosphere(2, noise=0.05, seed=2)
+    meshes = [S.MeshData(verts, np.concatenate([faces] * copies))]
+    nodes, pairs = build_bvh(meshes)
+    nodes["p0"] -= np.float32(widen)
+    nodes["p1"] += np.float32(widen)
+    n = 5003
+    lo, hi = S.scene_bounds(meshes)
+    rays = _edge_rays(S.rays_incoherent(np.asarray(lo) - 0.2, np.asarray(hi) + 0.2, n, 9), verts)
+    dev = Device(0)
+    scene = Scene(dev, meshes, (10.0, 20.0, 30.0), bvh=(nodes, pairs))
+    r = torch.from_numpy(rays).cuda()
+    stream = torch.cuda.current_stream().cuda_stream
+    out = []
+    try:
+        for counters in (True, False):
+            h = torch.full((n, 6), -7, dtype=torch.int32, device="cuda")
+            c = torch.zeros((n, 3), dtype=torch.int32, device="cuda")
+            f = torch.full((n, 15), -7.0, dtype=torch.float32, device="cuda")
+            scene.intersect_device(r.data_ptr(), n, h.data_ptr(), c.data_ptr() if counters else 0, f.data_ptr(), stream)
+            torch.cuda.synchronize()
+            out.append((h.cpu().numpy(), f.cpu().numpy()))
+        (h0, f0), (h1, f1) = out
+        assert np.array_equal(h0[:, :2], h1[:, :2])
+        assert np.array_equal(h0[:, 2:].view(np.float32), h1[:, 2:].view(np.float32), equal_nan=True)
+        assert np.array_equal(f0, f1, equal_nan=True)
+        cam = S.Camera(S.look_at((0.3, 0.5, -2.5), (0.0, 0.0, 0.0)), 50.0, 40, 30)
+        films = []
+        for form in (dict(), dict(plain_primary=_abi.PLAIN_CACHED), dict(render_mode=_abi.RENDER_WAVEFRONT)):
+            dev.set_tuning(**form)
+            films.append(render(scene, cam, 3, 3, 5).view(np.uint32))
+        assert np.array_equal(films[0], films[1]) and np.array_equal(films[0], films[2])
+    finally:
+        scene.close()
+        dev.close()
