@@ -1185,16 +1185,8 @@ __device__ __forceinline__ void p_begin(const DevScene &S, uint32_t wroot, Trav 
    }
 }
 
-// Three floats of a lane, in registers or in LDS (one plane of the block's lanes
-// per component).
-template <bool kInLds>
-struct LaneVec3 {
-   float v[3];
-   __device__ __forceinline__ float &operator[](uint32_t k) { return v[k]; }
-   __device__ __forceinline__ float operator[](uint32_t k) const { return v[k]; }
-};
-template <>
-struct LaneVec3<true> {
+// Three floats of a lane in LDS (one plane of the block's lanes per component).
+struct LdsVec3 {
    float *p;
    __device__ __forceinline__ float &operator[](uint32_t k) const { return p[k * 256]; }
 };
@@ -1274,8 +1266,10 @@ k_paths(const Chunk *chunks, uint32_t nchunks, uint32_t nslots, const JobDev *jo
    // record's flags in ray words a found hit no longer needs (origin, 1 / d)
    float src[3] = {1.f, 1.f, 1.f};
    // Next-event sum of the path (kNee).  In LDS beside the four-wide stack, where
-   // a block has 4 KB left of a fourth of the CU's 160 KB (the binary form none).
-   LaneVec3<kNee && kWide> direct{};
+   // a block has 4 KB left of a fourth of the CU's 160 KB; the binary form has
+   // none and keeps a plain array (in a struct of one it spills 20 registers
+   // instead of 15, and two next-event jobs take 7.70 instead of 7.30 ms).
+   std::conditional_t<kNee && kWide, LdsVec3, float[3]> direct{};
    if constexpr (kNee && kWide) {
       __shared__ float sums[3 * 256];
       direct.p = sums + threadIdx.x;
