@@ -313,6 +313,9 @@ typedef struct ptx_tuning {
                              /* and counters; ON is slower on MI355X as measured.    */
 } ptx_tuning;
 int ptx_set_tuning(ptx_device *dev, const ptx_tuning *t);
+/* The tuning as it was set.  lds_stack and block_size left at 0 come back as the
+ * value in use; refill_lanes, shade_lanes and leaf_lanes, whose default depends
+ * on the form a kernel steps over, stay 0, and what was got can be set back. */
 int ptx_get_tuning(ptx_device *dev, ptx_tuning *t);
 /* Times candidate tunings on `scene` and keeps the fastest. */
 int ptx_autotune(ptx_device *dev, ptx_scene *scene, ptx_tuning *chosen);

@@ -166,6 +166,7 @@ class Device:
         check(load().ptx_set_tuning(self.handle, C.byref(t)))
 
     def get_tuning(self) -> dict:
+        """The tuning as it was set; 0 = the default of the form a kernel steps over."""
         t = _abi.Tuning()
         check(load().ptx_get_tuning(self.handle, C.byref(t)))
         return {k: getattr(t, k) for k, _ in _abi.Tuning._fields_}

@@ -677,9 +677,9 @@ int ptx_get_tuning(ptx_device *dev, ptx_tuning *t) {
    *t = tuning_of(dev);
    if (!t->lds_stack) t->lds_stack = lds_depth_of(*t);
    if (!t->block_size) t->block_size = 256;
-   if (!t->refill_lanes) t->refill_lanes = kDefaultRefillLanes;
-   // leaf_lanes stays 0 when unset: each kernel family then uses its own default
-   if (!t->shade_lanes) t->shade_lanes = RenderEngine::kWideShadeLanes;   // what nearly every scene's kernels take
+   // refill_lanes, shade_lanes and leaf_lanes stay 0 when unset: the kernels over
+   // the four-wide tree and over binary records then use their own defaults, and
+   // setting back what was got changes none of them
    return PTX_OK;
 }
 

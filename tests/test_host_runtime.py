@@ -34,3 +34,7 @@ def run_check(tmp_path, name: str) -> str:
 
 def test_scene_creation_at_every_memory_limit(tmp_path):
     assert "\n0 failures" in run_check(tmp_path, "scene_memory_check")
+
+
+def test_tuning_that_was_got_can_be_set_back(tmp_path):
+    assert run_check(tmp_path, "tuning_check") == "0 failures\n"
