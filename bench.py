@@ -9,10 +9,11 @@ uniform on the sphere).  One step = one closest-hit launch over the 2^21
 incoherent rays, inputs resident in HBM; outputs are hit flag, (mesh, face),
 t and barycentrics per ray.
 
-Prints one JSON line: metric/value (incoherent Mrays/s), the roofline of the
-traversal kernel (algorithmic bytes per ray from the reference's own per-ray
-counters, which the kernel reproduces exactly), the coherent rate, and the CPU
-baseline (the reference CPU intersector when its build is present, otherwise
+Prints one JSON line: metric/value (incoherent Mrays/s), the traversal kernel's
+HBM traffic against the peak (bytes per launch from its counter profile), the
+bytes the reference's traversal reads for the same rays (from its own per-ray
+counters, which a counters query reproduces exactly), the coherent rate, and the
+CPU baseline (the reference CPU intersector when its build is present, otherwise
 the oracle restatement) timed on this host on a bounded sample.
 """
 from __future__ import annotations
@@ -147,7 +148,8 @@ def render_accounting(orc, jobs, t_batched: float, threads: int, row_step: int =
     the rays a sample traces and the reference's per-ray counters over them,
     scaled to the whole films.  The batched path traces a pixel's primary ray
     once (not once per sample), so it traces (spp - 1) * pixels fewer rays than
-    the integrator.  Bytes: per traced ray B_ray = 24 + 20 + 32 * N_box + 36 *
+    the integrator.  Bytes that the reference's traversal reads for these rays (the
+    four-wide kernels read others): per traced ray B_ray = 24 + 20 + 32 * N_box + 36 *
     N_tri, per sample 64 B of primary record and 12 B of result."""
     tot = {"rays": 0.0, "boxes": 0.0, "tris": 0.0, "samples": 0.0}
     gpu_rays = 0.0
@@ -170,8 +172,21 @@ def render_accounting(orc, jobs, t_batched: float, threads: int, row_step: int =
             "extend_mrays_per_s": round(gpu_rays / t_batched / 1e6, 1),
             "mean_box_tests_per_ray": round(mean_box, 2), "mean_face_tests_per_ray": round(mean_tri, 2),
             "bytes_per_ray": round(b_ray, 1), "algorithmic_bytes": round(total_bytes),
-            "achieved_gbs": round(total_bytes / t_batched / 1e9, 1),
-            "frac_of_hbm_peak": round(total_bytes / t_batched / 1e9 / HBM_PEAK_GBS, 4)}
+            "reference_bytes_gbs": round(total_bytes / t_batched / 1e9, 1)}
+
+
+def roofline(launch_ms: float, traffic, ray_windows: int = 0) -> dict:
+    """The launch's HBM bytes (profiled, of the default form; None for others) per
+    second against the peak.  The kernel is not bound by them: its VALU issues in
+    half of the cycles, and the rest waits on the longest rays' dependent loads."""
+    windows = ray_windows == 1
+    if windows:
+        traffic = None
+    gbs = traffic / (launch_ms / 1e3) / 1e9 if traffic else None
+    return {"bound": "dependent loads and VALU issue", "achieved": round(gbs, 1) if gbs else None,
+            "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4) if gbs else None,
+            "traffic": traffic, "kernel": "k_closest_hit" if windows else "k_closest_hit_wide",
+            "launch_ms": round(launch_ms, 4)}
 
 
 def render_section(dev, args):
@@ -265,8 +280,8 @@ def render_section(dev, args):
     if not args.skip_accounting:
         accounting = render_accounting(orc, jobs, t_batched, host_threads(args))
         print(f"[bench] render accounting: {accounting['extend_rays'] / 1e9:.3f} G extend rays, "
-              f"{accounting['extend_mrays_per_s']:.0f} Mrays/s, {accounting['achieved_gbs']:.0f} GB/s of algorithmic "
-              f"bytes", file=sys.stderr, flush=True)
+              f"{accounting['extend_mrays_per_s']:.0f} Mrays/s, {accounting['reference_bytes_gbs']:.0f} GB/s of the "
+              f"reference's bytes", file=sys.stderr, flush=True)
     if not args.skip_cpu:
         # CPU baseline: the oracle (port of the reference's integrator) on the same
         # scene and tree, the whole first job, on the host's cores
@@ -389,19 +404,27 @@ def serving_section(dev, args, n_requests: int, rate: float, burst: bool = False
     if not burst:
         out["offered_samples_per_s"] = round(total / max(1e-9, reqs[-1][0]), 1)
     out.update(_latency_stats(lat, total, last - first))
-    # the plain path over the same stream
-    dev.set_tuning(plain_primary=_abi.PLAIN_CACHED)
-    lat_p = []
-    t0 = time.perf_counter()
-    for arr, si, cam, spp, depth, seed in reqs:
-        delay = arr - (time.perf_counter() - t0)
-        if delay > 0:
-            time.sleep(delay)
-        render(scenes_[si], cam, spp, depth, seed)
-        lat_p.append(time.perf_counter() - (t0 + arr))
-    span = time.perf_counter() - t0
-    dev.set_tuning()
-    out["plain"] = _latency_stats(lat_p, total, span)
+    # the same stream through render(): one launch per sample, and, where the
+    # stream is not mostly waiting, as render() runs by default (a batch of one)
+    def one_at_a_time(form):
+        dev.set_tuning(plain_primary=form)
+        lat_p = []
+        t0 = time.perf_counter()
+        for arr, si, cam, spp, depth, seed in reqs:
+            delay = arr - (time.perf_counter() - t0)
+            if delay > 0:
+                time.sleep(delay)
+            render(scenes_[si], cam, spp, depth, seed)
+            lat_p.append(time.perf_counter() - (t0 + arr))
+        span = time.perf_counter() - t0
+        dev.set_tuning()
+        return _latency_stats(lat_p, total, span)
+
+    out["plain"] = one_at_a_time(_abi.PLAIN_CACHED)
+    if burst or rate > 50:
+        out["render"] = one_at_a_time(_abi.PLAIN_DEFAULT)
+        out["server_vs_render_throughput"] = round(
+            out["throughput_samples_per_s"] / out["render"]["throughput_samples_per_s"], 3)
     out["server_vs_plain_throughput"] = round(out["throughput_samples_per_s"] / out["plain"]["throughput_samples_per_s"], 3)
     out["server_vs_plain_p50_latency"] = round(out["plain"]["latency_p50_s"] / out["latency_p50_s"], 3)
     for s_ in scenes_:
@@ -444,7 +467,7 @@ def main():
     cnt = torch.empty(n_rays * 3, dtype=torch.int32, device="cuda")
     stream = torch.cuda.current_stream()
 
-    # algorithmic bytes of the incoherent half (untimed run with counters)
+    # the reference's bytes for the incoherent half (untimed run with counters)
     sc.intersect_device(inc_ptr, n_inc, hits.data_ptr(), cnt.data_ptr(), 0, stream.cuda_stream)
     torch.cuda.synchronize()
     c = cnt[: n_inc * 3].cpu().numpy().view(COUNTER_DTYPE)
@@ -475,7 +498,6 @@ def main():
     launch_ms = float(np.mean([s.elapsed_time(e) for s, e in ev]))
     ms_per_step = wall * 1e3 / args.steps
     mrays = n_inc / (ms_per_step / 1e3) / 1e6
-    achieved_gbs = mean_b * n_inc / (launch_ms / 1e3) / 1e9
 
     # PCIe-inclusive rate, not the metric: the host-buffer entry point on the
     # same rays (24 B of ray in, 24 B of hit out, between pageable numpy arrays,
@@ -491,7 +513,7 @@ def main():
 
     traffic = None
     tf = ROOT / "profiles" / "closest_hit_traffic.json"
-    if tf.exists():
+    if tf.exists() and args.subdiv == 8 and args.rays_log2 == 22:      # what the profile measured
         try:
             traffic = json.loads(tf.read_text()).get("hbm_bytes_per_launch")
         except Exception:
@@ -520,10 +542,9 @@ def main():
         "config": {"workload": "closest-hit microbench: icosphere subdiv 8 (1,310,720 tris), 2^21 incoherent "
                                "rays per step (of 2^22: half coherent 2048x1024, half incoherent)",
                    "triangles": meshes[0].num_faces, "rays_per_step": n_inc, "parallelism": "single GPU"},
-        "roofline": {"bound": "hbm", "achieved": round(achieved_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(achieved_gbs / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "bytes_per_ray": round(mean_b, 1), "kernel": "k_closest_hit",
-                     "launch_ms": round(launch_ms, 4)},
+        "roofline": roofline(launch_ms, traffic, args.ray_windows),
+        "reference_bytes": {"per_ray": round(mean_b, 1),
+                            "at_this_rate_gbs": round(mean_b * n_inc / (launch_ms / 1e3) / 1e9, 1)},
         "coherent_mrays_per_s": coherent_mrays,
         "host_buffers_mrays_per_s": host_mrays,
         "tuning": dev.get_tuning(),
