@@ -542,14 +542,20 @@ int RenderEngine::run_plain(const ptx_scene *scene, const ptx_job_desc &desc, fl
    // round's tables (0.62 against 0.71 ms; two of two bounces the same).
    // Where the slots (12 bytes each) find no memory, and with plain_primary
    // set, one launch per sample.
+   int rc;
    if (tun.plain_primary == PTX_PLAIN_DEFAULT && tun.render_mode != PTX_RENDER_WAVEFRONT && desc.spp > 1 &&
        (uint64_t)desc.spp * desc.max_depth > 2) {
       RenderJob job;
       job.desc = desc;
       job.npix = desc.camera.width * desc.camera.height;
-      const int rc = run_batch({job}, {scene}, {film_host}, kDefaultPlainPaths);
+      rc = run_batch({job}, {scene}, {film_host}, kDefaultPlainPaths);
       if (rc != PTX_ERR_OOM) return rc;
+   } else {
+      rc = run_launches(scene, desc, film_host);
+      if (rc != PTX_ERR_OOM || cap <= 1) return rc;
    }
+   // the path slots of this job or an earlier one may be what is missing
+   release();
    return run_launches(scene, desc, film_host);
 }
 

@@ -38,3 +38,7 @@ def test_scene_creation_at_every_memory_limit(tmp_path):
 
 def test_tuning_that_was_got_can_be_set_back(tmp_path):
     assert run_check(tmp_path, "tuning_check") == "0 failures\n"
+
+
+def test_render_at_memory_limits(tmp_path):
+    assert " 0 failures" in run_check(tmp_path, "render_memory_check")
