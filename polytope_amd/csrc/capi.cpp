@@ -55,17 +55,19 @@ struct Uploads {
    void add(const std::vector<T, A> &v, const T **dst) {
       add(v.data(), v.size(), dst);
    }
+   static size_t place(size_t bytes) { return (bytes + 255) & ~size_t(255); }
+   size_t bytes() const {
+      size_t all = 0;
+      for (const Item &i : items) all += place(i.bytes);
+      return all;
+   }
    // Makes them and leaves the list empty.
    int run() {
+      const size_t all = bytes();
       std::vector<Item> list;
       list.swap(items);
-      auto place = [](size_t bytes) { return (bytes + 255) & ~size_t(255); };
-      size_t all = 0;
       bool whole = true;
-      for (const Item &i : list) {
-         all += place(i.bytes);
-         whole = whole && i.src;
-      }
+      for (const Item &i : list) whole = whole && i.src;
       if (all == 0) return PTX_OK;
       char *p = nullptr;
       PTX_HIP_TRY(hipMalloc(reinterpret_cast<void **>(&p), all));
@@ -84,6 +86,21 @@ struct Uploads {
       return PTX_OK;
    }
 };
+
+// Whether a four-wide form of `bytes` leaves the device an eighth of its memory:
+// what a default batch needs beside its scenes is 12.9 GB of path slots and its
+// jobs' films and records, and forms of scenes that fill the device would take
+// it from renders that fitted without them.  Forms under 16 MB are not asked
+// about (the question takes as long as a small scene's copies).
+bool form_leaves_room(size_t bytes) {
+   size_t unused = 0, all = 0;
+   if (bytes < size_t(16) << 20) return true;
+   if (hipMemGetInfo(&unused, &all) != hipSuccess) {
+      (void)hipGetLastError();
+      return true;
+   }
+   return unused > bytes && unused - bytes >= all / 8;
+}
 
 // Faces up to which a scene's four-wide form is built by the calling thread and
 // its face records with it: a thread, a kernel and the wait for it take 35 us,
@@ -502,7 +519,7 @@ int ptx_scene_create(ptx_device *dev, const ptx_scene_desc *desc, ptx_scene **ou
    up.add(wide.leaves, &s->w.leaves);
    const uint8_t *flat = nullptr;
    if (few.empty()) up.add(wide.flat, &flat);
-   if (built && up.run() == PTX_OK) {
+   if (built && form_leaves_room(up.bytes()) && up.run() == PTX_OK) {
       s->w.root = wide.root;
       s->w.stack = wide.stack;
       if (few.empty()) {

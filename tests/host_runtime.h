@@ -125,6 +125,11 @@ hipError_t hipGetLastError(void) {
    state().last = hipSuccess;
    return e;
 }
+hipError_t hipMemGetInfo(size_t *unused, size_t *all) {
+   *all = state().limit;
+   *unused = state().limit - std::min(state().limit, state().used);
+   return hipSuccess;
+}
 hipError_t hipMalloc(void **p, size_t n) { return take(p, n); }
 hipError_t hipMallocAsync(void **p, size_t n, hipStream_t) { return take(p, n); }
 hipError_t hipMallocFromPoolAsync(void **p, size_t n, hipMemPool_t, hipStream_t) { return take(p, n); }

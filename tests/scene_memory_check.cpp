@@ -9,8 +9,9 @@
 #include "host_runtime.h"
 #include "ptx.h"
 
-// A sheet of 2 side^2 faces; returns the number of failures.
-static int check(uint32_t kSide) {
+// A sheet of 2 side^2 faces; returns the number of failures.  A form of 16 MB
+// or more (large) is made only where it leaves an eighth of the memory.
+static int check(uint32_t kSide, bool large, uint32_t steps) {
    const uint32_t kVerts = (kSide + 1) * (kSide + 1), kFaces = 2 * kSide * kSide, kTex = 16;
    std::vector<float> x(kVerts), y(kVerts), z(kVerts), up(kVerts, 1.f), flat(kVerts, 0.f), u(kVerts), v(kVerts);
    for (uint32_t i = 0; i < kVerts; i++) {
@@ -71,21 +72,21 @@ static int check(uint32_t kSide) {
    if (info.device_bytes != whole) std::printf("%zu bytes used, %zu told\n", whole, (size_t)info.device_bytes), bad++;
    ptx_scene_destroy(scene);
    // what it takes without the form: at the largest limit that the whole misses
-   rt.limit = base + whole - 1;
+   rt.limit = base + whole - (large ? 0 : 1);
    if (ptx_scene_create(dev, &desc, &scene) != PTX_OK) return std::printf("refused: %s\n", ptx_last_error()), 1;
    const size_t need = rt.used - base;
    if (need < least || need > least + 7 * 256) std::printf("%zu bytes without the form, %zu needed\n", need, least), bad++;
    ptx_scene_destroy(scene);
    uint32_t with = 0, without = 0, refused = 0;
-   const size_t step = whole / 211 + 1;
-   for (size_t limit = 0; limit <= whole; limit += limit + step < whole ? step : std::max<size_t>(1, whole - limit)) {
+   const size_t most = large ? whole * 5 / 4 : whole, step = most / steps + 1;
+   for (size_t limit = 0; limit <= most; limit += limit + step < most ? step : std::max<size_t>(1, most - limit)) {
       rt.limit = base + limit;
       scene = nullptr;
       const int rc = ptx_scene_create(dev, &desc, &scene);
       const size_t used = rt.used - base;
       if (rc == PTX_OK) {
          (void)ptx_scene_get_info(scene, &info);
-         if (limit < need || used != info.device_bytes || used != (limit < whole ? need : whole))
+         if (limit < need || used != info.device_bytes || used != (limit < whole || (large && limit - whole < (base + limit) / 8) ? need : whole))
             std::printf("limit %zu: a scene of %zu bytes, %zu told\n", limit, used, (size_t)info.device_bytes), bad++;
          (used == whole ? with : without)++;
          ptx_scene_destroy(scene);
@@ -95,7 +96,7 @@ static int check(uint32_t kSide) {
       }
       if (rt.used != base) std::printf("limit %zu: %zu bytes left\n", limit, rt.used - base), bad++;
       if (hipGetLastError() != hipSuccess) std::printf("limit %zu: an error left for the caller\n", limit), bad++;
-      if (limit == whole) break;
+      if (limit == most) break;
    }
    rt.limit = SIZE_MAX;
    ptx_device_close(dev);
@@ -105,7 +106,8 @@ static int check(uint32_t kSide) {
 
 int main() {
    int bad = 0;
-   for (uint32_t side : {4u, 24u, 48u}) bad += check(side);      // 32, 1,152 and 4,608 faces
+   for (uint32_t side : {4u, 24u, 48u}) bad += check(side, false, 211);      // 32, 1,152 and 4,608 faces
+   bad += check(400, true, 17);                                              // 320,000
    std::printf("%d failures\n", bad);
    return bad != 0;
 }
