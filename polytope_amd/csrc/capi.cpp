@@ -36,7 +36,7 @@ double now_s() {
 namespace {
 
 // Arrays of a scene that go up together, in one allocation (each costs about
-// 7 us, and its free more) and, while they are small, in one copy.
+// 7 us and its free 3) and, while they are small, in one copy.
 struct Uploads {
    static constexpr size_t kOneCopy = 256 << 10;
    struct Item {
@@ -635,7 +635,9 @@ int ptx_intersect_closest_device_noalloc(ptx_scene *scene, const float *d_rays, 
    PTX_HIP_TRY(hipSetDevice(dev->ordinal));
    uint32_t *work = static_cast<uint32_t *>(dev->noalloc_scratch);
    uint4 *spill = reinterpret_cast<uint4 *>(static_cast<char *>(dev->noalloc_scratch) + 256);
-   // the four-wide form wherever its spill takes no fewer blocks
+   // the four-wide form where the scratch holds its spill for a block per CU, or
+   // for all the blocks the rays fill (its entries are half as large and about
+   // twice as many: it holds nearly as many blocks as for the binary form)
    if (wide_query(scene, t, d_counters != nullptr)) {
       uint32_t wgrid = wide_query_grid(dev, t, lds, d_frames != nullptr);
       const size_t block = wide_spill_bytes(scene, 1, lds);

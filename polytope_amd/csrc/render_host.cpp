@@ -1,5 +1,5 @@
-// Host side of rendering: the plain one-job-per-launch-series path
-// (ptx_render), the batched path (ptx_render_batch) and the autotuner
+// Host side of rendering: the batched path (ptx_render_batch, and ptx_render as a
+// batch of one), ptx_render's launches per sample, and the autotuner
 // (ptx_autotune).
 //
 // The batched path keeps per-path results, a stack spill area and (for the

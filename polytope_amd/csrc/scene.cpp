@@ -61,7 +61,7 @@ inline __attribute__((always_inline)) void world_faces(const ptx_mesh_desc &m, W
 }
 
 // The same with the processor's fma in place of 36 calls of the library's a
-// face (the same values, every fma being rounded once): 39 -> 10 ns a face.
+// face (the same values, every fma being rounded once): 39 -> about 12 ns a face.
 __attribute__((target("fma"))) void world_faces_fma(const ptx_mesh_desc &m, WorldMesh &out, size_t lo, size_t hi) {
    world_faces(m, out, lo, hi);
 }
@@ -75,7 +75,7 @@ void world_vertices(const ptx_mesh_desc &m, WorldMesh &out, bool shading) {
    out.has_normals = m.nx && m.ny && m.nz;
    if (out.has_normals) out.wn.resize(size_t(9) * m.num_faces);
    const auto work = __builtin_cpu_supports("fma") ? world_faces_fma : world_faces_any;
-   host_ranges(m.num_faces, 0, 4096, [&](size_t lo, size_t hi) { work(m, out, lo, hi); });      // 40 us of them
+   host_ranges(m.num_faces, 0, 4096, [&](size_t lo, size_t hi) { work(m, out, lo, hi); });      // 50 us of them
    out.rec.brdf = m.brdf;
    std::copy(m.refl, m.refl + 3, out.rec.refl);
    out.rec.is_light = m.is_light;

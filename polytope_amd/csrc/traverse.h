@@ -1,12 +1,14 @@
-// Persistent closest-hit traversal shared by the ray-query kernel and the
-// render path's extend stage.
+// Persistent closest-hit traversals over the binary records, one lane per ray in
+// flight, and what the four-wide one (wide.h) shares with them.
 //
-// One lane per ray in flight.  Each loop iteration is one step for every lane
-// of the wave: lanes that finished take new work ids from a per-wave pool,
-// then every lane issues the loads of its step (a new ray, an interior record
-// or up to two leaf faces) before any lane computes, so the wave waits on
-// memory once per step.  The deferred-child stack lives in LDS (kLds entries
-// per lane), deeper entries spill to a global array sized from the tree depth.
+// query_trace serves ray queries: node steps and leaf steps in loops of their
+// own.  persistent_trace serves the render path's extend stage and primary rays:
+// each loop iteration is one step for every lane of the wave, lanes that finished
+// take new work ids from a per-wave pool, then every lane issues the loads of its
+// step (a new ray, an interior record or up to two leaf faces) before any lane
+// computes, so the wave waits on memory once per step.  The deferred-child stack
+// lives in LDS (kLds entries per lane), deeper entries spill to a global array
+// sized from the tree depth.
 #pragma once
 
 #include <type_traits>
@@ -350,7 +352,7 @@ struct Staged {
 // step.  An ended lane keeps its ray until enough have ended to take new ones,
 // or all have: a frame costs as much as a dozen node steps and was computed
 // for the whole wave every time one lane ended.  200,003 rays with counters
-// and frames on 81,920 faces 313 -> 155 us (43 % of the VALU's cycles busy, a
+// and frames on 81,920 faces 318 -> 170 us (43 % of the VALU's cycles busy, a
 // fifth of its lanes, before), a 4K frame's primary rays with counters on 1.3 M
 // faces 2,018 -> 1,490 us.  Five waves per SIMD gain 6 % there and lose 3 to 9 %
 // on 50,021 rays.
