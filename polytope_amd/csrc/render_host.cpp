@@ -407,12 +407,22 @@ uint32_t RenderEngine::capacity_for(uint64_t total_paths, uint32_t max_npix, boo
 
 int RenderEngine::run_batch(const std::vector<RenderJob> &jobs, const std::vector<const ptx_scene *> &scenes,
                             const std::vector<float *> &films_host, uint32_t regen_paths) {
+   int rc = batch(jobs, scenes, films_host, regen_paths, true);
+   if (rc == PTX_ERR_OOM) {
+      release();
+      rc = batch(jobs, scenes, films_host, regen_paths, false);
+   }
+   return rc;
+}
+
+int RenderEngine::batch(const std::vector<RenderJob> &jobs, const std::vector<const ptx_scene *> &scenes,
+                        const std::vector<float *> &films_host, uint32_t regen_paths, bool wide_spill) {
    const uint32_t nj = (uint32_t)jobs.size();
    uint32_t max_stack = 1, wide_stack = 0, max_npix = 1;
    uint64_t total_paths = 0;
    for (const auto *s : scenes) {
       max_stack = std::max(max_stack, s->d.max_stack);
-      wide_stack = std::max(wide_stack, s->w.stack);
+      if (wide_spill) wide_stack = std::max(wide_stack, s->w.stack);
    }
    for (const auto &j : jobs) {
       max_npix = std::max(max_npix, j.npix);
@@ -551,17 +561,22 @@ int RenderEngine::run_plain(const ptx_scene *scene, const ptx_job_desc &desc, fl
       rc = run_batch({job}, {scene}, {film_host}, kDefaultPlainPaths);
       if (rc != PTX_ERR_OOM) return rc;
    } else {
-      rc = run_launches(scene, desc, film_host);
-      if (rc != PTX_ERR_OOM || cap <= 1) return rc;
+      rc = run_launches(scene, desc, film_host, true);
+      if (rc != PTX_ERR_OOM) return rc;
    }
-   // the path slots of this job or an earlier one may be what is missing
-   release();
-   return run_launches(scene, desc, film_host);
+   // the path slots of this job or an earlier one may be what is missing, or
+   // the larger spill of the four-wide stack
+   for (const bool wide_spill : {true, false}) {
+      release();
+      rc = run_launches(scene, desc, film_host, wide_spill);
+      if (rc != PTX_ERR_OOM) break;
+   }
+   return rc;
 }
 
-int RenderEngine::run_launches(const ptx_scene *scene, const ptx_job_desc &desc, float *film_host) {
+int RenderEngine::run_launches(const ptx_scene *scene, const ptx_job_desc &desc, float *film_host, bool wide_spill) {
    const uint32_t npix = desc.camera.width * desc.camera.height;
-   int rc = ensure(cap ? cap : 1u, scene->d.max_stack, scene->w.stack, 1, 1, 1);
+   int rc = ensure(cap ? cap : 1u, scene->d.max_stack, wide_spill ? scene->w.stack : 0u, 1, 1, 1);
    if (rc) return rc;
    hipStream_t st = stream;
    // the default traces each pixel's primary ray once (every sample of a pixel

@@ -132,11 +132,17 @@ struct RenderEngine {
    void free_job(JobDev &J);
    uint32_t capacity_for(uint64_t total_paths, uint32_t max_npix, bool regen, uint32_t regen_paths) const;
    // regen_paths: path slots of a regeneration round when the tuning names none.
+   // Where a batch finds no memory the engine's buffers go back and it is tried
+   // again with a spill for the binary stack alone, 16 bytes a level and lane
+   // against 8 for each of up to three times as many entries (a scene whose
+   // four-wide stack does not fit it steps over binary records).
    int run_batch(const std::vector<RenderJob> &jobs, const std::vector<const ptx_scene *> &scenes,
                  const std::vector<float *> &films_host, uint32_t regen_paths = kDefaultRegenPaths);
+   int batch(const std::vector<RenderJob> &jobs, const std::vector<const ptx_scene *> &scenes,
+             const std::vector<float *> &films_host, uint32_t regen_paths, bool wide_spill);
    // ptx_render: a batch of one job, or one launch per sample (run_launches).
    int run_plain(const ptx_scene *scene, const ptx_job_desc &desc, float *film_host);
-   int run_launches(const ptx_scene *scene, const ptx_job_desc &desc, float *film_host);
+   int run_launches(const ptx_scene *scene, const ptx_job_desc &desc, float *film_host, bool wide_spill);
 };
 
 RenderEngine *engine_of(ptx_device *dev);

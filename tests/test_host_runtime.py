@@ -42,3 +42,7 @@ def test_tuning_that_was_got_can_be_set_back(tmp_path):
 
 def test_render_at_memory_limits(tmp_path):
     assert " 0 failures" in run_check(tmp_path, "render_memory_check")
+
+
+def test_stack_spill_at_memory_limits(tmp_path):
+    assert " 0 failures" in run_check(tmp_path, "spill_memory_check")
