@@ -225,20 +225,33 @@ uint32_t wide_refill_lanes_of(const ptx_tuning &t) {
 }  // namespace
 
 QueryLaunch::QueryLaunch(ptx_scene *s, uint32_t n, bool counters, bool frames, const ptx_tuning &t)
-    : scene(s), tun(t), lds(lds_depth_of(t)), wide(wide_query(s, t, counters)) {
-   ptx_device *dev = s->dev;
+    : scene(s), tun(t), n(n), lds(lds_depth_of(t)), extra(counters || frames) {
+   plan(wide_query(s, t, counters));
+}
+
+void QueryLaunch::plan(bool wide_form) {
+   ptx_device *dev = scene->dev;
    Deal deal;
+   wide = wide_form;
    if (wide) {
-      full = wide_query_grid(dev, t, lds, frames);
-      bytes = 256 + wide_spill_bytes(s, deal_ids(full, (uint32_t)dev->num_cus, n, deal), lds);
+      full = wide_query_grid(dev, tun, lds, extra);   // no counters here: extra is frames
+      bytes = 256 + wide_spill_bytes(scene, deal_ids(full, (uint32_t)dev->num_cus, n, deal), lds);
    } else {
-      win = n ? scene_windows(s, t) : nullptr;
-      full = closest_hit_grid(dev, t, lds, counters || frames, win != nullptr);
-      bytes = closest_hit_scratch_bytes(s, deal_ids(full, (uint32_t)dev->num_cus, n, deal), lds);
+      win = n ? scene_windows(scene, tun) : nullptr;
+      full = closest_hit_grid(dev, tun, lds, extra, win != nullptr);
+      bytes = closest_hit_scratch_bytes(scene, deal_ids(full, (uint32_t)dev->num_cus, n, deal), lds);
    }
 }
 
 int QueryLaunch::take_scratch(hipStream_t stream) {
+   if (wide) {
+      if (pool_malloc(scene->dev, &scratch, bytes, stream) == hipSuccess) return PTX_OK;
+      // the four-wide stack's spill may be what is too large: 8 bytes for each of
+      // up to three entries a level, against 16 for one
+      (void)hipGetLastError();
+      scratch = nullptr;
+      plan(false);
+   }
    PTX_HIP_TRY(pool_malloc(scene->dev, &scratch, bytes, stream));
    return PTX_OK;
 }

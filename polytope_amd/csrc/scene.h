@@ -114,14 +114,16 @@ size_t closest_hit_scratch_bytes(const ptx_scene *s, uint32_t grid, uint32_t lds
 struct QueryLaunch {
    ptx_scene *scene;
    ptx_tuning tun;
-   uint32_t lds;
-   bool wide;
+   uint32_t n, lds;
+   bool extra;                        // counters or frames
+   bool wide = false;
    const Node64 *win = nullptr;
    uint32_t full = 0;                 // blocks that fit the device
    size_t bytes = 0;
    void *scratch = nullptr;
    QueryLaunch(ptx_scene *s, uint32_t n, bool counters, bool frames, const ptx_tuning &t);
-   int take_scratch(hipStream_t stream);
+   void plan(bool wide_form);
+   int take_scratch(hipStream_t stream);   // of the binary form where the four-wide one's finds no memory
    int give_scratch(hipStream_t stream);
    int launch(const float *d_rays, uint32_t n, ptx_hit *d_hits, ptx_ray_counters *d_counters, ptx_hit_frame *d_frames,
               hipStream_t stream);

@@ -1,7 +1,7 @@
 // Host check of the stack spill at memory limits: wherever a scene without a
 // four-wide form renders (a batch, with next-event estimation, over wavefront
-// queues, one launch per sample) the same scene with one does too, although its
-// stack asks for more.  Prints the failures; exit 1
+// queues, one launch per sample) or answers device rays, the same scene with
+// one does too, although its stack asks for more.  Prints the failures; exit 1
 // on any.
 #include <cmath>
 #include <cstdio>
@@ -9,7 +9,7 @@
 #include "host_runtime.h"
 #include "ptx.h"
 
-enum Call { kBatch, kBatchNee, kWavefront, kLaunches, kCalls };
+enum Call { kBatch, kBatchNee, kWavefront, kLaunches, kRays, kCalls };
 
 static ptx_job_desc job_of(uint32_t w, uint32_t h, uint32_t spp, bool nee) {
    ptx_job_desc j{};
@@ -71,19 +71,26 @@ static int run(Call call, size_t limit, bool wide) {
    }
    rt.limit = rt.used + limit;
    static std::vector<float> film[2] = {std::vector<float>(3 * 512 * 400), std::vector<float>(3 * 256 * 256)};
-   const bool nee = call == kBatchNee;
-   ptx_tuning t{};
-   if (call == kWavefront) {
-      t.render_mode = PTX_RENDER_WAVEFRONT;
-      t.paths_per_wave = 1 << 18;
-   } else if (call == kLaunches) {
-      t.plain_primary = PTX_PLAIN_RETRACE;
+   int rc = -1;
+   if (call == kRays) {
+      float rays[6] = {0};
+      ptx_hit hit;
+      rc = ptx_intersect_closest_device(scene, rays, 1 << 20, &hit, nullptr, nullptr, nullptr);
+   } else {
+      const bool nee = call == kBatchNee;
+      ptx_tuning t{};
+      if (call == kWavefront) {
+         t.render_mode = PTX_RENDER_WAVEFRONT;
+         t.paths_per_wave = 1 << 18;
+      } else if (call == kLaunches) {
+         t.plain_primary = PTX_PLAIN_RETRACE;
+      }
+      (void)ptx_set_tuning(dev, &t);
+      const ptx_job_desc jobs[2] = {job_of(512, 400, 4, nee), job_of(256, 256, 16, nee)};
+      ptx_scene *scenes[2] = {scene, scene};
+      float *films[2] = {film[0].data(), film[1].data()};
+      rc = call == kLaunches ? ptx_render(scene, jobs, films[0]) : ptx_render_batch(scenes, jobs, 2, films);
    }
-   (void)ptx_set_tuning(dev, &t);
-   const ptx_job_desc jobs[2] = {job_of(512, 400, 4, nee), job_of(256, 256, 16, nee)};
-   ptx_scene *scenes[2] = {scene, scene};
-   float *films[2] = {film[0].data(), film[1].data()};
-   const int rc = call == kLaunches ? ptx_render(scene, jobs, films[0]) : ptx_render_batch(scenes, jobs, 2, films);
    rt.limit = SIZE_MAX;
    ptx_scene_destroy(scene);
    ptx_device_close(dev);
