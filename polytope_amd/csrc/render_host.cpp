@@ -154,8 +154,16 @@ void RenderEngine::release() {
    tables_host_bytes = 0;
    cap = qcap = 0;
    jobs_cap = scenes_cap = chunks_cap = 0;
+   spill_entries = binary_entries = 0;
+   graphs_stale = true;
+}
+
+bool RenderEngine::drop_wide_spill() {
+   if (spill_entries <= binary_entries) return false;
+   dfree(spill);
    spill_entries = 0;
    graphs_stale = true;
+   return true;
 }
 
 size_t RenderEngine::bytes_for(uint32_t paths, bool queues) {
@@ -185,13 +193,18 @@ int RenderEngine::ensure(uint32_t paths, uint32_t max_stack, uint32_t wide_stack
    const uint32_t stride_threads = std::max({ext_grid, mega_grid, mega_nee_grid, paths_grid, connect_grid,
                                              primary_wide_grid, mega_wide_grid, mega_wide_nee_grid}) * 256;
    // 16-byte entries of the binary stack, or 8-byte ones of the four-wide
-   const uint32_t levels = std::max(max_stack > lds ? max_stack - lds : 0u,
-                                    wide_stack > lds ? (wide_stack - lds + 1) / 2 : 0u);
-   const size_t need_spill = (size_t)levels * stride_threads;
+   const size_t wide_entries = wide_stack > lds ? (size_t)((wide_stack - lds + 1) / 2) * stride_threads : 0;
+   binary_entries = std::max(binary_entries, max_stack > lds ? (size_t)(max_stack - lds) * stride_threads : 0);
+   size_t need_spill = std::max(binary_entries, wide_entries);
    int rc;
    if (paths > cap) {
       dfree(res);
-      if ((rc = dalloc(this, &res, (size_t)paths * 3))) {
+      rc = dalloc(this, &res, (size_t)paths * 3);
+      if (rc && drop_wide_spill()) {
+         need_spill = binary_entries;
+         rc = dalloc(this, &res, (size_t)paths * 3);
+      }
+      if (rc) {
          release();
          return rc;
       }
@@ -204,7 +217,13 @@ int RenderEngine::ensure(uint32_t paths, uint32_t max_stack, uint32_t wide_stack
    }
    if (need_spill > spill_entries) {
       dfree(spill);
-      if ((rc = dalloc(this, &spill, need_spill))) { release(); return rc; }
+      spill_entries = 0;
+      rc = dalloc(this, &spill, need_spill);
+      if (rc && need_spill > binary_entries) {
+         need_spill = binary_entries;
+         rc = dalloc(this, &spill, need_spill);
+      }
+      if (rc) { release(); return rc; }
       spill_entries = need_spill;
       graphs_stale = true;
    }
@@ -408,10 +427,7 @@ uint32_t RenderEngine::capacity_for(uint64_t total_paths, uint32_t max_npix, boo
 int RenderEngine::run_batch(const std::vector<RenderJob> &jobs, const std::vector<const ptx_scene *> &scenes,
                             const std::vector<float *> &films_host, uint32_t regen_paths) {
    int rc = batch(jobs, scenes, films_host, regen_paths, true);
-   if (rc == PTX_ERR_OOM) {
-      release();
-      rc = batch(jobs, scenes, films_host, regen_paths, false);
-   }
+   if (rc == PTX_ERR_OOM && drop_wide_spill()) rc = batch(jobs, scenes, films_host, regen_paths, false);
    return rc;
 }
 
@@ -561,20 +577,21 @@ int RenderEngine::run_plain(const ptx_scene *scene, const ptx_job_desc &desc, fl
       rc = run_batch({job}, {scene}, {film_host}, kDefaultPlainPaths);
       if (rc != PTX_ERR_OOM) return rc;
    } else {
-      rc = run_launches(scene, desc, film_host, true);
-      if (rc != PTX_ERR_OOM) return rc;
+      rc = run_launches(scene, desc, film_host);
+      if (rc != PTX_ERR_OOM || cap <= 1) return rc;
    }
-   // the path slots of this job or an earlier one may be what is missing, or
-   // the larger spill of the four-wide stack
-   for (const bool wide_spill : {true, false}) {
-      release();
-      rc = run_launches(scene, desc, film_host, wide_spill);
-      if (rc != PTX_ERR_OOM) break;
-   }
+   // the path slots of this job or an earlier one may be what is missing
+   release();
+   return run_launches(scene, desc, film_host);
+}
+
+int RenderEngine::run_launches(const ptx_scene *scene, const ptx_job_desc &desc, float *film_host) {
+   int rc = launches(scene, desc, film_host, true);
+   if (rc == PTX_ERR_OOM && drop_wide_spill()) rc = launches(scene, desc, film_host, false);
    return rc;
 }
 
-int RenderEngine::run_launches(const ptx_scene *scene, const ptx_job_desc &desc, float *film_host, bool wide_spill) {
+int RenderEngine::launches(const ptx_scene *scene, const ptx_job_desc &desc, float *film_host, bool wide_spill) {
    const uint32_t npix = desc.camera.width * desc.camera.height;
    int rc = ensure(cap ? cap : 1u, scene->d.max_stack, wide_spill ? scene->w.stack : 0u, 1, 1, 1);
    if (rc) return rc;

@@ -52,7 +52,11 @@ struct RenderEngine {
    uint32_t *words = nullptr;
    uint4 *spill = nullptr;
    float4 *nee_scratch = nullptr;           // per resident lane of the regeneration kernel, 48 bytes
-   size_t spill_entries = 0;
+   // Spill entries of 16 bytes: allocated, and what the binary stacks need of
+   // them (16 bytes a level and lane; the four-wide stack takes 8 for each of up
+   // to three entries a level, and a scene whose stack does not fit the spill
+   // steps over binary records).
+   size_t spill_entries = 0, binary_entries = 0;
    uint32_t stack_cap = 0;                  // binary stack levels the spill holds
    uint32_t wide_cap = 0;                   // four-wide stack entries it holds
    // The round tables, one device allocation: jobs, offsets, scenes, four-wide
@@ -132,17 +136,18 @@ struct RenderEngine {
    void free_job(JobDev &J);
    uint32_t capacity_for(uint64_t total_paths, uint32_t max_npix, bool regen, uint32_t regen_paths) const;
    // regen_paths: path slots of a regeneration round when the tuning names none.
-   // Where a batch finds no memory the engine's buffers go back and it is tried
-   // again with a spill for the binary stack alone, 16 bytes a level and lane
-   // against 8 for each of up to three times as many entries (a scene whose
-   // four-wide stack does not fit it steps over binary records).
+   // Where a batch or the launches of one find no memory while the spill is
+   // larger than the binary stacks need, they are tried again without that part.
    int run_batch(const std::vector<RenderJob> &jobs, const std::vector<const ptx_scene *> &scenes,
                  const std::vector<float *> &films_host, uint32_t regen_paths = kDefaultRegenPaths);
    int batch(const std::vector<RenderJob> &jobs, const std::vector<const ptx_scene *> &scenes,
              const std::vector<float *> &films_host, uint32_t regen_paths, bool wide_spill);
    // ptx_render: a batch of one job, or one launch per sample (run_launches).
    int run_plain(const ptx_scene *scene, const ptx_job_desc &desc, float *film_host);
-   int run_launches(const ptx_scene *scene, const ptx_job_desc &desc, float *film_host, bool wide_spill);
+   int run_launches(const ptx_scene *scene, const ptx_job_desc &desc, float *film_host);
+   int launches(const ptx_scene *scene, const ptx_job_desc &desc, float *film_host, bool wide_spill);
+   // Frees a spill that only the four-wide stacks need; false where there is none.
+   bool drop_wide_spill();
 };
 
 RenderEngine *engine_of(ptx_device *dev);
